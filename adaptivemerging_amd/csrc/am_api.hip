@@ -603,7 +603,6 @@ int do_detect(am_ctx* c) {
 // ---- learned warm start helpers ------------------------------------------
 constexpr int OW1 = 0, OW2 = kPadW1, OW3 = OW2 + kPadW2, OW4 = OW3 + kPadW3;
 constexpr int OB1 = OW4 + kPadW4, OB2 = OB1 + kPadB1, OB3 = OB2 + kPadB2, OB4 = OB3 + kPadB3;
-constexpr int kBfTotal = kPadW1 + kPadW2 + kPadW3 + kPadW4;
 
 // flat (reference layout of include/am.h) <-> padded device layout
 void pack_params(const float* flat, std::vector<float>& pad) {
@@ -639,17 +638,13 @@ MlpWeights mlp_weights(am_ctx* c) {
     const float* p = c->m_p.p;
     return MlpWeights{bf + OW1, bf + OW2, bf + OW3, bf + OW4, p + OB1, p + OB2, p + OB3, p + OB4};
 }
-MlpGrads mlp_grads(am_ctx* c) {
-    float* g = c->m_g.p;
-    return MlpGrads{g + OW1, g + OW2, g + OW3, g + OW4, g + OB1, g + OB2, g + OB3, g + OB4};
-}
 
 int mlp_alloc(am_ctx* c) {
     AM_HIP(c, c->m_p.ensure(kPadTotal));
     AM_HIP(c, c->m_g.ensure(kPadTotal));
     AM_HIP(c, c->m_m.ensure(kPadTotal));
     AM_HIP(c, c->m_v.ensure(kPadTotal));
-    AM_HIP(c, c->m_bf.ensure(kBfTotal));
+    AM_HIP(c, c->m_bf.ensure(kPadWeights));
     AM_HIP(c, c->d_loss.ensure(4));
     return AM_OK;
 }
@@ -662,10 +657,9 @@ int mlp_upload(am_ctx* c, const float* flat) {
     hipStream_t s = c->stream;
     AM_HIP(c, hipMemcpyAsync(c->m_p.p, pad.data(), kPadTotal * 4, hipMemcpyHostToDevice, s));
     std::vector<float> z(kPadTotal, 0.f);
-    AM_HIP(c, hipMemcpyAsync(c->m_g.p, z.data(), kPadTotal * 4, hipMemcpyHostToDevice, s));
     AM_HIP(c, hipMemcpyAsync(c->m_m.p, z.data(), kPadTotal * 4, hipMemcpyHostToDevice, s));
     AM_HIP(c, hipMemcpyAsync(c->m_v.p, z.data(), kPadTotal * 4, hipMemcpyHostToDevice, s));
-    launch_to_bf16(s, c->m_p.p, c->m_bf.p, kBfTotal);
+    launch_to_bf16(s, c->m_p.p, c->m_bf.p, kPadWeights);
     AM_HIP(c, hipGetLastError());
     AM_HIP(c, hipStreamSynchronize(s));
     c->adam_step = 0;
@@ -2320,26 +2314,22 @@ int am_mlp_gradients(am_ctx* c, const float* x, const float* t, int32_t n, float
     if (!c->mlp_ready) return fail(c, AM_ERR_STATE, "MLP not initialised");
     if (n <= 0 || !x || !t || !grads) return fail(c, AM_ERR_INVALID, "bad MLP arrays");
     DBuf<float> dx, dt_;
-    DBuf<int> di;
     AM_HIP(c, dx.ensure((size_t)n * kMlpIn));
     AM_HIP(c, dt_.ensure((size_t)n * kMlpOut));
-    AM_HIP(c, di.ensure(n));
-    std::vector<int> idx(n);
-    for (int i = 0; i < n; i++) idx[i] = i;
     hipStream_t s = c->stream;
     AM_HIP(c, hipMemcpyAsync(dx.p, x, (size_t)n * kMlpIn * 4, hipMemcpyHostToDevice, s));
     AM_HIP(c, hipMemcpyAsync(dt_.p, t, (size_t)n * kMlpOut * 4, hipMemcpyHostToDevice, s));
-    AM_HIP(c, hipMemcpyAsync(di.p, idx.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
-    fill_int(s, (int*)c->m_g.p, kPadTotal, 0);
     fill_int(s, (int*)c->d_loss.p, 1, 0);
-    launch_mlp_backward(s, mlp_weights(c), dx.p, dt_.p, di.p, n, 1.0f / (float)n, mlp_grads(c), c->d_loss.p);
+    AM_HIP(c, c->m_partial.ensure(mlp_partial_floats(n)));
+    AdamArgs A{};
+    A.g = c->m_g.p;
+    launch_mlp_backward(s, mlp_weights(c), dx.p, dt_.p, nullptr, n, 1.0f / (float)n, c->m_partial.p, A, c->d_loss.p);
     AM_HIP(c, hipGetLastError());
     std::vector<float> pad(kPadTotal);
     float l = 0;
     AM_HIP(c, hipMemcpyAsync(pad.data(), c->m_g.p, kPadTotal * 4, hipMemcpyDeviceToHost, s));
     AM_HIP(c, hipMemcpyAsync(&l, c->d_loss.p, 4, hipMemcpyDeviceToHost, s));
     AM_HIP(c, hipStreamSynchronize(s));
-    fill_int(s, (int*)c->m_g.p, kPadTotal, 0);
     unpack_params(pad, grads);
     if (loss) *loss = l;
     return AM_OK;
@@ -2379,6 +2369,7 @@ int am_train_epochs(am_ctx* c, int32_t epochs, int32_t batch, float lr, uint64_t
     const int n = c->t_n;
     hipStream_t s = c->stream;
     AM_HIP(c, c->t_idx.ensure(n));
+    AM_HIP(c, c->m_partial.ensure(mlp_partial_floats(std::min(batch, n))));
     std::vector<int> perm(n);
     for (int i = 0; i < n; i++) perm[i] = i;
     uint64_t st = seed;
@@ -2393,13 +2384,21 @@ int am_train_epochs(am_ctx* c, int32_t epochs, int32_t batch, float lr, uint64_t
         fill_int(s, (int*)c->d_loss.p, 1, 0);
         for (int b0 = 0; b0 < n; b0 += batch) {
             int m = std::min(batch, n - b0);
-            launch_mlp_backward(s, mlp_weights(c), c->t_X.p, c->t_T.p, c->t_idx.p + b0, m, 1.0f / (float)m,
-                                mlp_grads(c), c->d_loss.p);
             c->adam_step++;
-            launch_adam(s, c->m_p.p, c->m_g.p, c->m_m.p, c->m_v.p, c->m_bf.p, kBfTotal, lr, 0.9f, 0.999f, 1e-8f,
-                        c->adam_step, nullptr);
-            launch_adam(s, c->m_p.p + kBfTotal, c->m_g.p + kBfTotal, c->m_m.p + kBfTotal, c->m_v.p + kBfTotal,
-                        nullptr, kPadTotal - kBfTotal, lr, 0.9f, 0.999f, 1e-8f, c->adam_step, nullptr);
+            AdamArgs A;
+            A.g = nullptr;
+            A.p = c->m_p.p;
+            A.m = c->m_m.p;
+            A.v = c->m_v.p;
+            A.bf = c->m_bf.p;
+            A.lr = lr;
+            A.b1 = 0.9f;
+            A.b2 = 0.999f;
+            A.eps = 1e-8f;
+            A.c1 = 1.f - powf(A.b1, (float)c->adam_step);
+            A.c2 = 1.f - powf(A.b2, (float)c->adam_step);
+            launch_mlp_backward(s, mlp_weights(c), c->t_X.p, c->t_T.p, c->t_idx.p + b0, m, 1.0f / (float)m,
+                                c->m_partial.p, A, c->d_loss.p);
         }
         AM_HIP(c, hipGetLastError());
         AM_HIP(c, hipMemcpyAsync(&loss, c->d_loss.p, 4, hipMemcpyDeviceToHost, s));

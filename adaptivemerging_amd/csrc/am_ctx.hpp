@@ -221,6 +221,7 @@ struct am_ctx {
     // learned warm start
     bool mlp_ready = false;
     DBuf<float> m_p, m_g, m_m, m_v;  // padded FP32 parameters, gradients, Adam moments
+    DBuf<float> m_partial;           // the backward pass's per-wave gradients
     DBuf<unsigned short> m_bf;       // padded BF16 weights
     DBuf<float> f_X, f_Y, d_loss;
     DBuf<double> f_scale, f_lam, s_start, dv_save;

@@ -88,42 +88,61 @@ AMD_INLINE float bf2f(unsigned short h) { return __uint_as_float(((unsigned)h) <
 
 // Layer geometry: padded input 32, hidden 64, padded output 16.
 constexpr int kIn = 32, kH = 64, kOut = 16;
-// bf16 weights in LDS, row-major [in][out]
-struct MlpLds {
-    unsigned short w1[kIn * kH];
-    unsigned short w2[kH * kH];
-    unsigned short w3[kH * kH];
-    unsigned short w4[kH * kOut];
-    float b1[kH], b2[kH], b3[kH], b4[kOut];
-};
 
-// One 16x16 output tile C += A(16 x K) * B(K x 16) with v_mfma_f32_16x16x16_bf16.
-// Lane l holds A[l%16][k0+4(l/16)+j], B[k0+4(l/16)+j][l%16] and returns
-// C[4(l/16)+j][l%16] for j = 0..3.  A and B are read from LDS through strides
-// (sa_r, sa_k) and (sb_k, sb_n), so transposed operands are just strides.
-AMD_INLINE float4v mfma_tile(const unsigned short* A, int sa_r, int sa_k, const unsigned short* Bm, int sb_k,
-                             int sb_n, int K, float4v c) {
-    const int l = threadIdx.x & 63;
-    const int row = l & 15, kq = (l >> 4) * 4;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        short4v a, b;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            a[j] = (short)A[row * sa_r + (k0 + kq + j) * sa_k];
-            b[j] = (short)Bm[(k0 + kq + j) * sb_k + row * sb_n];
-        }
-        c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-    }
-    return c;
+// Every product runs transposed, D (n x rows) = W^T (n x k) * in^T (k x rows),
+// on v_mfma_f32_16x16x16_bf16: lane l holds A[l%16][4(l/16)+j],
+// B[4(l/16)+j][l%16] and D[4(l/16)+j][l%16] for j = 0..3.  With the weights
+// stored [out][in] and the activations [row][unit], each lane's four operand
+// values are one 8-byte LDS read, and its four results are consecutive units
+// of one row, one 8-byte write of the next layer's input.  Rows are padded by
+// 8 values so that the 16 lanes of a fragment start on different banks.
+constexpr int kInS = kIn + 8, kHS = kH + 8, kOutS = kOut + 4;
+typedef short4v __attribute__((may_alias)) short4a;
+AMD_INLINE short4v ld4(const unsigned short* p) { return *reinterpret_cast<const short4a*>(p); }
+AMD_INLINE void st4(unsigned short* p, const unsigned short (&v)[4]) {
+    short4v s = {(short)v[0], (short)v[1], (short)v[2], (short)v[3]};
+    *reinterpret_cast<short4a*>(p) = s;
+}
+AMD_INLINE float4v mfma16(short4v a, short4v b, float4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+// LDS of one wave is read back by other lanes of it: order the accesses.
+AMD_INLINE void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-AMD_INLINE void load_weights(const MlpWeights& W, MlpLds& L) {
-    for (int i = threadIdx.x; i < kIn * kH; i += blockDim.x) L.w1[i] = W.w1_bf[i];
-    for (int i = threadIdx.x; i < kH * kH; i += blockDim.x) {
-        L.w2[i] = W.w2_bf[i];
-        L.w3[i] = W.w3_bf[i];
+// Weights in LDS as [out][in] (forward), biases.
+struct MlpLds {
+    alignas(16) unsigned short t1[kH * kInS];
+    alignas(16) unsigned short t2[kH * kHS];
+    alignas(16) unsigned short t3[kH * kHS];
+    alignas(16) unsigned short t4[kOut * kHS];
+    float b1[kH], b2[kH], b3[kH], b4[kOut];
+};
+// The same weights as [in][out], which the backward pass multiplies by.
+struct MlpLdsBack {
+    alignas(16) unsigned short w2[kH * kHS];
+    alignas(16) unsigned short w3[kH * kHS];
+    alignas(16) unsigned short w4[kH * kOutS];
+};
+
+// one matrix of `in` rows and `out` (16 or 64) columns, four values a thread
+AMD_INLINE void load_matrix(const unsigned short* W, int in, int out, unsigned short* t, int ts, unsigned short* w,
+                            int ws) {
+    for (int i = threadIdx.x; i < in * out / 4; i += blockDim.x) {
+        const int r = i / (out / 4), c = (i % (out / 4)) * 4;
+        const short4v v = ld4(W + r * out + c);
+#pragma unroll
+        for (int j = 0; j < 4; j++) t[(c + j) * ts + r] = (unsigned short)v[j];
+        if (w) *reinterpret_cast<short4a*>(w + r * ws + c) = v;
     }
-    for (int i = threadIdx.x; i < kH * kOut; i += blockDim.x) L.w4[i] = W.w4_bf[i];
+}
+AMD_INLINE void load_weights(const MlpWeights& W, MlpLds& L, MlpLdsBack* B) {
+    load_matrix(W.w1_bf, kIn, kH, L.t1, kInS, nullptr, 0);
+    load_matrix(W.w2_bf, kH, kH, L.t2, kHS, B ? B->w2 : nullptr, kHS);
+    load_matrix(W.w3_bf, kH, kH, L.t3, kHS, B ? B->w3 : nullptr, kHS);
+    load_matrix(W.w4_bf, kH, kOut, L.t4, kHS, B ? B->w4 : nullptr, kOutS);
     for (int i = threadIdx.x; i < kH; i += blockDim.x) {
         L.b1[i] = W.b1[i];
         L.b2[i] = W.b2[i];
@@ -133,75 +152,115 @@ AMD_INLINE void load_weights(const MlpWeights& W, MlpLds& L) {
     __syncthreads();
 }
 
-// Per-wave activation buffers: x (16 x 32), h1..h3 (16 x 64), all bf16.
+// Activations of one wave's 16-row tile, bf16: the input and two layers in
+// turn as [row][unit]; for the backward pass also every layer as [unit][row]
+// (the operands of the weights' gradients, whose sums run over rows).
 struct WaveAct {
-    unsigned short x[16 * kIn];
-    unsigned short h1[16 * kH];
-    unsigned short h2[16 * kH];
-    unsigned short h3[16 * kH];
-    unsigned short dy[16 * kOut];
-    unsigned short d3_[16 * kH];
-    unsigned short d2_[16 * kH];
-    unsigned short d1_[16 * kH];
+    alignas(16) unsigned short x[16 * kInS];
+    alignas(16) unsigned short h[2][16 * kHS];
+};
+struct WaveBack {
+    alignas(16) unsigned short xt[kIn * 16];
+    alignas(16) unsigned short ht[3][kH * 16];
+    alignas(16) unsigned short dy[16 * kOutS];
+    alignas(16) unsigned short dyt[kOut * 16];
+    alignas(16) unsigned short dt[kH * 16];
 };
 
 constexpr int kMlpWaves = 4;
 
-// dense layer: out(16 x 64) = relu(in(16 x K) W(K x 64) + b), written as bf16
-AMD_INLINE void dense_relu(const unsigned short* in, int K, const unsigned short* W, const float* bias,
-                           unsigned short* out) {
-    const int l = threadIdx.x & 63;
+// out (16 x 64) = relu(in (16 x K) W + bias); with outt also as [unit][row],
+// and with mask bit 4 t + j set where this lane's unit 16 t + 4 (l/16) + j is positive
+template <int K>
+AMD_INLINE void dense_relu(const unsigned short* wt, int ws, const unsigned short* in, int is, const float* bias,
+                           unsigned short* out, unsigned short* outt, unsigned* mask) {
+    const int col = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+    short4v b[K / 16];
+#pragma unroll
+    for (int k = 0; k < K / 16; k++) b[k] = ld4(in + col * is + k * 16 + 4 * q);
+    unsigned m = 0;
+#pragma unroll
     for (int t = 0; t < kH / 16; t++) {
         float4v c = {0, 0, 0, 0};
-        c = mfma_tile(in, K, 1, W + t * 16, kH, 1, K, c);
+#pragma unroll
+        for (int k = 0; k < K / 16; k++) c = mfma16(ld4(wt + (t * 16 + col) * ws + k * 16 + 4 * q), b[k], c);
+        unsigned short v[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            int r = (l >> 4) * 4 + j, col = t * 16 + (l & 15);
-            float v = c[j] + bias[col];
-            out[r * kH + col] = f2bf(v > 0.f ? v : 0.f);
+            const float z = c[j] + bias[t * 16 + 4 * q + j];
+            v[j] = f2bf(z > 0.f ? z : 0.f);
+            if (outt) outt[(t * 16 + 4 * q + j) * 16 + col] = v[j];
+            m |= (v[j] != 0 ? 1u : 0u) << (4 * t + j);
         }
+        st4(out + col * kHS + t * 16 + 4 * q, v);
     }
+    if (mask) *mask = m;
 }
 
-AMD_INLINE void load_x_tile(const float* X, int row0, int n, unsigned short* x) {
-    const int l = threadIdx.x & 63;
-    for (int i = l; i < 16 * kIn; i += 64) {
-        int r = i / kIn, cidx = i % kIn;
-        float v = (row0 + r < n && cidx < kMlpIn) ? X[(size_t)(row0 + r) * kMlpIn + cidx] : 0.f;
-        x[i] = f2bf(v);
+// A tile's input rows (24 floats each, row r of X at rows(r); a missing row
+// and the padding columns read 0): four lanes a row, six floats each.
+template <class F>
+AMD_INLINE void load_x_tile(const float* X, int row0, int n, F rows, unsigned short* x, unsigned short* xt) {
+    const int l = threadIdx.x & 63, r = l >> 2, c0 = 6 * (l & 3);
+    float v[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (row0 + r < n) {
+        const float2* src = reinterpret_cast<const float2*>(X + (size_t)rows(row0 + r) * kMlpIn + c0);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const float2 p = src[i];
+            v[2 * i] = p.x;
+            v[2 * i + 1] = p.y;
+        }
     }
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        const unsigned short h = f2bf(v[i]);
+        x[r * kInS + c0 + i] = h;
+        if (xt) xt[(c0 + i) * 16 + r] = h;
+    }
+}
+AMD_INLINE void clear_x_padding(unsigned short* x, unsigned short* xt) {
+    const int l = threadIdx.x & 63;
+    for (int i = l; i < 16 * (kIn - kMlpIn); i += 64) {
+        x[(i & 15) * kInS + kMlpIn + (i >> 4)] = 0;
+        if (xt) xt[kMlpIn * 16 + i] = 0;
+    }
+}
+// the output layer: lane l holds unit 4 (l/16) + j of row l%16
+AMD_INLINE float4v out_layer(const MlpLds& L, const unsigned short* h) {
+    const int col = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+    float4v c = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < kH / 16; k++)
+        c = mfma16(ld4(L.t4 + col * kHS + k * 16 + 4 * q), ld4(h + col * kHS + k * 16 + 4 * q), c);
+    return c;
 }
 
 // forward: Y[n x 3] = mlp(X[n x 24])
 __global__ __launch_bounds__(kMlpWaves * 64) void k_mlp_forward(MlpWeights W, const float* X, int n, float* Y) {
     __shared__ MlpLds L;
     __shared__ WaveAct act[kMlpWaves];
-    load_weights(W, L);
+    load_weights(W, L, nullptr);
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
     WaveAct& A = act[wave];
+    clear_x_padding(A.x, nullptr);
     const int tiles = (n + 15) / 16;
     for (int tile = blockIdx.x * kMlpWaves + wave; tile < tiles; tile += gridDim.x * kMlpWaves) {
         const int row0 = tile * 16;
-        load_x_tile(X, row0, n, A.x);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        dense_relu(A.x, kIn, L.w1, L.b1, A.h1);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        dense_relu(A.h1, kH, L.w2, L.b2, A.h2);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        dense_relu(A.h2, kH, L.w3, L.b3, A.h3);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        float4v c = {0, 0, 0, 0};
-        c = mfma_tile(A.h3, kH, 1, L.w4, kOut, 1, kH, c);
+        load_x_tile(X, row0, n, [](int r) { return r; }, A.x, nullptr);
+        wave_sync();
+        dense_relu<kIn>(L.t1, kInS, A.x, kInS, L.b1, A.h[0], nullptr, nullptr);
+        wave_sync();
+        dense_relu<kH>(L.t2, kHS, A.h[0], kHS, L.b2, A.h[1], nullptr, nullptr);
+        wave_sync();
+        dense_relu<kH>(L.t3, kHS, A.h[1], kHS, L.b3, A.h[0], nullptr, nullptr);
+        wave_sync();
+        const float4v c = out_layer(L, A.h[0]);
+        const int row = row0 + (l & 15);
+        if (l < 16 && row < n)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            int r = (l >> 4) * 4 + j, col = l & 15;
-            if (col < kMlpOut && row0 + r < n) Y[(size_t)(row0 + r) * kMlpOut + col] = c[j] + L.b4[col];
-        }
-        __builtin_amdgcn_wave_barrier();
+            for (int j = 0; j < kMlpOut; j++) Y[(size_t)row * kMlpOut + j] = c[j] + L.b4[j];
+        wave_sync();
     }
 }
 
@@ -213,149 +272,230 @@ void launch_mlp_forward(hipStream_t s, const MlpWeights& W, const float* X, int 
 }
 
 // ---------------------------------------------------------------------------
-// backward: loss = sum over rows of |y - t|^2 / n_total; gradients of every
-// weight and bias accumulated (FP32 atomics) into G.  rows = idx[0..n) of X/T.
-AMD_INLINE void grad_tile_atomic(const float4v& c, float* G, int ld, int r0, int c0, int rows, int cols) {
-    const int l = threadIdx.x & 63;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        int r = r0 + (l >> 4) * 4 + j, col = c0 + (l & 15);
-        if (r < rows && col < cols) atomicAdd(&G[r * ld + col], c[j]);
-    }
-}
+// backward: loss = sum over rows of |y - t|^2 / n_total, rows = idx[0..n) of
+// X/T (all in order when idx is null).
+//
+// Each wave keeps the gradients of every weight in matrix accumulators over
+// all its tiles (44 of 16 x 16, 176 registers: one workgroup a CU gives a wave
+// 512) and writes them once, to its own part of `partial`; k_grad_apply sums
+// the parts.  Bound by latency: the chain of layers of a tile, and at a batch
+// of 256 the copy of the weights into LDS.  Measured: 42 us for 20,001 rows
+// and 22 us for a batch of 256, the sums 11 and 5 us more.  A form that added
+// each tile's gradients to the weights with atomics spent its time on those
+// (2636 and 80 us).
 
-// dh (16 x 64) = (dnext (16 x kn) W^T) * relu'(h), W is [64][wn]; then
-// dW (kin x 64) += in^T dh and db += column sums of dh.
-AMD_INLINE void back_layer(const unsigned short* dnext, int kn, const unsigned short* W, int wn,
-                           const unsigned short* h, const unsigned short* in, int kin, unsigned short* dh, float* gw,
-                           float* gb, int gw_rows, int row0, int n) {
-    const int l = threadIdx.x & 63;
+// dh (16 x 64) = (dnext (16 x KN) W^T) * relu'(h): w is [64][KN] with stride
+// ws, dnext [row][KN]; written as [row][unit] (when dh is not null) and
+// [unit][row]; unrounded column sums go to db.
+template <int KN>
+AMD_INLINE void back_layer(const unsigned short* w, int ws, const unsigned short* dnext, int ds, unsigned mask,
+                           bool valid, unsigned short* dh, unsigned short* dt, float4v (&db)[kH / 16]) {
+    const int col = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+    short4v b[KN / 16];
+#pragma unroll
+    for (int k = 0; k < KN / 16; k++) b[k] = ld4(dnext + col * ds + k * 16 + 4 * q);
+#pragma unroll
     for (int t = 0; t < kH / 16; t++) {
         float4v c = {0, 0, 0, 0};
-        c = mfma_tile(dnext, kn, 1, W + t * 16 * wn, 1, wn, kn, c);
+#pragma unroll
+        for (int k = 0; k < KN / 16; k++) c = mfma16(ld4(w + (t * 16 + col) * ws + k * 16 + 4 * q), b[k], c);
+        unsigned short v[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            int r = (l >> 4) * 4 + j, col = t * 16 + (l & 15);
-            float hv = bf2f(h[r * kH + col]);
-            float g = hv > 0.f ? c[j] : 0.f;
-            dh[r * kH + col] = f2bf(g);
-            if (row0 + r < n) atomicAdd(&gb[col], g);
+            const float g = valid && ((mask >> (4 * t + j)) & 1u) ? c[j] : 0.f;
+            db[t][j] += g;
+            v[j] = f2bf(g);
+            dt[(t * 16 + 4 * q + j) * 16 + col] = v[j];
         }
+        if (dh) st4(dh + col * kHS + t * 16 + 4 * q, v);
     }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    for (int m = 0; m < kin / 16; m++)
-        for (int t = 0; t < kH / 16; t++) {
-            float4v c = {0, 0, 0, 0};
-            c = mfma_tile(in + m * 16, 1, kin, dh + t * 16, kH, 1, 16, c);
-            grad_tile_atomic(c, gw, kH, m * 16, t * 16, gw_rows, kH);
+}
+// dW (16 M x 64) += in^T dh over the tile's 16 rows, both as [unit][row]
+template <int M>
+AMD_INLINE void weight_grad(const unsigned short* int_, const unsigned short* dt, float4v (&g)[M][kH / 16]) {
+    const int col = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+    short4v b[kH / 16];
+#pragma unroll
+    for (int t = 0; t < kH / 16; t++) b[t] = ld4(dt + (t * 16 + col) * 16 + 4 * q);
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        const short4v a = ld4(int_ + (m * 16 + col) * 16 + 4 * q);
+#pragma unroll
+        for (int t = 0; t < kH / 16; t++) g[m][t] = mfma16(a, b[t], g[m][t]);
+    }
+}
+template <int M>
+AMD_INLINE void store_grad(const float4v (&g)[M][kH / 16], float* out) {
+    const int col = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int t = 0; t < kH / 16; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) out[(m * 16 + 4 * q + j) * kH + t * 16 + col] = g[m][t][j];
+}
+// sum over the 16 rows (lanes l % 16) of each of the lane's units
+AMD_INLINE void store_bias(const float4v (&db)[kH / 16], float* out) {
+    const int col = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int t = 0; t < kH / 16; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float v = db[t][j];
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, 64);
+            if (col == 0) out[t * 16 + 4 * q + j] = v;
         }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
 }
 
-__global__ __launch_bounds__(kMlpWaves * 64) void k_mlp_backward(MlpWeights W, const float* X, const float* T,
-                                                                 const int* idx, int n, float inv_total,
-                                                                 MlpGrads G, float* loss) {
+__global__ __launch_bounds__(kMlpWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_mlp_backward(
+    MlpWeights W, const float* X, const float* T, const int* idx, int n, float inv_total, float* partial) {
     __shared__ MlpLds L;
+    __shared__ MlpLdsBack LB;
     __shared__ WaveAct act[kMlpWaves];
-    load_weights(W, L);
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+    __shared__ WaveBack back[kMlpWaves];
+    load_weights(W, L, &LB);
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, col = l & 15, q = l >> 4;
     WaveAct& A = act[wave];
+    WaveBack& K = back[wave];
+    clear_x_padding(A.x, K.xt);
     const int tiles = (n + 15) / 16;
+    auto source = [&](int r) { return idx ? idx[r] : r; };
+    const float4v zero = {0, 0, 0, 0};
+    float4v g1[kIn / 16][kH / 16], g2[kH / 16][kH / 16], g3[kH / 16][kH / 16], g4[kH / 16];
+    float4v s1[kH / 16], s2[kH / 16], s3[kH / 16], s4 = zero;
+#pragma unroll
+    for (int t = 0; t < kH / 16; t++) {
+#pragma unroll
+        for (int m = 0; m < kH / 16; m++) {
+            if (m < kIn / 16) g1[m][t] = zero;
+            g2[m][t] = zero;
+            g3[m][t] = zero;
+        }
+        g4[t] = s1[t] = s2[t] = s3[t] = zero;
+    }
     float my_loss = 0.f;
     for (int tile = blockIdx.x * kMlpWaves + wave; tile < tiles; tile += gridDim.x * kMlpWaves) {
         const int row0 = tile * 16;
-        for (int i = l; i < 16 * kIn; i += 64) {
-            int r = i / kIn, cidx = i % kIn;
-            float v = 0.f;
-            if (row0 + r < n && cidx < kMlpIn) v = X[(size_t)idx[row0 + r] * kMlpIn + cidx];
-            A.x[i] = f2bf(v);
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        dense_relu(A.x, kIn, L.w1, L.b1, A.h1);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        dense_relu(A.h1, kH, L.w2, L.b2, A.h2);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        dense_relu(A.h2, kH, L.w3, L.b3, A.h3);
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // output layer and dL/dy = 2 (y - t) / n_total
-        {
-            float4v c = {0, 0, 0, 0};
-            c = mfma_tile(A.h3, kH, 1, L.w4, kOut, 1, kH, c);
+        const bool valid = row0 + col < n;
+        unsigned m1, m2, m3;
+        load_x_tile(X, row0, n, source, A.x, K.xt);
+        wave_sync();
+        dense_relu<kIn>(L.t1, kInS, A.x, kInS, L.b1, A.h[0], K.ht[0], &m1);
+        wave_sync();
+        dense_relu<kH>(L.t2, kHS, A.h[0], kHS, L.b2, A.h[1], K.ht[1], &m2);
+        wave_sync();
+        dense_relu<kH>(L.t3, kHS, A.h[1], kHS, L.b3, A.h[0], K.ht[2], &m3);
+        wave_sync();
+        // output layer and dL/dy = 2 (y - t) / n_total: units 0-2 sit in lanes 0-15
+        const float4v c = out_layer(L, A.h[0]);
+        unsigned short d[4] = {0, 0, 0, 0};
+        if (q == 0 && valid) {
+            const float* want = T + (size_t)source(row0 + col) * kMlpOut;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                int r = (l >> 4) * 4 + j, col = l & 15;
-                float g = 0.f;
-                if (col < kMlpOut && row0 + r < n) {
-                    float y = c[j] + L.b4[col];
-                    float t = T[(size_t)idx[row0 + r] * kMlpOut + col];
-                    float e = y - t;
-                    my_loss += e * e * inv_total;
-                    g = 2.f * e * inv_total;
-                    atomicAdd(&G.b4[col], g);
-                }
-                A.dy[r * kOut + col] = f2bf(g);
+            for (int j = 0; j < kMlpOut; j++) {
+                const float e = c[j] + L.b4[j] - want[j];
+                my_loss += e * e * inv_total;
+                const float g = 2.f * e * inv_total;
+                s4[j] += g;
+                d[j] = f2bf(g);
             }
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // dW4 (64 x 16) += h3^T (64 x 16 rows) dy (16 x 16)
-        for (int m = 0; m < kH / 16; m++) {
-            float4v c = {0, 0, 0, 0};
-            c = mfma_tile(A.h3 + m * 16, 1, kH, A.dy, kOut, 1, 16, c);
-            grad_tile_atomic(c, G.w4, kOut, m * 16, 0, kH, kMlpOut);
+        st4(K.dy + col * kOutS + 4 * q, d);
+#pragma unroll
+        for (int j = 0; j < 4; j++) K.dyt[(4 * q + j) * 16 + col] = d[j];
+        wave_sync();
+        // dW4 (64 x 16) += h3^T dy
+        {
+            const short4v b = ld4(K.dyt + col * 16 + 4 * q);
+#pragma unroll
+            for (int m = 0; m < kH / 16; m++) g4[m] = mfma16(ld4(K.ht[2] + (m * 16 + col) * 16 + 4 * q), b, g4[m]);
         }
-        // back through layers 3, 2, 1: dh = (d_next W^T) * relu'(h)
-        back_layer(A.dy, kOut, L.w4, kOut, A.h3, A.h2, kH, A.d3_, G.w3, G.b3, kH, row0, n);
-        back_layer(A.d3_, kH, L.w3, kH, A.h2, A.h1, kH, A.d2_, G.w2, G.b2, kH, row0, n);
-        back_layer(A.d2_, kH, L.w2, kH, A.h1, A.x, kIn, A.d1_, G.w1, G.b1, kMlpIn, row0, n);
-        __builtin_amdgcn_wave_barrier();
+        // back through layers 3, 2, 1
+        back_layer<kOut>(LB.w4, kOutS, K.dy, kOutS, m3, valid, A.h[1], K.dt, s3);
+        wave_sync();
+        weight_grad<kH / 16>(K.ht[1], K.dt, g3);
+        wave_sync();
+        back_layer<kH>(LB.w3, kHS, A.h[1], kHS, m2, valid, A.h[0], K.dt, s2);
+        wave_sync();
+        weight_grad<kH / 16>(K.ht[0], K.dt, g2);
+        wave_sync();
+        back_layer<kH>(LB.w2, kHS, A.h[0], kHS, m1, valid, nullptr, K.dt, s1);
+        wave_sync();
+        weight_grad<kIn / 16>(K.xt, K.dt, g1);
+        wave_sync();
     }
-    // loss reduction
+    float* out = partial + (size_t)(blockIdx.x * kMlpWaves + wave) * kPartial;
+    store_grad(g1, out);
+    out += kPadW1;
+    store_grad(g2, out);
+    out += kPadW2;
+    store_grad(g3, out);
+    out += kPadW3;
+#pragma unroll
+    for (int m = 0; m < kH / 16; m++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) out[(m * 16 + 4 * q + j) * kOut + col] = g4[m][j];
+    out += kPadW4;
+    store_bias(s1, out);
+    store_bias(s2, out + kPadB1);
+    store_bias(s3, out + kPadB1 + kPadB2);
+    out += kPadB1 + kPadB2 + kPadB3;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float v = s4[j];
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, 64);
+        if (col == 0) out[4 * q + j] = v;
+    }
     for (int o = 32; o > 0; o >>= 1) my_loss += __shfl_xor(my_loss, o, 64);
-    if (l == 0 && loss) atomicAdd(loss, my_loss);
+    if (l == 0) out[kPadB4] = my_loss;
 }
 
-void launch_mlp_backward(hipStream_t s, const MlpWeights& W, const float* X, const float* T, const int* idx, int n,
-                         float inv_total, const MlpGrads& G, float* loss) {
-    if (n <= 0) return;
-    int tiles = (n + 15) / 16;
-    int blocks = std::min((tiles + kMlpWaves - 1) / kMlpWaves, 512);
-    hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(kMlpWaves * 64), 0, s, W, X, T, idx, n, inv_total, G, loss);
-}
-
-// ---------------------------------------------------------------------------
-// Adam on the FP32 master weights, then BF16 copies; gradients cleared.
-__global__ void k_adam(float* p, float* g, float* m, float* v, unsigned short* bf, int n, float lr, float b1,
-                       float b2, float eps, float c1, float c2, const unsigned char* mask) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float gi = g[i];
-    g[i] = 0.f;
-    if (mask && !mask[i]) {
-        if (bf) bf[i] = f2bf(p[i]);
+// Sums the waves' partial gradients in a fixed order, 64 parameters a
+// workgroup, 16 threads each (a thread alone would walk the parts of all the
+// waves one load after the other); then, with P.p set, the Adam update of the
+// FP32 master weights and their BF16 copies, else the sums go to P.g.  The
+// last entry is the loss, added to *loss.
+__global__ __launch_bounds__(1024) void k_grad_apply(AdamArgs P, const float* partial, int parts, float* loss) {
+    __shared__ float sum[16][64];
+    const int e = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + e;
+    float g = 0.f;
+    if (i <= kPadTotal)
+        for (int k = w; k < parts; k += 16) g += partial[(size_t)k * kPartial + i];
+    sum[w][e] = g;
+    __syncthreads();
+    if (w != 0 || i > kPadTotal) return;
+#pragma unroll
+    for (int k = 1; k < 16; k++) g += sum[k][e];
+    if (i == kPadTotal) {
+        *loss += g;
         return;
     }
-    float mi = b1 * m[i] + (1.f - b1) * gi;
-    float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    p[i] = pi;
-    if (bf) bf[i] = f2bf(pi);
+    if (!P.p) {
+        P.g[i] = g;
+        return;
+    }
+    float mi = P.b1 * P.m[i] + (1.f - P.b1) * g;
+    float vi = P.b2 * P.v[i] + (1.f - P.b2) * g * g;
+    P.m[i] = mi;
+    P.v[i] = vi;
+    float pi = P.p[i] - P.lr * (mi / P.c1) / (sqrtf(vi / P.c2) + P.eps);
+    P.p[i] = pi;
+    if (i < kPadWeights) P.bf[i] = f2bf(pi);
 }
 
-void launch_adam(hipStream_t s, float* p, float* g, float* m, float* v, unsigned short* bf, int n, float lr, float b1,
-                 float b2, float eps, int step, const unsigned char* mask) {
+// Workgroups of the backward pass: a 16-row tile a wave up to 512 waves.
+static int backward_blocks(int n) { return std::min(((n + 15) / 16 + kMlpWaves - 1) / kMlpWaves, 128); }
+size_t mlp_partial_floats(int n) { return (size_t)backward_blocks(n) * kMlpWaves * kPartial; }
+
+void launch_mlp_backward(hipStream_t s, const MlpWeights& W, const float* X, const float* T, const int* idx, int n,
+                         float inv_total, float* partial, const AdamArgs& P, float* loss) {
     if (n <= 0) return;
-    float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    hipLaunchKernelGGL(k_adam, dim3((n + 255) / 256), dim3(256), 0, s, p, g, m, v, bf, n, lr, b1, b2, eps, c1, c2,
-                       mask);
+    const int blocks = backward_blocks(n);
+    hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(kMlpWaves * 64), 0, s, W, X, T, idx, n, inv_total, partial);
+    hipLaunchKernelGGL(k_grad_apply, dim3(kPadTotal / 64 + 1), dim3(1024), 0, s, P, partial, blocks * kMlpWaves, loss);
 }
 
 __global__ void k_to_bf16(const float* p, unsigned short* bf, int n) {

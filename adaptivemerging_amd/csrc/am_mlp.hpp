@@ -37,29 +37,32 @@ struct MlpWeights {
     const float* b4;
 };
 
-// FP32 gradients in the same padded layout.
-struct MlpGrads {
-    float* w1;
-    float* w2;
-    float* w3;
-    float* w4;
-    float* b1;
-    float* b2;
-    float* b3;
-    float* b4;
-};
-
 // padded sizes
 constexpr int kPadW1 = 32 * 64, kPadW2 = 64 * 64, kPadW3 = 64 * 64, kPadW4 = 64 * 16;
 constexpr int kPadB1 = 64, kPadB2 = 64, kPadB3 = 64, kPadB4 = 16;
-constexpr int kPadTotal = kPadW1 + kPadW2 + kPadW3 + kPadW4 + kPadB1 + kPadB2 + kPadB3 + kPadB4;
+constexpr int kPadWeights = kPadW1 + kPadW2 + kPadW3 + kPadW4;
+constexpr int kPadTotal = kPadWeights + kPadB1 + kPadB2 + kPadB3 + kPadB4;
+// one wave's gradients in the same layout, then its part of the loss (and a pad to whole cache lines)
+constexpr int kPartial = kPadTotal + 16;
+
+// Adam on the padded parameters (p null: the gradients go to g instead).
+struct AdamArgs {
+    float* g;
+    float* p;
+    float* m;
+    float* v;
+    unsigned short* bf;
+    float lr, b1, b2, eps;
+    float c1, c2;  // 1 - b1^step, 1 - b2^step
+};
 
 void launch_features(hipStream_t s, const FeatureArgs& F);
 void launch_mlp_forward(hipStream_t s, const MlpWeights& W, const float* X, int n, float* Y);
+// floats of workspace (`partial`) a backward pass over n rows needs
+size_t mlp_partial_floats(int n);
+// adds the batch's loss to *loss
 void launch_mlp_backward(hipStream_t s, const MlpWeights& W, const float* X, const float* T, const int* idx, int n,
-                         float inv_total, const MlpGrads& G, float* loss);
-void launch_adam(hipStream_t s, float* p, float* g, float* m, float* v, unsigned short* bf, int n, float lr, float b1,
-                 float b2, float eps, int step, const unsigned char* mask);
+                         float inv_total, float* partial, const AdamArgs& P, float* loss);
 void launch_to_bf16(hipStream_t s, const float* p, unsigned short* bf, int n);
 void launch_apply_prediction(hipStream_t s, ContactsView C, BodiesView B, const float* Y, const double* scale, int n,
                              int fric_ovr, double fric_val, double* lam_out);

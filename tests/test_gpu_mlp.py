@@ -62,6 +62,30 @@ def test_mlp_gradients_match_fp64_reference(gpu_lib):
     np.testing.assert_allclose(G, Gr, rtol=2e-3, atol=2e-4 * scale)
 
 
+# tiles of 16 rows, four a workgroup, 512 at once: around one tile, one
+# workgroup and one pass of all waves.  Tolerances as above: FP32 sums against
+# FP64 ones differ by about 1e-6, and a sum that crosses a BF16 rounding point
+# moves one of a row's 195 units by 2^-9 of itself.
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 8192, 8193])
+def test_mlp_gradients_at_tile_edges(gpu_lib, n):
+    ctx = Context()
+    rng = np.random.default_rng(n)
+    p = (rng.normal(size=_lib.MLP_PARAMS) * 0.2).astype(np.float32)
+    mlp_call(ctx, "am_mlp_set_params", _lib.ptr(p), len(p))
+    X = rng.normal(size=(n, 24)).astype(np.float32)
+    T = rng.normal(size=(n, 3)).astype(np.float32)
+    Y = np.zeros((n, 3), np.float32)
+    mlp_call(ctx, "am_mlp_forward", _lib.ptr(X), n, _lib.ptr(Y))
+    np.testing.assert_allclose(Y, mlp_ref.forward(p, X)[0], rtol=5e-3, atol=5e-3)
+    loss = C.c_float()
+    G = np.zeros(_lib.MLP_PARAMS, np.float32)
+    for _ in range(2):  # the workspace is kept: a second call must not add to the first
+        mlp_call(ctx, "am_mlp_gradients", _lib.ptr(X), _lib.ptr(T), n, _lib.ptr(G), C.byref(loss))
+    Gr, lr = mlp_ref.gradients(p, X, T)
+    assert abs(loss.value - lr) < 1e-4 * max(1.0, lr)
+    np.testing.assert_allclose(G, Gr, rtol=2e-3, atol=2e-4 * np.max(np.abs(Gr)))
+
+
 def test_training_reduces_loss(gpu_lib):
     """Pairs come only from solves that reach the tolerance: a shallow pile of
     100 boxes, whose solves reach 1e-6 within the cap."""
