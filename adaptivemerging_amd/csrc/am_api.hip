@@ -456,7 +456,7 @@ int build_layout(am_ctx* c) {
         launch_colour_keys(s, ng, cin, c->g_start.p, c->g_keys.p);
         sort_u64(s, c->g_keys.p, c->g_keys_sorted.p, ng, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
     }
-    AM_HIP(c, c->s_colour_start.ensure(kMaxColours + 2));
+    AM_HIP(c, c->s_colour_start.ensure(kMaxColours + 4));
     AM_HIP(c, c->s_group_desc.ensure((size_t)std::max(ng, 1) * 4));
     launch_colour_layout(s, ng, c->g_keys_sorted.p, c->g_start.p, c->g_a.p, c->g_b.p, c->s_colour_start.p,
                          c->g_sizes.p, c->g_pos_start.p, c->s_order.p, c->s_group_desc.p, c->s_pos_a.p,
@@ -465,10 +465,23 @@ int build_layout(am_ctx* c) {
     AM_HIP(c, c->s_pred.ensure((size_t)std::max(ng, 1) * 2));
     launch_flow_ranks(s, c->n_ent, ng, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p, c->g_spos.p,
                       c->s_group_desc.p, c->s_flow.p, c->s_pred.p);
+    if (c->resident_max_grid == 0) {
+        bool ok = false;
+        c->resident_max_grid = pgs_resident_max_blocks(&ok);
+        if (!ok) c->resident_max_grid = -1;
+    }
+    AM_HIP(c, c->s_used.ensure(kResidentMaxWaves));
+    // a group a wave as far as there are waves
+    const int rgrid = std::min((std::min(ng, kResidentMaxWaves) + 3) / 4, c->resident_max_grid);
+    if (rgrid > 0)
+        launch_resident_plan(s, c->s_colour_start.p, c->s_group_desc.p, 4 * rgrid, c->s_used.p,
+                             c->s_colour_start.p + kMaxColours + 2);
     AM_HIP(c, hipGetLastError());
-    int cs[kMaxColours + 2];
+    int cs[kMaxColours + 4];
     AM_HIP(c, hipMemcpyAsync(cs, c->s_colour_start.p, sizeof cs, hipMemcpyDeviceToHost, s));
     AM_HIP(c, hipStreamSynchronize(s));
+    const bool fits = rgrid > 0 && cs[kMaxColours + 2] <= kResidentDoubles && cs[kMaxColours + 3] <= kResidentSteps;
+    c->resident_grid = fits ? rgrid : 0;
     int ncol = 0, maxc = 0;
     for (int q = 0; q <= kMaxColours; q++) {
         int sz = cs[q + 1] - cs[q];
@@ -748,6 +761,18 @@ int start_residual(am_ctx* c, PgsArgs G, double* out) {
 // threads per workgroup, clamped to what can be co-resident.
 void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
     bool ok = false;
+    // Everything resident in LDS wherever it fits: it was the faster on every
+    // contact set tried (us per sweep, k_pgs_flow -> resident, by contacts: 12:
+    // 9 -> 6.3; 1,100 in a tower, one long chain: 24 -> 24; 750 between sphere
+    // trees, up to 60 in a group: 46 -> 26; 5,000 in a pile: 30 -> 22; 37,000:
+    // 47 -> 27; 8,000 in one colour: 13 -> 5.4; 27,000 in 48 scenes: 47 -> 30).
+    // Its arrival words take 1 KiB a sweep, hence the bound on the sweeps.  A
+    // given pgs_grid asks for k_pgs_flow.
+    if (P.pgs_schedule == 0 && P.pgs_grid == 0 && c->resident_grid > 0 && P.iterations <= kResidentMaxSweeps) {
+        *grid = c->resident_grid;
+        *block = kResidentThreads;
+        return;
+    }
     if (P.pgs_schedule == 0) {
         if (c->flow_max_grid == 0) {
             c->flow_max_grid = pgs_flow_max_blocks(&ok);
@@ -919,9 +944,11 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         AM_HIP(c, c->dv_alt.ensure(std::max(n_dv, (size_t)6)));
         const size_t n_slot = (size_t)2 * 2 * std::max(c->n_groups, 1) * kSlotDoubles;
         AM_HIP(c, c->f_slot.ensure(n_slot));
-        AM_HIP(c, c->d_pass_done.ensure((size_t)(iterations + 2) * kPassWords));
+        const size_t n_pass = block == kResidentThreads ? ((size_t)(iterations + 1) * kPassWords + 1) * kPassStride
+                                                        : (size_t)(iterations + 2) * kPassWords;
+        AM_HIP(c, c->d_pass_done.ensure(n_pass));
         fill_u64(s, c->f_slot.p, n_slot, kSlotEmpty);
-        fill_int(s, (int*)c->d_pass_done.p, 2 * (iterations + 2) * kPassWords, 0);
+        fill_u64(s, c->d_pass_done.p, n_pass, 0);
         AM_HIP(c, hipMemcpyAsync(c->dv_alt.p, c->d_dv.p, n_dv * sizeof(double), hipMemcpyDeviceToDevice, s));
         const int fgrid = grid;
         FlowArgs F;
@@ -933,11 +960,12 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         F.dv_alt = c->dv_alt.p;
         F.lam_alt = c->s_lam_alt.p;
         F.pass_done = c->d_pass_done.p;
+        F.resident_used = c->s_used.p;
         F.n_waves = (unsigned)fgrid;
         S.lam_alt = c->s_lam_alt.p;
         S.iters_used = G.iters_used;
         AM_HIP(c, hipEventRecord(c->kev[1], s));
-        AM_HIP(c, launch_pgs_flow(s, F, fgrid, P.pgs_plain_launch != 0, (int)n_dv, bodies_view(c)));
+        AM_HIP(c, launch_pgs_flow(s, F, fgrid, block, P.pgs_plain_launch != 0, (int)n_dv, bodies_view(c)));
         AM_HIP(c, hipEventRecord(c->kev[2], s));
     } else {
         AM_HIP(c, hipEventRecord(c->kev[1], s));

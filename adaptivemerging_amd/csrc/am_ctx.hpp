@@ -172,11 +172,13 @@ struct am_ctx {
     DBuf<unsigned long long> s_iter_max;
     // dataflow schedule: sorted position per group, ranks and degrees, previous-update
     // incidences, pass completion counts, deltaV slots, odd-pass buffers
-    DBuf<int> g_spos, s_flow, s_pred;
+    DBuf<int> g_spos, s_flow, s_pred, s_used;
     DBuf<unsigned long long> d_pass_done;
     DBuf<double> f_slot;
     DBuf<double> dv_alt, s_lam_alt;
     int flow_max_grid = 0;
+    int resident_max_grid = 0;  // co-resident workgroups of the resident kernel (-1: none)
+    int resident_grid = 0;      // workgroups it takes on the current layout, 0 where it does not fit
     // poses advanced by dt for the position-level motion metric
     DBuf<double> pose_xa, pose_Ra;
     // springs (RigidBodySystem.springs)

@@ -149,23 +149,22 @@ constexpr int kTreeStack = 128;
 constexpr int kMaxColours = 64;     // colours 0..63 run in parallel; 64 is the sequential tail
 
 // Solve record: the per-contact data the PGS sweep reads, packed in sweep order.
-// Per row (n, t1, t2), 15 doubles: ja.w, jb.v, jb.w (ja.v = -jb.v exactly),
-// then jinv_a ja.w and jinv_b jb.w (constant during a solve, so computed once
-// in setup with the same operations the update would do).  Then b[3], D[3],
-// mu, lambda[3] (read and written in place), the solve bodies a | b << 32 as
-// raw bits, the clamp flag, then D + C [3] and the refined reciprocals of
-// D + C [3] (the dataflow sweep's division), one pad: 64 doubles (512 B,
+// Per row (n, t1, t2), five quads of 4 doubles: jb.v (ja.v = -jb.v exactly),
+// ja.w, jb.w, jinv_a ja.w, jinv_b jb.w (the products are constant during a
+// solve, so computed once in setup with the same operations the update would
+// do), each with a scalar behind its 3 components: b, D, D + C, the refined
+// reciprocal of D + C (the dataflow sweeps' division), and behind the last quad
+// of the rows mu, the clamp flag and the solve bodies a | b << 32 as raw bits.
+// Then lambda[3] (read and written in place) and a pad: 64 doubles (512 B,
 // 16-byte aligned).
 constexpr int kRecDoubles = 64;
-constexpr int kRecRow = 15;
-constexpr int kRecB = 45;
-constexpr int kRecD = 48;
-constexpr int kRecMu = 51;
-constexpr int kRecLambda = 52;
-constexpr int kRecAB = 55;
-constexpr int kRecClamp = 56;
-constexpr int kRecDen = 57;
-constexpr int kRecY = 60;
+constexpr int kRecRow = 20;
+constexpr int kRecBv = 0, kRecAw = 4, kRecBw = 8, kRecTa = 12, kRecTb = 16;  // in a row
+constexpr int kRecB = 3, kRecD = 7, kRecDen = 11, kRecY = 15;                // in a row
+constexpr int kRecMu = 19;
+constexpr int kRecClamp = kRecRow + 19;
+constexpr int kRecAB = 2 * kRecRow + 19;
+constexpr int kRecLambda = 3 * kRecRow;
 
 // ---- launchers (am_detect.hip) ----
 struct PairArgs {

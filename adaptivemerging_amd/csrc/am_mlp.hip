@@ -584,10 +584,11 @@ __global__ void k_start_residual(const double* rec, const int* meta, const doubl
         double lam[3] = {R[kRecLambda], R[kRecLambda + 1], R[kRecLambda + 2]};
         for (int r = 0; r < 3; r++) {
             const double* q = R + r * kRecRow;
-            double jd = (-q[3] * da[0] + -q[4] * da[1] + -q[5] * da[2]) + (q[0] * da[3] + q[1] * da[4] + q[2] * da[5]) +
-                        (q[3] * db[0] + q[4] * db[1] + q[5] * db[2]) + (q[6] * db[3] + q[7] * db[4] + q[8] * db[5]);
-            double D = R[kRecD + r];
-            double l = (D * lam[r] - omega * (R[kRecB + r] + jd)) / (D + compliance);
+            const double *bv = q + kRecBv, *aw = q + kRecAw, *bw = q + kRecBw;
+            double jd = (-bv[0] * da[0] + -bv[1] * da[1] + -bv[2] * da[2]) + (aw[0] * da[3] + aw[1] * da[4] + aw[2] * da[5]) +
+                        (bv[0] * db[0] + bv[1] * db[1] + bv[2] * db[2]) + (bw[0] * db[3] + bw[1] * db[4] + bw[2] * db[5]);
+            double D = q[kRecD];
+            double l = (D * lam[r] - omega * (q[kRecB] + jd)) / (D + compliance);
             if (m.z) {
                 if (r == 0) l = fmax(0.0, l);
                 else l = fmin(fmax(l, -R[kRecMu] * lam[0]), R[kRecMu] * lam[0]);

@@ -217,10 +217,14 @@ __global__ void k_colour_keys(int n_groups, const int* colour, const int* group_
 
 // colour_start[c] = first sorted position with colour >= c, c = 0..kMaxColours;
 // colour_start[kMaxColours + 1] = n_groups (the tail holds every colour from
-// kMaxColours on, in colour order)
+// kMaxColours on, in colour order); the two words after it are cleared for
+// k_resident_plan
 __global__ void k_colour_starts(int n_groups, const uint64_t* sorted, int* colour_start) {
     int c = threadIdx.x;
-    if (c > kMaxColours + 1) return;
+    if (c > kMaxColours + 1) {
+        if (c < kMaxColours + 4) colour_start[c] = 0;
+        return;
+    }
     if (c == kMaxColours + 1) {
         colour_start[c] = n_groups;
         return;
@@ -434,26 +438,21 @@ __global__ void k_setup(SetupArgs S) {
         const double* J0 = Jr + row * 12;
         double* q = rec + row * kRecRow;
         if (!flip) {
-            st3(q + 0, ld3(J0 + 3));   // ja.w
-            st3(q + 3, ld3(J0 + 6));   // jb.v
-            st3(q + 6, ld3(J0 + 9));   // jb.w
-            st3(q + 9, ta[row]);
-            st3(q + 12, tb[row]);
+            st3(q + kRecBv, ld3(J0 + 6));
+            st3(q + kRecAw, ld3(J0 + 3));
+            st3(q + kRecBw, ld3(J0 + 9));
+            st3(q + kRecTa, ta[row]);
+            st3(q + kRecTb, tb[row]);
         } else {
-            st3(q + 0, ld3(J0 + 9));   // jb.w
-            st3(q + 3, ld3(J0 + 0));   // ja.v = -jb.v
-            st3(q + 6, ld3(J0 + 3));   // ja.w
-            st3(q + 9, tb[row]);
-            st3(q + 12, ta[row]);
+            st3(q + kRecBv, ld3(J0 + 0));  // ja.v = -jb.v
+            st3(q + kRecAw, ld3(J0 + 9));
+            st3(q + kRecBw, ld3(J0 + 3));
+            st3(q + kRecTa, tb[row]);
+            st3(q + kRecTb, ta[row]);
         }
     }
     const int ea = flip ? b : a, eb = flip ? a : b;
-    rec[kRecB + 0] = bn;
-    rec[kRecB + 1] = bt1;
-    rec[kRecB + 2] = bt2;
-    rec[kRecD + 0] = D[0];
-    rec[kRecD + 1] = D[1];
-    rec[kRecD + 2] = D[2];
+    const double bs[3] = {bn, bt1, bt2};
     rec[kRecMu] = contact_mu(B.desc[b1], B.desc[b2], S.fric_ovr, S.fric_val);
 #pragma unroll
     for (int r = 0; r < 3; r++) rec[kRecLambda + r] = C.lam[c * 3 + r];
@@ -462,10 +461,13 @@ __global__ void k_setup(SetupArgs S) {
     bool recips = true;
 #pragma unroll
     for (int r = 0; r < 3; r++) {
-        const double den = rec[kRecD + r] + S.compliance;
-        rec[kRecDen + r] = den;
-        rec[kRecY + r] = div_recip(den);
-        recips = recips && rec[kRecY + r] != 0.0;
+        double* q = rec + r * kRecRow;
+        const double den = D[r] + S.compliance, y = div_recip(den);
+        q[kRecB] = bs[r];
+        q[kRecD] = D[r];
+        q[kRecDen] = den;
+        q[kRecY] = y;
+        recips = recips && y != 0.0;
     }
     // 0: not clamped; 1: clamped, every row's reciprocal stored (the
     // dataflow kernel's fast update may take it); 2: clamped otherwise
@@ -496,8 +498,8 @@ __global__ void k_unpack(SetupArgs S) {
 #pragma unroll
     for (int r = 0; r < 3; r++) {
         C.lam[c * 3 + r] = rec[kRecLambda + r];
-        C.b[c * 3 + r] = rec[kRecB + r];
-        C.D[c * 3 + r] = rec[kRecD + r];
+        C.b[c * 3 + r] = rec[r * kRecRow + kRecB];
+        C.D[c * 3 + r] = rec[r * kRecRow + kRecD];
     }
     C.state[c] = S.sstate[k];
 }
@@ -543,8 +545,7 @@ struct Row {
 };
 AMD_INLINE Row row_of(const double* rec, int r) {
     const double* q = rec + r * kRecRow;
-    return Row{mk(q[0], q[1], q[2]), mk(q[3], q[4], q[5]), mk(q[6], q[7], q[8]), mk(q[9], q[10], q[11]),
-               mk(q[12], q[13], q[14])};
+    return Row{ld3(q + kRecAw), ld3(q + kRecBv), ld3(q + kRecBw), ld3(q + kRecTa), ld3(q + kRecTb)};
 }
 
 // PGS.updateDeltaVwithLambdai (PGS.java:221-245)
@@ -574,13 +575,12 @@ AMD_INLINE double jdv(const Row& R, const BodyRegs& A, const BodyRegs& Bb) {
 }
 
 constexpr int kRec2 = kRecDoubles / 2;  // 16-byte words per record
-constexpr int kRecLoad = 58;            // the coloured sweep reads up to the clamp flag
 struct Rec {
-    double v[kRecLoad];
+    double v[kRecDoubles];
 };
 AMD_INLINE void load_rec(const double2* src, Rec& r) {
 #pragma unroll
-    for (int i = 0; i < kRecLoad / 2; i++) {
+    for (int i = 0; i < kRec2; i++) {
         double2 t = src[i];
         r.v[2 * i] = t.x;
         r.v[2 * i + 1] = t.y;
@@ -614,8 +614,8 @@ AMD_INLINE void process_group(const PgsArgs& P, int4 gd, const double2* recs, in
                 Row R = row_of(rec, r);
                 double Jd = jdv(R, ra, rb);
                 double prev = lam[r];
-                double Dr = rec[kRecD + r];
-                double l = (Dr * lam[r] - omega * (rec[kRecB + r] + Jd)) / (Dr + P.compliance);
+                double Dr = rec[r * kRecRow + kRecD];
+                double l = (Dr * lam[r] - omega * (rec[r * kRecRow + kRecB] + Jd)) / (Dr + P.compliance);
                 if (clamp) {
                     if (r == 0) {
                         l = jmax(0, l);
@@ -638,8 +638,8 @@ AMD_INLINE void process_group(const PgsArgs& P, int4 gd, const double2* recs, in
             dst[2] = lam[2];
             if (last_iter) {
                 // Contact.updateContactState (Contact.java:385-398)
-                double w1 = rec[kRecB + 1] + jdv(row_of(rec, 1), ra, rb);
-                double w2 = rec[kRecB + 2] + jdv(row_of(rec, 2), ra, rb);
+                double w1 = rec[kRecRow + kRecB] + jdv(row_of(rec, 1), ra, rb);
+                double w2 = rec[2 * kRecRow + kRecB] + jdv(row_of(rec, 2), ra, rb);
                 int st;
                 if (fabs(lam[0]) <= 1e-14) st = AM_STATE_BROKEN;
                 else if (fabs(w1) > P.sliding) st = AM_STATE_ONEDGE;
@@ -919,8 +919,8 @@ struct LaneMap {
 AMD_INLINE LaneMap lane_map(int li) {
     const int q = li >> 2, j = (li & 3) < 3 ? (li & 3) : 0;
     LaneMap m;
-    m.jofs = (q == 1 ? 0 : q == 3 ? 6 : 3) + j;
-    m.cofs = q == 1 ? 9 + j : q == 3 ? 12 + j : m.jofs;
+    m.jofs = (q == 1 ? kRecAw : q == 3 ? kRecBw : kRecBv) + j;
+    m.cofs = q == 1 ? kRecTa + j : q == 3 ? kRecTb + j : m.jofs;
     m.sign = q == 0 ? 0x80000000u : 0u;
     return m;
 }
@@ -938,12 +938,13 @@ AMD_INLINE void read_wave_rec(const double* rec, const double* lam, const LaneMa
     w.sign = m.sign;
 #pragma unroll
     for (int r = 0; r < 3; r++) {
-        w.jc[2 * r] = rec[r * kRecRow + m.jofs];
-        w.jc[2 * r + 1] = rec[r * kRecRow + m.cofs];
-        w.b[r] = rec[kRecB + r];
-        w.d[r] = rec[kRecD + r];
-        w.den[r] = rec[kRecDen + r];
-        w.y[r] = rec[kRecY + r];
+        const double* q = rec + r * kRecRow;
+        w.jc[2 * r] = q[m.jofs];
+        w.jc[2 * r + 1] = q[m.cofs];
+        w.b[r] = q[kRecB];
+        w.d[r] = q[kRecD];
+        w.den[r] = q[kRecDen];
+        w.y[r] = q[kRecY];
         w.lam[r] = lam[r];
     }
     w.mu = rec[kRecMu];
@@ -1504,18 +1505,842 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     }
 }
 
+// ---------------------------------------------------------------------------
+// The dataflow schedule with everything that a wave needs resident in LDS.
+//
+// Where the solve fits (kResDoubles of LDS for the four waves of each CU: about
+// 55,000 contacts), every wave keeps its groups' records, lambdas and
+// bookkeeping in LDS for the whole solve, and a pass reads no global memory
+// but the slots.  What bounds it is the chain of dependent group updates, a
+// link of which costs the handoff of deltaV (0.4 us between CUs) and the
+// contacts' arithmetic.  So the arithmetic is laid out for latency:
+//  - A quad of lanes holds a group (A.v, A.w, B.v, B.w, three components
+//    each): a row's J.dv is three products and two additions per lane and two
+//    DPP exchanges, where a 16-lane row with one component per lane needs two
+//    more stages.  16 groups of a colour share a wave's instructions.
+//  - Friction limits are applied with min and max, not compares and selects
+//    (46 cycles a bound, against 10).
+//  - The next contact's record is read while the current one runs, the first
+//    one's while the wave waits for its inputs.
+//  - Nothing waits before a publish, and the slot that was read is emptied
+//    after it.  It must be seen empty before its next writer fills it; that
+//    writer comes after this group's own publish of the next pass (the body's
+//    updates are one chain), and the stores of this pass have landed by the
+//    wait after that pass's poll.
+//  - A body with a single group hands its deltaV to itself through LDS.
+// The gates between passes are kept by a fifth wave of each workgroup: it
+// reports the passes its workgroup's waves have finished, follows the sweeps'
+// verdicts, and leaves both in LDS, where a sweeping wave finds them without
+// a global read.
+//
+// Groups are spread over all waves: a step takes ceil(groups of the colour /
+// waves) groups, at most 16, so a colour is one step per wave while it can be.
+// Measured (per sweep, against k_pgs_flow): see the dispatch in pgs_shape.
+constexpr int kResWaves = 4;                        // sweeping waves of a workgroup
+constexpr int kQuads = 16;                          // groups of a step
+constexpr int kResDoubles = kResidentDoubles;       // LDS of a workgroup's waves together
+// A contact in LDS.  Per row, what each kind of lane reads (its J entries, then
+// its update coefficients) as 6 doubles in a row, three 16-byte reads: jb.v
+// twice for the v lanes, ja.w and jinv_a ja.w, jb.w and jinv_b jb.w; then b, D,
+// D + C and its reciprocal of each row; then lambda and mu, once for even and
+// once for odd passes.  A wave issues an LDS read every 20 cycles or so, so a
+// contact is laid out for few of them (17; 21 with the records' own layout).
+constexpr int kResRow = 18, kResV = 0, kResAw = 6, kResBw = 12;
+constexpr int kResScalars = 3 * kResRow;  // 4 a row
+constexpr int kResLam = kResScalars + 12, kResLamOdd = kResLam + 4;
+constexpr int kResContact = kResLamOdd + 4;
+// per group, for each side: deltaV (6) of a body that is only this group's or
+// pinned, minv, {LDS offset of the first contact, contacts}, {body, incidence of
+// its previous update, flags, scene (side A) or the scene's groups (side B)}
+constexpr int kResSide = 10, kResGroup = 2 * kResSide;
+constexpr int kResF = 6, kResFirst = 7, kResInts = 8;
+enum { kSideDyn = 1, kSideSelf = 2, kSideRank0 = 4, kSideLast = 8 };
+
+struct ResidentSteps {
+    int n[kMaxColours + 1], per[kMaxColours + 1], first[kMaxColours + 1];
+};
+struct ResidentLds {
+    double2 region[kResDoubles / 2];       // the waves' groups, each wave as much as the plan counted for it
+    // LDS offset of its groups, first sorted group, groups | every contact's clamp
+    // flag is 1 << 7 | contacts of its largest << 8, contacts; first sweep position
+    int4 step[kResWaves][kResidentSteps];
+    int step_k0[kResWaves][kResidentSteps];
+    ResidentSteps steps;
+    double pass_max[4][kResWaves * kQuads];  // by pass % 4: max |dl| of each quad
+    int done[kResWaves];                   // passes that each wave has finished
+    int published;  // passes up to this one are reported
+    int known;      // sweeps 1..known are known not to have converged
+    int stop;       // the sweep that converged
+    int failed;
+};
+static_assert(sizeof(ResidentLds) <= 160 * 1024, "LDS of a CU");
+
+// The steps of W waves: colour c has n[c] of per[c] groups each (one each in the
+// sequential tail), and step i of it belongs to wave (first[c] + i) % W.  While
+// there is a wave for every step they follow each other.  Otherwise the colours
+// start 5/8 of the waves apart, as each begins with its largest groups: those of
+// 8 colours in a row then fall to different waves (27,000 contacts of 48 batched
+// scenes need 25,000 doubles in the fullest workgroup when they follow each
+// other, and fit like this).  A wave takes its steps colour by colour.
+AMD_INLINE void resident_steps(const int* cs, int W, ResidentSteps& S) {
+    int total = 0;
+    for (int c = 0; c <= kMaxColours; c++) {
+        const int g = cs[c + 1] - cs[c];
+        S.per[c] = c < kMaxColours ? max(1, min(kQuads, (g + W - 1) / W)) : 1;
+        S.n[c] = (g + S.per[c] - 1) / S.per[c];
+        S.first[c] = total % W;
+        total += S.n[c];
+    }
+    if (total > W)
+        for (int c = 0; c <= kMaxColours; c++) S.first[c] = (int)((long)(c & 7) * 5 * W / 8) % W;
+}
+struct StepWalk {
+    int c = -1, i = 0;
+    // the wave's next step: its first sorted group and its groups; false at the end
+    AMD_INLINE bool next(const ResidentSteps& S, const int* cs, int W, int w, int& q0, int& count) {
+        if (c >= 0) i += W;
+        while (c < 0 || i >= S.n[c]) {
+            if (++c > kMaxColours) return false;
+            i = w - S.first[c];
+            if (i < 0) i += W;
+        }
+        q0 = cs[c] + i * S.per[c];
+        count = min(S.per[c], cs[c + 1] - q0);
+        return true;
+    }
+};
+
+// used[w] = LDS doubles of wave w; plan[0] = those of the fullest workgroup,
+// plan[1] = steps of the busiest wave (counted only as far as the limits)
+__global__ __launch_bounds__(256) void k_resident_plan(const int* cs, const int* group_desc, int W, int* used,
+                                                       int* plan) {
+    __shared__ ResidentSteps S;
+    if (threadIdx.x == 0) resident_steps(cs, W, S);
+    __syncthreads();
+    const int w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= W) return;  // W is a multiple of kResWaves, which divides the wavefront
+    const int4* gdesc = reinterpret_cast<const int4*>(group_desc);
+    int sum = 0, steps = 0, q0, count;
+    StepWalk walk;
+    while (walk.next(S, cs, W, w, q0, count)) {
+        const int contacts = gdesc[q0 + count - 1].y - gdesc[q0].x;
+        sum += count * kResGroup + min(contacts, kResDoubles) * kResContact;
+        steps++;
+        if (sum > kResDoubles || steps > kResidentSteps) break;
+    }
+    used[w] = sum;
+    int total = sum;
+#pragma unroll
+    for (int o = 1; o < kResWaves; o <<= 1) total += __shfl_xor(total, o, 64);
+    if (w % kResWaves == 0) atomicMax(&plan[0], total);
+    atomicMax(&plan[1], steps);
+}
+void launch_resident_plan(hipStream_t s, const int* colour_start, const int* group_desc, int waves, int* used,
+                          int* plan) {
+    hipLaunchKernelGGL(k_resident_plan, dim3((waves + 255) / 256), dim3(256), 0, s, colour_start, group_desc, waves,
+                       used, plan);
+}
+
+AMD_INLINE int lds_int(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+AMD_INLINE void set_lds_int(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+AMD_INLINE void lds_landed() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0)
+// LDS operations of one wave are performed in order: only the compiler is held back
+AMD_INLINE void lds_order() { asm volatile("" ::: "memory"); }
+
+// One contact as a lane of its quad needs it: its three J entries and update
+// coefficients per row, and the contact's scalars.
+typedef double d2v __attribute__((ext_vector_type(2)));
+struct QuadRec {
+    double j[3][3], c[3][3];
+    double b[3], d[3], den[3], y[3], mu, lam[3];
+};
+struct QuadMap {
+    int ofs;        // of this kind of lane in a row
+    unsigned sign;  // A.v lanes: their entries are -jb.v
+};
+// at: the contact in LDS; lam: its lambda and mu for this pass
+AMD_INLINE void read_quad_rec(const double* at, const double* lam, const QuadMap& m, QuadRec& w) {
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const d2v* q = reinterpret_cast<const d2v*>(at + r * kResRow + m.ofs);
+        const d2v q0 = q[0], q1 = q[1], q2 = q[2];
+        w.j[r][0] = q0.x;
+        w.j[r][1] = q0.y;
+        w.j[r][2] = q1.x;
+        w.c[r][0] = q1.y;
+        w.c[r][1] = q2.x;
+        w.c[r][2] = q2.y;
+        const d2v* sc = reinterpret_cast<const d2v*>(at + kResScalars + 4 * r);
+        const d2v s0 = sc[0], s1 = sc[1];
+        w.b[r] = s0.x;
+        w.d[r] = s0.y;
+        w.den[r] = s1.x;
+        w.y[r] = s1.y;
+    }
+    const d2v* l = reinterpret_cast<const d2v*>(lam);
+    const d2v l0 = l[0], l1 = l[1];
+    w.lam[0] = l0.x;
+    w.lam[1] = l0.y;
+    w.lam[2] = l1.x;
+    w.mu = l1.y;
+}
+// The places (one or two, else -1) in a contact in LDS of double d of its record.
+AMD_INLINE void resident_places(int d, int& first, int& second) {
+    first = second = -1;
+    if (d >= kRecLambda) {
+        if (d < kRecLambda + 3) {
+            first = kResLam + d - kRecLambda;
+            second = kResLamOdd + d - kRecLambda;
+        }
+        return;
+    }
+    const int r = d / kRecRow, q = (d % kRecRow) / 4, i = d % 4, row = r * kResRow;
+    if (i == 3) {
+        if (q < 4) {
+            first = kResScalars + 4 * r + q;  // b, D, D + C, its reciprocal
+        } else if (r == 0) {
+            first = kResLam + 3;
+            second = kResLamOdd + 3;
+        }
+        return;
+    }
+    if (q == 0) {
+        first = row + kResV + i;
+        second = row + kResV + 3 + i;
+    } else {
+        first = row + i + (q == 1 ? kResAw : q == 2 ? kResBw : q == 3 ? kResAw + 3 : kResBw + 3);
+    }
+}
+static_assert(kRecB == 3 && kRecD == 7 && kRecDen == 11 && kRecY == 15 && kRecMu == 19, "resident_places");
+constexpr int kQuadSwap1 = 0xB1, kQuadSwap2 = 0x4E;  // quad_perm: lanes 0-1 and 2-3, then the pairs
+// Contact.getJdv (Contact.java:362-378), the same sum in every lane of the
+// quad.  kExact flips the A.v lanes' entries; otherwise their sum is flipped,
+// which differs only in the sign of a zero.
+template <bool kExact>
+AMD_INLINE double quad_jdv(const double (&j)[3], unsigned sign, const double (&dv)[3]) {
+    double s;
+    if (kExact) {
+        s = flip(j[0], sign) * dv[0] + flip(j[1], sign) * dv[1] + flip(j[2], sign) * dv[2];
+    } else {
+        s = flip(j[0] * dv[0] + j[1] * dv[1] + j[2] * dv[2], sign);
+    }
+    const double h = s + dpp_d<kQuadSwap1>(s);
+    return h + dpp_d<kQuadSwap2>(h);
+}
+// f: minv on v lanes, 1 on w lanes, negative on A.v lanes ((-f dl) c is (f dl)
+// (-c) exactly)
+AMD_INLINE void quad_apply(const double (&c)[3], double f, double dl, double (&dv)[3]) {
+    const double s = f * dl;
+#pragma unroll
+    for (int i = 0; i < 3; i++) dv[i] = s * c[i] + dv[i];
+}
+
+// row_contact_fast on a quad: the conditions are those of FastCheck, with the
+// numerators' range as one unsigned distance from its lower end.  There a
+// numerator is normal and nonzero, so the sign of a zero J.dv changes nothing,
+// and min and max are the plain selects (a limit of +0 against -l gives -0 in
+// both).
+struct QuadCheck {
+    unsigned num = 0;    // max of 2 |numerator|'s high word - 2 * 0x30500000
+    unsigned limit = 0;  // max high word of the friction limits (sign included)
+    AMD_INLINE bool ok() const { return num < 2u * (0x4F900000u - 0x30500000u) && limit < 0x7FF00000u; }
+};
+AMD_INLINE void quad_contact_fast(double omega, const QuadRec& c, unsigned sign, double f, double (&dv)[3], double& mx,
+                                  QuadCheck& chk, double (&lam)[3]) {
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const double jd = quad_jdv<false>(c.j[r], sign, dv);
+        const double num = c.d[r] * c.lam[r] - omega * (c.b[r] + jd);
+        unsigned h = hi_word(num);
+        asm("" : "+v"(h));  // else the shift becomes a 64-bit one
+        chk.num = max(chk.num, (h << 1) - 2u * 0x30500000u);
+        const double q0 = num * c.y[r];
+        const double rr = __builtin_fma(-c.den[r], q0, num);
+        double l = __builtin_fma(rr, c.y[r], q0);
+        if (r == 0) {
+            l = __builtin_fmax(l, 0.0);
+        } else {
+            const double limit = c.mu * lam[0];
+            chk.limit = max(chk.limit, hi_word(limit));
+            l = __builtin_fmin(__builtin_fmax(l, -limit), limit);
+        }
+        lam[r] = l;
+        const double diff = l - c.lam[r];
+        quad_apply(c.c[r], f, diff, dv);
+        mx = fmax(mx, fabs(diff));
+    }
+}
+// row_contact on a quad: every form of the update
+AMD_INLINE void quad_contact(double omega, const QuadRec& c, bool clamp, unsigned sign, double f, double (&dv)[3],
+                             double& mx, bool& nan, double (&lam)[3]) {
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const double jd = quad_jdv<true>(c.j[r], sign, dv);
+        const double prev = c.lam[r];
+        const double num = c.d[r] * prev - omega * (c.b[r] + jd);
+        double l = div_row(num, c.den[r], c.y[r]);
+        double lc;
+        if (r == 0) {
+            lc = jmax(0, l);
+        } else {
+            const double limit = c.mu * lam[0];
+            lc = jmin(jmax(l, -limit), limit);
+        }
+        l = clamp ? lc : l;
+        lam[r] = l;
+        const double diff = l - prev;
+        quad_apply(c.c[r], f, diff, dv);
+        mx = fmax(mx, fabs(diff));
+        nan = nan || diff != diff;
+    }
+}
+
+// The pass keeper: one wave of the workgroup.  Workgroups count themselves in
+// at a sweep's arrival words (kPassWords of them, a cache line apart); workgroup
+// 0's keeper alone reads those, and leaves the verdict in one word that the
+// others read: with every keeper polling the arrival words, the adds took
+// longer to get through than a pass.
+AMD_INLINE void keep_passes(const FlowArgs& F, ResidentLds& L, int lane) {
+    const PgsArgs& P = F.P;
+    const int lastp = P.iterations;
+    unsigned long long* verdict = F.pass_done;  // sweeps known not to have converged | converged sweep << 32
+    unsigned long long* arrive = F.pass_done + kPassStride;
+    int a = 1;    // next sweep of this workgroup to report
+    int chk = 0;  // sweeps 1..chk are known not to have converged
+    long spins = 0;
+    while (true) {
+        bool moved = false;
+        if (a <= lastp && __all(lds_int(&L.done[lane & (kResWaves - 1)]) >= a)) {
+            // Math.max over the quads, by the bits (non-negative doubles order as
+            // their bits, a NaN above all)
+            unsigned long long mx = (unsigned long long)__double_as_longlong(
+                __hip_atomic_load(&L.pass_max[a & 3][lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long v = __shfl_xor(mx, o, 64);
+                mx = v > mx ? v : mx;
+            }
+            if (lane == 0) {
+                const bool over = mx && !(__longlong_as_double((long long)mx) < P.tolerance);  // NaN over
+                if (P.check_tolerance)
+                    __hip_atomic_fetch_add(&arrive[((size_t)a * kPassWords + blockIdx.x % kPassWords) * kPassStride],
+                                           (1ull << 32) | (over ? 1ull : 0ull), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                if (mx) atomicMax(&P.iter_max[a - 1], mx);
+                // the ring's entries are written again four passes on, which wait for this
+                set_lds_int(&L.published, a);
+            }
+            a++;
+            moved = true;
+        }
+        if (P.check_tolerance && chk < lastp - 1) {
+            int known = chk, stop = 0;
+            if (blockIdx.x == 0) {
+                if (chk + 1 < a) {
+                    const unsigned long long v =
+                        lane < kPassWords ? ld_cnt64(&arrive[((size_t)(chk + 1) * kPassWords + lane) * kPassStride]) : 0;
+                    int here = (int)(v >> 32), over = (int)(unsigned)v;
+#pragma unroll
+                    for (int o = 1; o < kPassWords; o <<= 1) {
+                        here += __shfl_xor(here, o, 64);
+                        over += __shfl_xor(over, o, 64);
+                    }
+                    if (uniform(here) == (int)gridDim.x) {
+                        if (uniform(over) == 0) stop = chk + 1;
+                        else known = chk + 1;
+                        if (lane == 0)
+                            __hip_atomic_store(verdict, ((unsigned long long)stop << 32) | (unsigned)known,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+            } else if (chk + 1 < a) {
+                const unsigned long long v = ld_cnt64(verdict);
+                known = uniform((int)(unsigned)v);
+                stop = uniform((int)(v >> 32));
+            }
+            if (known != chk) {
+                chk = known;
+                if (lane == 0) set_lds_int(&L.known, chk);
+                moved = true;
+            }
+            if (stop) {
+                if (lane == 0) set_lds_int(&L.stop, stop);
+                return;
+            }
+        } else if (a > lastp) {
+            return;
+        }
+        if (moved) {
+            spins = 0;
+            continue;
+        }
+        if (uniform(lds_int(&L.failed))) return;
+        if (++spins > kFlowSpinLimit ||
+            ((spins & 255) == 0 && uniform(__hip_atomic_load(P.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
+            if (lane == 0) {
+                atomicOr(P.error, 1);
+                set_lds_int(&L.failed, 1);
+            }
+            return;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+template <bool kScenes>
+__global__ __launch_bounds__((kResWaves + 1) * 64) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_pgs_resident(
+    FlowArgs F) {
+    __shared__ ResidentLds L;
+    const PgsArgs& P = F.P;
+    const int* cs = P.colour_start;
+    const int W = gridDim.x * kResWaves;
+    const int wave = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) {
+        resident_steps(cs, W, L.steps);
+        L.published = L.known = L.stop = L.failed = 0;
+        for (int i = 0; i < kResWaves; i++) L.done[i] = 0;
+    }
+    __syncthreads();
+    if (wave == kResWaves) {
+        keep_passes(F, L, lane);
+        return;
+    }
+    const int w = blockIdx.x * kResWaves + wave;
+    const int quad = lane >> 2, lt = lane & 3, side = lt >> 1, wpart = lt & 1;
+    const bool lead = lt == 0;
+    const int first = P.warm_start ? 0 : 1;
+    const int lastp = P.iterations;
+    const double omega = P.omega;
+    const int4* gdesc = reinterpret_cast<const int4*>(P.group_desc);
+    double* reg = reinterpret_cast<double*>(&L.region[0]);
+    int room = 0;  // this wave's part of the region ends there
+    int off = 0;
+    for (int v = 0; v <= wave; v++) {
+        off = room;
+        room += F.resident_used[blockIdx.x * kResWaves + v];
+    }
+    room = min(room, kResDoubles);
+    QuadMap map;
+    map.ofs = lt == 1 ? kResAw : lt == 3 ? kResBw : kResV;
+    map.sign = lt == 0 ? 0x80000000u : 0u;
+
+    // take this wave's groups into LDS
+    int n_steps = 0;
+    {
+        const double* start_dv = (first & 1) ? P.dv : F.dv_alt;
+        const int4* fdesc = reinterpret_cast<const int4*>(F.flow);
+        const int2* gpred = reinterpret_cast<const int2*>(F.pred);
+        const double2* recs = reinterpret_cast<const double2*>(P.rec);
+        // a lane copies 16 bytes of a record, the two halves of the wave two records
+        int to[4];
+        resident_places(2 * (lane & 31), to[0], to[1]);
+        resident_places(2 * (lane & 31) + 1, to[2], to[3]);
+        StepWalk walk;
+        int q0 = 0, count = 0;
+        int4 gd = make_int4(0, 0, 0, 0), fd = gd;
+        int2 pr = make_int2(0, 0);
+        auto fetch = [&]() -> bool {
+            if (!walk.next(L.steps, cs, W, w, q0, count)) return false;
+            const int q = q0 + (quad < count ? quad : 0);
+            gd = gdesc[q];
+            fd = fdesc[q];
+            pr = gpred[q];
+            return true;
+        };
+        bool more = fetch();
+        while (more) {
+            const int4 g = gd, fl = fd;
+            const int2 pd = pr;
+            const int q_first = q0, n_groups = count;
+            more = fetch();
+            const bool has = quad < n_groups;
+            const int k0 = uniform(g.x), contacts = __builtin_amdgcn_readlane(g.y, 4 * (n_groups - 1)) - k0;
+            const int first_contact = off + n_groups * kResGroup;
+            if (n_steps >= kResidentSteps || contacts > kResDoubles ||
+                first_contact + contacts * kResContact > room) {  // the plan allows none of these
+                if (lane == 0) {
+                    atomicOr(P.error, 1);
+                    set_lds_int(&L.failed, 1);
+                }
+                return;
+            }
+            const int e = side ? g.w : g.z, rank = side ? fl.z : fl.x, deg = side ? fl.w : fl.y;
+            double v[3], minv = 0.0;
+            int extra = 0;
+            if (has) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) v[i] = ld_coherent(&start_dv[e * 6 + 3 * wpart + i]);
+                minv = P.minv[e];
+                if (kScenes) {
+                    extra = P.g_scene[q_first + quad];
+                    if (side) extra = (int)P.scene_groups[extra];
+                }
+            }
+            bool plain = true;
+            constexpr int kAhead = 4;  // pairs of records in flight
+            for (int i0 = 0; i0 < contacts; i0 += 2 * kAhead) {
+                double2 d[kAhead];
+#pragma unroll
+                for (int u = 0; u < kAhead; u++) {
+                    const int i = min(i0 + 2 * u + (lane >> 5), contacts - 1);
+                    d[u] = recs[(size_t)(k0 + i) * kRec2 + (lane & 31)];
+                }
+#pragma unroll
+                for (int u = 0; u < kAhead; u++) {
+                    const int i = min(i0 + 2 * u + (lane >> 5), contacts - 1);
+                    double* at = reg + first_contact + i * kResContact;
+                    if (to[0] >= 0) at[to[0]] = d[u].x;
+                    if (to[1] >= 0) at[to[1]] = d[u].x;
+                    if (to[2] >= 0) at[to[2]] = d[u].y;
+                    if (to[3] >= 0) at[to[3]] = d[u].y;
+                    if ((lane & 31) == kRecClamp / 2) plain = plain && (kRecClamp % 2 ? d[u].y : d[u].x) == 1.0;
+                }
+            }
+            int nmax = has ? g.y - g.x : 0;
+#pragma unroll
+            for (int o = 4; o < 64; o <<= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
+            plain = __all(plain);
+            if (lane == 0) {
+                L.step[wave][n_steps] =
+                    make_int4(off, q_first, n_groups | (plain ? 0x80 : 0) | (nmax << 8), contacts);
+                L.step_k0[wave][n_steps] = k0;
+            }
+            if (has) {
+                double* blk = reg + off + quad * kResGroup + side * kResSide;
+#pragma unroll
+                for (int i = 0; i < 3; i++) blk[3 * wpart + i] = v[i];
+                if (wpart == 0) {
+                    const int flags = (deg ? kSideDyn : 0) | (deg == 1 ? kSideSelf : 0) | (rank == 0 ? kSideRank0 : 0) |
+                                      (rank == deg - 1 ? kSideLast : 0);
+                    auto pack = [](int lo, int hi) {
+                        return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+                    };
+                    blk[kResF] = minv;
+                    blk[kResFirst] = pack(first_contact + (g.x - k0) * kResContact, g.y - g.x);
+                    blk[kResInts] = pack(e, side ? pd.y : pd.x);
+                    blk[kResInts + 1] = pack(flags, extra);
+                }
+            }
+            off = first_contact + contacts * kResContact;
+            n_steps++;
+        }
+    }
+
+    // bookkeeping of the next step
+    struct Next {
+        int q0, count, nmax;
+        bool plain;
+        double* blk;
+        double f;
+        long long where, who, what;  // first contact and contacts; body and incidence; flags and extra
+    } nx;
+    auto next_step = [&](int s) {
+        const int4 T = L.step[wave][s];
+        const int goff = uniform(T.x);
+        nx.q0 = uniform(T.y);
+        nx.count = uniform(T.z) & 0x7f;
+        nx.plain = uniform(T.z) & 0x80;
+        nx.nmax = uniform(T.z) >> 8;
+        nx.blk = reg + goff + (quad < nx.count ? quad : 0) * kResGroup + side * kResSide;
+        nx.f = nx.blk[kResF];
+        nx.where = __double_as_longlong(nx.blk[kResFirst]);
+        nx.who = __double_as_longlong(nx.blk[kResInts]);
+        nx.what = __double_as_longlong(nx.blk[kResInts + 1]);
+    };
+    if (n_steps > 0) next_step(0);
+    for (int p = first; p <= lastp; p++) {
+        // pass gates: sweep p-2 must be known not converged (p-1 for the last
+        // sweep), and the workgroup's pass ring must have room
+        if (p >= 2) {
+            const int need = !P.check_tolerance ? 0 : p == lastp ? p - 1 : p - 2;
+            bool leave = false;
+            for (long spins = 0;; spins++) {
+                const int stop = uniform(lds_int(&L.stop)), known = uniform(lds_int(&L.known)),
+                          pub = uniform(lds_int(&L.published));
+                // every wave runs the sweep after the converged one and leaves then
+                leave = (stop && stop <= need) || uniform(lds_int(&L.failed));
+                if (leave || (known >= need && pub >= p - 3)) break;
+                if (spins > 16 * kFlowSpinLimit) {  // the keeper gives up long before
+                    if (lane == 0) atomicOr(P.error, 1);
+                    leave = true;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (leave) break;
+        }
+        const bool last = p == lastp;
+        const int lam_r = (p >= 1 && ((p - 1) & 1)) ? kResLamOdd : kResLam, lam_w = (p & 1) ? kResLamOdd : kResLam;
+        double* cur = (p & 1) ? F.dv_alt : P.dv;
+        const double* prv = (p & 1) ? P.dv : F.dv_alt;
+        double mx = 0.0;
+        bool nan = false;
+        for (int s = 0; s < n_steps; s++) {
+            // this step's bookkeeping was read during the one before
+            const int q0 = nx.q0, nmax = nx.nmax;
+            const bool plain = nx.plain;
+            // A quad without a group runs the first one's again and keeps the
+            // result to itself: a wave with most of its lanes switched off takes
+            // longer over a contact, not less (1000 to 1600 cycles, against 670).
+            const bool owner = quad < nx.count;
+            const int group = q0 + (owner ? quad : 0);
+            bool skipped = false;
+            double* blk = nx.blk;
+            const int e = (int)nx.who, pred = (int)(nx.who >> 32), flags = (int)nx.what, extra = (int)(nx.what >> 32);
+            const double f = wpart ? 1.0 : lead ? -nx.f : nx.f;
+            double* rec = reg + (int)nx.where;
+            int n = (int)(nx.where >> 32);
+            auto load = [&](int t, QuadRec& rc) {
+                const double* at = rec + min(t, max(n - 1, 0)) * kResContact;
+                read_quad_rec(at, at + lam_r, map, rc);
+            };
+            QuadRec ra, rb;
+            // inputs: LDS for pinned bodies and bodies of this group alone, the
+            // launch buffer for a body's first update, else the slot of the
+            // body's previous update
+            double dv[3] = {blk[3 * wpart], blk[3 * wpart + 1], blk[3 * wpart + 2]};
+            double* src = nullptr;
+            const bool own = !(flags & kSideDyn) || (flags & kSideSelf);
+            if (!own) {
+                if (p == first && (flags & kSideRank0)) {
+#pragma unroll
+                    for (int i = 0; i < 3; i++) dv[i] = ld_coherent(&prv[e * 6 + 3 * wpart + i]);
+                } else {
+                    src = slot_at(F, (flags & kSideRank0) ? ((p - 1) & 1) : (p & 1), pred) + 4 * wpart;
+                }
+            }
+            // the first poll is on its way while the first record is read
+            double v0 = 0.0, v1 = 0.0, v2 = 0.0;
+            if (src) {
+                v0 = ld_coherent(src);
+                v1 = ld_coherent(src + 1);
+                v2 = ld_coherent(src + 2);
+            }
+            load(0, ra);
+            {
+                bool got = src == nullptr;
+                long spins = 0;
+                auto spin = [&]() -> bool {  // false: give up (error flag set)
+                    __builtin_amdgcn_s_sleep(1);
+                    if (!got) {
+                        v0 = ld_coherent(src);
+                        v1 = ld_coherent(src + 1);
+                        v2 = ld_coherent(src + 2);
+                    }
+                    if (++spins > kFlowSpinLimit ||
+                        ((spins & 255) == 0 &&
+                         uniform(__hip_atomic_load(P.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
+                        if (lane == 0) {
+                            atomicOr(P.error, 1);
+                            set_lds_int(&L.failed, 1);
+                        }
+                        return false;
+                    }
+                    return true;
+                };
+                auto poll = [&]() {
+                    if (!got) {
+                        auto filled = [](double v) { return (unsigned long long)__double_as_longlong(v) != kSlotEmpty; };
+                        if (filled(v0) && filled(v1) && filled(v2)) {
+                            dv[0] = v0;
+                            dv[1] = v1;
+                            dv[2] = v2;
+                            got = true;
+                        }
+                    }
+                };
+                const int t1 = p - 2, t2 = last ? p - 1 : 0;
+                if (!(kScenes && p >= 1 && P.check_tolerance && (t1 >= 1 || t2 >= 1))) {
+                    while (true) {
+                        poll();
+                        if (__all(got)) break;
+                        if (!spin()) return;
+                    }
+                } else {
+                    // Per-scene exits, as in k_pgs_flow: a group whose scene was
+                    // under the tolerance at sweep p-2 or p-3 (p-1 before the
+                    // last) skips this pass and every later one.
+                    bool resolved = !lead, skip = false;
+                    unsigned want = 0;
+                    if (lead) want = (unsigned)(__double_as_longlong(blk[kResSide + kResInts + 1]) >> 32);
+                    const unsigned long long* cnt = &P.scene_done[(size_t)(lead ? extra : 0) * (P.iterations + 1)];
+                    const int ta = t1 >= 1 ? t1 : t2, tb = t1 >= 2 ? t1 - 1 : ta, tc = t2 >= 1 ? t2 : ta;
+                    while (true) {
+                        poll();
+                        if (!resolved) {
+                            const unsigned long long wa = ld_cnt64(&cnt[ta]), wb = ld_cnt64(&cnt[tb]),
+                                                     wc = ld_cnt64(&cnt[tc]);
+                            if ((unsigned)(wa >> 32) == want && (unsigned)(wb >> 32) == want &&
+                                (unsigned)(wc >> 32) == want) {
+                                skip = (unsigned)wa == 0u || (unsigned)wb == 0u || (unsigned)wc == 0u;
+                                resolved = true;
+                            }
+                        }
+                        const int flagged = (resolved ? 1 : 0) | (skip ? 2 : 0);
+                        const int of_quad = __builtin_amdgcn_mov_dpp(flagged, kQuadLane0, 0xF, 0xF, true);
+                        if (__all((of_quad & 1) && ((of_quad & 2) || got))) {
+                            if (of_quad & 2) {
+                                skipped = true;
+                                n = 0;
+                                src = nullptr;
+                            }
+                            break;
+                        }
+                        if (!spin()) return;
+                    }
+                }
+            }
+            // the inputs were the last loads: this wave's stores of the pass before have landed
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+            double smx = 0.0;
+            bool snan = false;
+            double lam[3];
+            // every lane of the quad writes the same values to the same place
+            auto keep_lambda = [&](int t) {
+                double* to = rec + t * kResContact + lam_w;
+                to[0] = lam[0];
+                to[1] = lam[1];
+                to[2] = lam[2];
+            };
+            // Contact.updateContactState (Contact.java:385-398)
+            auto state = [&](int t, const QuadRec& c) {
+                const double w1 = c.b[1] + quad_jdv<true>(c.j[1], map.sign, dv);
+                const double w2 = c.b[2] + quad_jdv<true>(c.j[2], map.sign, dv);
+                if (lead && owner) {
+                    int st;
+                    if (fabs(lam[0]) <= 1e-14) st = AM_STATE_BROKEN;
+                    else if (fabs(w1) > P.sliding) st = AM_STATE_ONEDGE;
+                    else if (fabs(w2) > P.sliding) st = AM_STATE_ONEDGE;
+                    else st = AM_STATE_CLEAR;
+                    P.sstate[gdesc[group].x + t] = st;
+                }
+            };
+            // sweeps but the last (whose contacts get their states) try the
+            // fast update; the general one runs again from the step's start
+            lds_landed();
+            bool general = p == 0 || last || !plain;
+            if (!general) {
+                const double dv0[3] = {dv[0], dv[1], dv[2]};
+                QuadCheck chk;
+                // A record is read while the one before it runs; the wait for it
+                // stands before the reads of the one after it (their number is
+                // more than the counter of LDS operations tells apart)
+                auto one = [&](int t, const QuadRec& now, QuadRec& then) {
+                    if (t < n) {
+                        load(t + 1, then);
+                        quad_contact_fast(omega, now, map.sign, f, dv, smx, chk, lam);
+                    }
+                    lds_landed();
+                    if (t < n) keep_lambda(t);
+                };
+                for (int t = 0; t < nmax; t += 2) {
+                    one(t, ra, rb);
+                    if (t + 1 >= nmax) break;
+                    one(t + 1, rb, ra);
+                }
+                if (__builtin_expect(!__all(chk.ok()), 0)) {
+                    dv[0] = dv0[0];
+                    dv[1] = dv0[1];
+                    dv[2] = dv0[2];
+                    smx = 0.0;
+                    general = true;
+                }
+            }
+            if (general) {
+                for (int t = 0; t < nmax; t++) {
+                    load(t, ra);
+                    if (t >= n) continue;
+                    if (p == 0) {
+                        // confidentWarmStart (PGS.java:250-256)
+#pragma unroll
+                        for (int r = 0; r < 3; r++) quad_apply(ra.c[r], f, ra.lam[r], dv);
+                        continue;
+                    }
+                    const bool clamp = P.rec[(size_t)(gdesc[group].x + t) * kRecDoubles + kRecClamp] != 0.0;
+                    quad_contact(omega, ra, clamp, map.sign, f, dv, smx, snan, lam);
+                    keep_lambda(t);
+                    if (last) state(t, ra);
+                }
+            }
+            // publish: the next update's slot, or LDS for a body of this group
+            // alone; the body's last update of a pass also to the pass's buffer
+            if (owner && !skipped && (flags & kSideDyn)) {
+                if (flags & kSideSelf) {
+#pragma unroll
+                    for (int i = 0; i < 3; i++) blk[3 * wpart + i] = dv[i];
+                } else {
+                    double* dst = slot_at(F, p & 1, 2 * group + side) + 4 * wpart;
+#pragma unroll
+                    for (int i = 0; i < 3; i++) st_coherent(dst + i, dv[i]);
+                }
+                if (flags & kSideLast)
+#pragma unroll
+                    for (int i = 0; i < 3; i++) st_coherent(&cur[e * 6 + 3 * wpart + i], dv[i]);
+            }
+            // the slot that was read is empty again only now, behind the values
+            // that the next update waits for
+            if (src && owner)
+#pragma unroll
+                for (int i = 0; i < 3; i++) st_coherent(src + i, __longlong_as_double((long long)kSlotEmpty));
+            if (n_steps > 1) next_step(s + 1 < n_steps ? s + 1 : 0);
+            mx = fmax(mx, smx);
+            nan = nan || snan;
+            if (kScenes && p >= 1 && P.per_scene && owner && lead) {
+                const size_t sc = (size_t)extra;
+                if (!skipped && !(smx <= 0))
+                    atomicMax(&P.scene_max[sc * P.iterations + p - 1],
+                              (unsigned long long)__double_as_longlong(
+                                  snan ? __longlong_as_double(0x7ff8000000000000ll) : smx));
+                // over the tolerance (NaN included), as the scene's max would be
+                const bool over = !skipped && !(smx <= 0) && (snan || !(smx < P.tolerance));
+                __hip_atomic_fetch_add(&P.scene_done[sc * (P.iterations + 1) + p], (1ull << 32) | (over ? 1ull : 0ull),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if (p >= 1) {
+            if (nan) mx = __longlong_as_double(0x7ff8000000000000ll);
+            L.pass_max[p & 3][wave * kQuads + quad] = mx;  // the same from every lane of the quad
+            lds_order();
+            set_lds_int(&L.done[wave], p);
+        }
+    }
+    // lambdas of the last even and the last odd pass; k_unpack takes the one
+    // that the sweeps used say
+    for (int s = 0; s < n_steps; s++) {
+        const int4 T = L.step[wave][s];
+        const int goff = uniform(T.x), count = uniform(T.z) & 0x7f, contacts = uniform(T.w);
+        const int k0 = uniform(L.step_k0[wave][s]);
+        const double* at = reg + goff + count * kResGroup;
+        for (int i = lane; i < 3 * contacts; i += 64) {
+            const int t = i / 3, r = i - 3 * t;
+            P.rec[(size_t)(k0 + t) * kRecDoubles + kRecLambda + r] = at[t * kResContact + kResLam + r];
+            if (lastp >= 1) F.lam_alt[4 * (size_t)(k0 + t) + r] = at[t * kResContact + kResLamOdd + r];
+        }
+    }
+}
+
+int pgs_resident_max_blocks(bool* ok) {
+    int dev = 0, n_cu = 0, a = 0, b = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_pgs_resident<false>, (kResWaves + 1) * 64, 0);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_pgs_resident<true>, (kResWaves + 1) * 64, 0);
+    *ok = std::min(a, b) > 0;
+    return n_cu * std::min(a, b);
+}
+
 // Sweeps used (the first converged sweep, else all), then the buffers of the
 // last pass become the results.
 __global__ void k_flow_finish(PgsArgs P) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
     int used = P.iterations;
     if (P.check_tolerance)
-        for (int t = 1; t <= P.iterations; t++)
+        for (int t = 1 + (int)threadIdx.x; t <= P.iterations; t += 64)
             if (__longlong_as_double((long long)P.iter_max[t - 1]) < P.tolerance) {
                 used = t;
                 break;
             }
-    *P.iters_used = used;
+    for (int o = 32; o > 0; o >>= 1) used = min(used, __shfl_xor(used, o, 64));
+    if (threadIdx.x == 0) *P.iters_used = used;
 }
 __global__ void k_flow_select_dv(double* dv, const double* dv_alt, int n, const int* iters_used,
                                  const int* scene_used, const am_body_desc* desc) {
@@ -1585,14 +2410,16 @@ int pgs_flow_max_blocks(bool* ok) {
     return n_cu * (per_cu > 0 ? per_cu : 1);
 }
 
-hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, bool plain, int n_dv, const BodiesView& B) {
+hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain, int n_dv,
+                           const BodiesView& B) {
+    const bool resident = block != 64;
+    void (*kernel)(FlowArgs) = resident ? (F.P.per_scene ? k_pgs_resident<true> : k_pgs_resident<false>)
+                                        : (F.P.per_scene ? k_pgs_flow<true> : k_pgs_flow<false>);
     if (plain) {
-        if (F.P.per_scene) hipLaunchKernelGGL(k_pgs_flow<true>, dim3(grid), dim3(64), 0, s, F);
-        else hipLaunchKernelGGL(k_pgs_flow<false>, dim3(grid), dim3(64), 0, s, F);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, s, F);
     } else {
-        const void* kernel = F.P.per_scene ? (const void*)k_pgs_flow<true> : (const void*)k_pgs_flow<false>;
         void* args[] = {(void*)&F};
-        hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(64), args, 0, s);
+        hipError_t e = hipLaunchCooperativeKernel((const void*)kernel, dim3(grid), dim3(block), args, 0, s);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k_flow_finish, dim3(1), dim3(64), 0, s, F.P);

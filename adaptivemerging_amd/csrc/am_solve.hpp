@@ -75,6 +75,15 @@ struct PgsArgs {
 constexpr int kSlotDoubles = 8;
 constexpr unsigned long long kSlotEmpty = 0xFFF5A5A5A5A5A5A5ull;  // a signalling NaN: no arithmetic result
 constexpr int kPassWords = 8;  // the pass words spread the waves' adds over this many addresses
+constexpr int kPassStride = 16;  // resident kernel: arrival words are a cache line (128 B) apart
+
+// The resident kernel: LDS doubles a workgroup can hold and steps a wave can;
+// a workgroup is 4 sweeping waves and the pass keeper.
+constexpr int kResidentDoubles = 4 * 4912;
+constexpr int kResidentSteps = 40;
+constexpr int kResidentThreads = 320;
+constexpr int kResidentMaxWaves = 1024;
+constexpr int kResidentMaxSweeps = 65536;
 
 struct FlowArgs {
     PgsArgs P;
@@ -87,7 +96,10 @@ struct FlowArgs {
     // per pass, kPassWords words (zeroed before launch): waves that have
     // finished it in the high 32 bits, those whose max |dl| was not under the
     // tolerance in the low; wave w adds to word w % kPassWords
+    // (the resident kernel: the verdict word, then kPassWords arrival words per
+    // sweep, kPassStride apart, counting workgroups)
     unsigned long long* pass_done;
+    const int* resident_used;  // resident kernel: LDS doubles of each wave (launch_resident_plan)
     unsigned n_waves;
 };
 
@@ -116,7 +128,14 @@ void launch_unpack(hipStream_t s, const SetupArgs& S, int cap);
 int pgs_max_blocks(int block, bool* ok);
 hipError_t launch_pgs(hipStream_t s, const PgsArgs& P, int grid, int block, bool plain);
 int pgs_flow_max_blocks(bool* ok);
-hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, bool plain, int n_dv, const BodiesView& B);
+// block 64: k_pgs_flow; kResidentThreads: the resident kernel
+hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain, int n_dv,
+                           const BodiesView& B);
+int pgs_resident_max_blocks(bool* ok);
+// what `waves` resident waves would hold: used[] LDS doubles of each, plan[0]
+// those of the fullest workgroup, plan[1] steps of the busiest wave
+void launch_resident_plan(hipStream_t s, const int* colour_start, const int* group_desc, int waves, int* used,
+                          int* plan);
 void launch_flow_ranks(hipStream_t s, int n_ent, int n_groups, const int* bflags, const int* inc_start,
                        const int* inc_count, const int* inc_items, const int* spos, const int* group_desc,
                        int* flow, int* pred);

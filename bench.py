@@ -570,7 +570,8 @@ def main(argv=None) -> int:
     achieved = res_p["_pgs_bytes"] / (res_p["_pgs_ms"] * 1e-3) / 1e9 if res_p["_pgs_ms"] > 0 else 0.0
     roofline = {
         "bound": "hbm",
-        "kernel": ("am::k_pgs_flow<false> (persistent dataflow PGS)" if args.pgs_schedule == "dataflow"
+        "kernel": ("am::k_pgs_resident<false> (dataflow PGS resident in LDS)" if args.pgs_schedule == "dataflow" and block_used > 64
+                   else "am::k_pgs_flow<false> (persistent dataflow PGS)" if args.pgs_schedule == "dataflow"
                    else "am::k_pgs<false> (persistent coloured PGS)"),
         "achieved": achieved,
         "peak": HBM_PEAK_GBS,

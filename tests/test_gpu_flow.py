@@ -111,3 +111,37 @@ def test_flow_unclamped_contacts_take_the_general_update(gpu_lib, schedule):
         scene.bodies[i]["flags"] = int(scene.bodies[i]["flags"]) | AM_BODY_MAGNET_ACTIVE
     for iterations in (1, 2, 9):
         _solve_pair(scene, 7, iterations=iterations, tolerance=0.0, gravity_amount=9.81, pgs_schedule=schedule)
+
+
+@pytest.mark.parametrize("spheres,boxes", [(1, 0), (5, 1), (1024, 0), (1025, 0), (0, 1030), (16384, 0), (16385, 3),
+                                           (40000, 0), (56000, 0)])
+def test_resident_steps_at_their_edges(gpu_lib, spheres, boxes):
+    """Bodies of one contact (spheres) and of four (boxes), each alone on a
+    plane: one colour, whose groups go to the resident kernel's waves (1024 of
+    them, steps of at most 16 groups).  Below and past a group a wave, a full
+    step each, a second step for some waves, and more than the LDS of the card
+    holds, where k_pgs_flow runs instead.  Against the oracle, bit for bit."""
+    from adaptivemerging_amd.scene import Scene
+
+    s = Scene()
+    s.add_plane([0, 0, 0], [0, 1, 0], friction=0.6)
+    for i in range(spheres + boxes):
+        x, z = (i % 200) * 0.5, (i // 200) * 0.5
+        v = [0.3, -0.5, 0.1 * (i % 7)]
+        if i < spheres:
+            s.add_sphere(0.1, [x, 0.099, z], v=v, density=300.0 + i % 11)
+        else:
+            s.add_box([0.2, 0.1, 0.2], [x, 0.049, z], v=v, density=300.0 + i % 11)
+    for iterations in (1, 4):
+        ctx, orc = twin(s, iterations=iterations, tolerance=0.0, gravity_amount=9.81)
+        ctx.apply_gravity(); orc.apply_gravity()
+        n = ctx.detect(0.01); orc.detect()
+        ctx.solve(0.01)
+        shape = ctx.launch_shape()
+        print("contacts", n, "shape", shape, flush=True)
+        assert n == spheres + 4 * boxes
+        assert shape[1] == (64 if spheres == 56000 else 320)
+        orc.solve(ctx.solve_order(), 0.01)
+        assert_contacts_equal(ctx.contacts(), orc.contacts())
+        assert_bits_equal("deltaV", ctx.pull_deltav(), orc.pull_deltav())
+        ctx.close()
