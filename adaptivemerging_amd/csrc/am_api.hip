@@ -135,8 +135,7 @@ int ensure_contact_capacity(am_ctx* c, int want, int keep) {
     AM_HIP(c, c->g_start.ensure(cap + 1));
     AM_HIP(c, c->g_a.ensure(cap));
     AM_HIP(c, c->g_b.ensure(cap));
-    AM_HIP(c, c->g_colour_a.ensure(cap));
-    AM_HIP(c, c->g_colour_b.ensure(cap));
+    AM_HIP(c, c->g_colour.ensure(cap));
     AM_HIP(c, c->g_keys.ensure(cap));
     AM_HIP(c, c->g_keys_sorted.ensure(cap));
     AM_HIP(c, c->g_spos.ensure(cap));
@@ -425,61 +424,86 @@ int build_layout(am_ctx* c) {
     if (ng >= (1 << 28)) return fail(c, AM_ERR_INVALID, "more than 2^28 contact groups");
     hipStream_t s = c->stream;
     int* sc = c->d_scalars.p;
-    fill_int(s, c->inc_count.p, c->n_ent + 1, 0);
-    fill_int(s, c->inc_cursor.p, c->n_ent + 1, 0);
-    if (ng > 0) {
-        launch_incidence(s, false, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_count.p, nullptr, nullptr, nullptr);
-        exclusive_scan(s, c->inc_count.p, c->inc_start.p, c->n_ent + 1, sc + 3, c->d_scan_temp.p);
-        AM_HIP(c, c->inc_items.ensure(2 * (size_t)ng + 1));
-        launch_incidence(s, true, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_count.p, c->inc_start.p,
-                         c->inc_cursor.p, c->inc_items.p);
-        fill_int(s, c->g_colour_a.p, ng, -1);
-        AM_HIP(c, c->g_blocker.ensure(std::max(ng, 1)));
-        fill_int(s, c->g_blocker.p, ng, -1);
-        int* cin = c->g_colour_a.p;
-        int* cout = c->g_colour_b.p;
-        // Rounds run in batches between reads of a flag that some group is
-        // still uncoloured: a round after the last one only copies the
-        // colours, so the colouring does not depend on the batch size.
-        constexpr int kRoundsPerCheck = 8;
-        for (int round = 0; round < 4096; round += kRoundsPerCheck) {
-            for (int k = 0; k < kRoundsPerCheck; k++) {
-                fill_int(s, sc + 5, 1, 0);
-                launch_colour_round(s, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_start.p, c->inc_count.p,
-                                    c->inc_items.p, cin, cout, sc + 5, c->layout_layer, c->g_blocker.p);
-                std::swap(cin, cout);
-            }
-            int r = read_scalars(c, 5, 1);
-            if (r) return r;
-            if (c->h_scalars[5] == 0) break;
-        }
-        launch_colour_keys(s, ng, cin, c->g_start.p, c->g_keys.p);
-        sort_u64(s, c->g_keys.p, c->g_keys_sorted.p, ng, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
-    }
     AM_HIP(c, c->s_colour_start.ensure(kMaxColours + 4));
     AM_HIP(c, c->s_group_desc.ensure((size_t)std::max(ng, 1) * 4));
-    launch_colour_layout(s, ng, c->g_keys_sorted.p, c->g_start.p, c->g_a.p, c->g_b.p, c->s_colour_start.p,
-                         c->g_sizes.p, c->g_pos_start.p, c->s_order.p, c->s_group_desc.p, c->s_pos_a.p,
-                         c->g_spos.p, sc + 9, c->d_scan_temp.p);
     AM_HIP(c, c->s_flow.ensure((size_t)std::max(ng, 1) * 4));
     AM_HIP(c, c->s_pred.ensure((size_t)std::max(ng, 1) * 2));
-    launch_flow_ranks(s, c->n_ent, ng, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p, c->g_spos.p,
-                      c->s_group_desc.p, c->s_flow.p, c->s_pred.p);
+    AM_HIP(c, c->s_used.ensure(kResidentMaxWaves));
     if (c->resident_max_grid == 0) {
         bool ok = false;
         c->resident_max_grid = pgs_resident_max_blocks(&ok);
         if (!ok) c->resident_max_grid = -1;
     }
-    AM_HIP(c, c->s_used.ensure(kResidentMaxWaves));
     // a group a wave as far as there are waves
-    const int rgrid = std::min((std::min(ng, kResidentMaxWaves) + 3) / 4, c->resident_max_grid);
-    if (rgrid > 0)
-        launch_resident_plan(s, c->s_colour_start.p, c->s_group_desc.p, 4 * rgrid, c->s_used.p,
-                             c->s_colour_start.p + kMaxColours + 2);
-    AM_HIP(c, hipGetLastError());
+    const int rgrid = std::max(0, std::min((std::min(ng, kResidentMaxWaves) + 3) / 4, c->resident_max_grid));
+    const bool small = ng > 0 && ng <= kSmallLayout;
+    if (small) {
+        SmallLayoutArgs A;
+        A.n_groups = ng;
+        A.n_ent = c->n_ent;
+        A.waves = 4 * rgrid;
+        A.ga = c->g_a.p;
+        A.gb = c->g_b.p;
+        A.bflags = c->d_flags.p;
+        A.group_start = c->g_start.p;
+        A.layer = c->layout_layer;
+        A.inc_count = c->inc_count.p;
+        A.inc_start = c->inc_start.p;
+        A.colour_start = c->s_colour_start.p;
+        A.pos_start = c->g_pos_start.p;
+        A.order = c->s_order.p;
+        A.pos_a = c->s_pos_a.p;
+        A.group_desc = c->s_group_desc.p;
+        A.flow = c->s_flow.p;
+        A.pred = c->s_pred.p;
+        A.used = c->s_used.p;
+        launch_layout_small(s, A);
+    } else if (ng > 0) {
+        fill_int(s, c->inc_count.p, c->n_ent + 1, 0);
+        fill_int(s, c->inc_cursor.p, c->n_ent + 1, 0);
+        launch_incidence(s, false, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_count.p, nullptr, nullptr, nullptr);
+        exclusive_scan(s, c->inc_count.p, c->inc_start.p, c->n_ent + 1, sc + 3, c->d_scan_temp.p);
+        AM_HIP(c, c->inc_items.ensure(2 * (size_t)ng + 1));
+        launch_incidence(s, true, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_count.p, c->inc_start.p,
+                         c->inc_cursor.p, c->inc_items.p);
+        fill_int(s, c->g_colour.p, ng, -1);
+        if (c->layout_layer) {
+            AM_HIP(c, c->g_blocker.ensure(ng));
+            fill_int(s, c->g_blocker.p, ng, -1);
+        } else {
+            AM_HIP(c, c->g_rank.ensure(2 * (size_t)ng));
+            AM_HIP(c, c->g_taken.ensure(c->n_ent));
+            fill_u64(s, c->g_taken.p, 2 * (size_t)c->n_ent, 0);
+        }
+    }
     int cs[kMaxColours + 4];
-    AM_HIP(c, hipMemcpyAsync(cs, c->s_colour_start.p, sizeof cs, hipMemcpyDeviceToHost, s));
-    AM_HIP(c, hipStreamSynchronize(s));
+    // again if groups were left without a colour (launch_colour)
+    for (int round = 0;; round++) {
+        if (!small) {
+            if (ng > 0) {
+                fill_int(s, sc + 5, 1, 0);
+                launch_colour(s, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_start.p, c->inc_count.p,
+                              c->inc_items.p, c->g_colour.p, c->g_taken.p, c->g_rank.p, sc + 5, c->layout_layer,
+                              c->g_blocker.p, round > 0);
+                launch_colour_keys(s, ng, c->g_colour.p, c->g_start.p, c->g_keys.p);
+                sort_u64(s, c->g_keys.p, c->g_keys_sorted.p, ng, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
+            }
+            launch_colour_layout(s, ng, c->g_keys_sorted.p, c->g_start.p, c->g_a.p, c->g_b.p, c->s_colour_start.p,
+                                 c->g_sizes.p, c->g_pos_start.p, c->s_order.p, c->s_group_desc.p, c->s_pos_a.p,
+                                 c->g_spos.p, sc + 9, c->d_scan_temp.p);
+            launch_flow_ranks(s, ng, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p,
+                              c->g_spos.p, c->s_group_desc.p, c->s_flow.p, c->s_pred.p);
+            if (rgrid > 0)
+                launch_resident_plan(s, c->s_colour_start.p, c->s_group_desc.p, 4 * rgrid, c->s_used.p,
+                                     c->s_colour_start.p + kMaxColours + 2);
+        }
+        AM_HIP(c, hipGetLastError());
+        AM_HIP(c, hipMemcpyAsync(cs, c->s_colour_start.p, sizeof cs, hipMemcpyDeviceToHost, s));
+        int r = read_scalars(c, 5, 1);
+        if (r) return r;
+        if (small || ng == 0 || c->h_scalars[5] == 0) break;
+        if (round == 1000) return fail(c, AM_ERR_HIP, "colouring stopped making progress");
+    }
     const bool fits = rgrid > 0 && cs[kMaxColours + 2] <= kResidentDoubles && cs[kMaxColours + 3] <= kResidentSteps;
     c->resident_grid = fits ? rgrid : 0;
     int ncol = 0, maxc = 0;

@@ -164,7 +164,7 @@ struct am_ctx {
     DBuf<double> o_pB1, o_lam, o_viol, o_prev;
 
     // groups, colouring, solve layout
-    DBuf<int> g_flags, g_scanned, g_start, g_a, g_b, g_colour_a, g_colour_b, inc_count, inc_start, inc_cursor, inc_items,
+    DBuf<int> g_flags, g_scanned, g_start, g_a, g_b, g_colour, inc_count, inc_start, inc_cursor, inc_items,
         g_sizes, g_pos_start, s_order, s_colour_start;
     DBuf<uint64_t> g_keys, g_keys_sorted;
     DBuf<double> s_rec, s_lam;
@@ -263,7 +263,8 @@ struct am_ctx {
     int last_merged = 0, last_unmerged = 0;
     // breadth-first layers of the single sweep's groups (getOrganizedContacts)
     DBuf<int> g_layer, bfs_mark;
-    DBuf<int> g_blocker;  // colouring: the neighbour a waiting group waits for
+    DBuf<int> g_blocker, g_rank;  // colouring: the neighbour a layered group waits for; priority ranks
+    DBuf<am::TakenColours> g_taken;
     const int* layout_layer = nullptr;  // set while the single sweep builds its layout
     DBuf<int> sweep_order;              // order of the last single sweep inside collections
     int sweep_order_n = -1;             // -1: none since the last solve or detection

@@ -121,85 +121,211 @@ AMD_INLINE bool higher(uint32_t h, uint32_t g) {
     return ph > pg || (ph == pg && h > g);
 }
 
-// One Jones-Plassmann round: an uncoloured group whose priority is the highest
-// among its uncoloured neighbours takes the smallest colour unused by its
-// coloured neighbours (colours read from the previous round's array, so the
-// result does not depend on scheduling).
+// Jones-Plassmann colouring: a group whose neighbours of higher priority all
+// have their colours takes the smallest one unused by them.  Its neighbours of
+// lower priority wait for it, so its colour follows from the priorities alone,
+// whatever the order in which groups get there: there are no rounds, every
+// group polls until it can be coloured.
 //
+// A body's groups get their colours in order of priority, so a group is ready
+// when as many groups of each of its bodies have theirs as come before it there
+// (its rank), and the colours to avoid are all those taken at the two bodies.
+// A body's state is the set of its taken colours and the number of its groups in
+// the sequential tail.  A group adds to one of the two, in one store (nobody else
+// writes there until it has), so their sum is the rank only when both are final.
+// priority rank of a group on a body: item(i) is the body's i-th group
+template <class Item>
+AMD_INLINE int colour_rank(int g, int deg, Item item) {
+    constexpr int kAhead = 4;
+    int rank = 0;
+    for (int i0 = 0; i0 < deg; i0 += kAhead) {
+        int h[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) h[u] = item(min(i0 + u, deg - 1));
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) rank += i0 + u < deg && higher((uint32_t)h[u], (uint32_t)g) ? 1 : 0;
+    }
+    return rank;
+}
+// sequential tail if all 64 parallel colours are taken
+AMD_INLINE int free_colour(unsigned long long used) { return ~used != 0 ? __ffsll((long long)~used) - 1 : kMaxColours; }
+
 // With layers (the single sweep's breadth-first layers), a group also waits
 // for its neighbours of lower layers and takes a colour above all of theirs,
 // so along every body the sweep visits the groups layer by layer; only
 // neighbours of its own layer compete for colours.  Colours then may pass
 // the parallel ones: those groups run in the sequential tail in colour order.
-__global__ void k_colour_round(int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
-                               const int* inc_count, const int* inc_items, const int* col_in, int* col_out,
-                               int* remaining, const int* layer, int* blocker) {
-    int g = blockIdx.x * blockDim.x + threadIdx.x;
+// A quad of lanes holds a group and goes through the lists of its two bodies 16
+// neighbours at a time.  colour_of(h), item(i), layer_of(h): the colour of a
+// group (negative: none yet), entry i of the bodies' lists, a group's layer.
+// try_layered gives the group's colour, or -1 and the neighbour it waits for.
+struct ColourLists {
+    int start_a, n_a, start_b, n_b;
+};
+constexpr int kQuadSwap1 = 0xB1, kQuadSwap2 = 0x4E;  // quad_perm: lanes 0-1 and 2-3, then the pairs
+AMD_INLINE unsigned quad_or(unsigned v) {
+    v |= (unsigned)__builtin_amdgcn_mov_dpp((int)v, kQuadSwap1, 0xF, 0xF, true);
+    return v | (unsigned)__builtin_amdgcn_mov_dpp((int)v, kQuadSwap2, 0xF, 0xF, true);
+}
+AMD_INLINE int quad_max(int v) {
+    v = max(v, __builtin_amdgcn_mov_dpp(v, kQuadSwap1, 0xF, 0xF, true));
+    return max(v, __builtin_amdgcn_mov_dpp(v, kQuadSwap2, 0xF, 0xF, true));
+}
+template <class Colour, class Item, class Layer>
+AMD_INLINE int try_layered(int g, const ColourLists& b, Colour colour_of, Item item, Layer layer_of, int& blocker) {
+    constexpr int kAhead = 4;
+    const int lane = threadIdx.x & 3, n = b.n_a + b.n_b, lg = layer_of(g);
+    int lo = 0;                   // the colour must be at least lo (above every lower-layer neighbour)
+    unsigned long long used = 0;  // colours lo .. lo + 63 taken by same-layer neighbours
+    for (int pass = 0; pass < 2; pass++) {
+        for (int i0 = 0; i0 < n; i0 += 4 * kAhead) {
+            int h[kAhead], ch[kAhead], lh[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int i = min(i0 + 4 * u + lane, n - 1);
+                h[u] = item(i < b.n_a ? b.start_a + i : b.start_b + i - b.n_a);
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                ch[u] = colour_of(h[u]);
+                lh[u] = layer_of(h[u]);
+            }
+            int wait = -1;
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                if (h[u] == g) continue;
+                if (pass == 0) {
+                    if (lh[u] >= lg) continue;
+                    if (ch[u] < 0) wait = h[u];
+                    else lo = max(lo, ch[u] + 1);
+                } else {
+                    if (lh[u] != lg) continue;
+                    if (ch[u] < 0) {
+                        if (higher((uint32_t)h[u], (uint32_t)g)) wait = h[u];
+                    } else if (ch[u] >= lo && ch[u] - lo < 64) {
+                        used |= 1ull << (ch[u] - lo);
+                    }
+                }
+            }
+            wait = quad_max(wait);
+            if (wait >= 0) {
+                blocker = wait;
+                return -1;
+            }
+        }
+        lo = quad_max(lo);
+    }
+    used = ((unsigned long long)quad_or((unsigned)(used >> 32)) << 32) | quad_or((unsigned)used);
+    return lo + free_colour(used);
+}
+AMD_INLINE int ld_int(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+AMD_INLINE void st_int(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+AMD_INLINE unsigned long long ld_u64(const unsigned long long* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+AMD_INLINE void st_u64(unsigned long long* p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// colour[] starts negative, taken[] (by body) empty.  A thread's groups are
+// g, g + threads, ...; it polls those without a colour in turn, a bounded number
+// of times: if some are left then (workgroups that were not resident together),
+// *remaining is set and the launch is repeated.  What bounds it is the chain of
+// groups each waiting for another, a link of which costs a store and the load
+// that sees it (settled 20,000-box pile, 104,000 groups: 84 us; a launch per
+// round of the colouring, which went through the lists again, took 1500).
+constexpr int kColourPolls = 20000;
+// rank[2 g + side]: the group's priority rank on its body, -1 for a pinned one
+__global__ void k_colour_ranks(int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
+                               const int* inc_count, const int* inc_items, int* rank) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, g = i >> 1;
     if (g >= n_groups) return;
-    int c = col_in[g];
-    if (c >= 0) {
-        col_out[g] = c;
-        return;
+    const int e = (i & 1) ? gb[g] : ga[g];
+    int r = -1;
+    if (dynamic_body(bflags, e)) {
+        const int* list = &inc_items[inc_start[e]];
+        r = colour_rank(g, inc_count[e], [&](int k) { return list[k]; });
     }
-    const int lg = layer ? layer[g] : 0;
-    int lo = 0;  // the colour must be at least lo (above every lower-layer neighbour)
-    // The neighbour that kept this group waiting in an earlier round keeps it
-    // waiting while it is uncoloured (priorities and layers do not change),
-    // so the incidence lists are scanned again only once it has its colour.
-    const int bl = blocker[g];
-    bool ready = !(bl >= 0 && col_in[bl] < 0);
-    const int bodies[2] = {ga[g], gb[g]};
-    if (layer) {
-        for (int s = 0; s < 2 && ready; s++) {
-            int e = bodies[s];
-            if (!dynamic_body(bflags, e)) continue;
-            int st = inc_start[e], cnt = inc_count[e];
-            for (int q = 0; q < cnt; q++) {
-                int h = inc_items[st + q];
-                if (h == g || layer[h] >= lg) continue;
-                int ch = col_in[h];
-                if (ch < 0) {
-                    ready = false;
-                    blocker[g] = h;
-                    break;
-                }
-                lo = max(lo, ch + 1);
-            }
+    rank[i] = r;
+}
+__global__ __launch_bounds__(256) void k_colour(int n_groups, const int* ga, const int* gb, const int* rank,
+                                                int* colour, TakenColours* taken, int* remaining) {
+    const int threads = gridDim.x * blockDim.x, first = blockIdx.x * blockDim.x + threadIdx.x;
+    struct Group {
+        int a, b, ra, rb;
+    };
+    auto load = [&](int g) { return Group{ga[g], gb[g], rank[2 * g], rank[2 * g + 1]}; };
+    // true once the group has its colour
+    auto attempt = [&](int g, const Group& m) {
+        unsigned long long set_a = 0, set_b = 0, tail_a = 0, tail_b = 0;
+        if (m.ra >= 0) {
+            set_a = ld_u64(&taken[m.a].set);
+            tail_a = ld_u64(&taken[m.a].in_tail);
         }
-    }
-    uint64_t used = 0;  // colours lo .. lo + 63 taken by same-layer neighbours
-    for (int s = 0; s < 2 && ready; s++) {
-        int e = bodies[s];
-        if (!dynamic_body(bflags, e)) continue;
-        int st = inc_start[e], cnt = inc_count[e];
-        for (int q = 0; q < cnt; q++) {
-            int h = inc_items[st + q];
-            if (h == g || (layer && layer[h] != lg)) continue;
-            int ch = col_in[h];
-            if (ch < 0) {
-                if (higher((uint32_t)h, (uint32_t)g)) {
-                    ready = false;
-                    blocker[g] = h;
-                    break;
-                }
-            } else if (ch >= lo && ch - lo < 64) {
-                used |= (uint64_t)1 << (ch - lo);
-            }
+        if (m.rb >= 0) {
+            set_b = ld_u64(&taken[m.b].set);
+            tail_b = ld_u64(&taken[m.b].in_tail);
         }
-    }
-    int pick = -1;
-    if (ready) {
-        if (!layer) {
-            pick = kMaxColours;  // sequential tail if all 64 parallel colours are taken
-            if (~used != 0) pick = __ffsll((long long)~used) - 1;
+        if ((m.ra >= 0 && __popcll(set_a) + (int)tail_a != m.ra) || (m.rb >= 0 && __popcll(set_b) + (int)tail_b != m.rb))
+            return false;
+        const int c = free_colour(set_a | set_b);
+        colour[g] = c;
+        if (c < kMaxColours) {
+            if (m.ra >= 0) st_u64(&taken[m.a].set, set_a | 1ull << c);
+            if (m.rb >= 0) st_u64(&taken[m.b].set, set_b | 1ull << c);
         } else {
-            pick = lo + (~used != 0 ? __ffsll((long long)~used) - 1 : 64);
+            if (m.ra >= 0) st_u64(&taken[m.a].in_tail, tail_a + 1);
+            if (m.rb >= 0) st_u64(&taken[m.b].in_tail, tail_b + 1);
+        }
+        return true;
+    };
+    // the thread's first group (its only one up to 500,000 groups) in registers
+    Group m = {0, 0, -1, -1};
+    bool done = first >= n_groups || colour[first] >= 0;
+    if (!done) m = load(first);
+    for (int polls = 0;; polls++) {
+        if (!done) done = attempt(first, m);
+        bool left = !done;
+        for (int g = first + threads; g < n_groups; g += threads)
+            if (colour[g] < 0 && !attempt(g, load(g))) left = true;
+        if (!__any(left)) return;
+        if (polls >= kColourPolls) {
+            *remaining = 1;
+            return;
         }
     }
-    col_out[g] = pick;
-    // some group is still uncoloured: one flag store per wave
-    const unsigned long long waiting = __ballot(!ready);
-    if (waiting && (int)(threadIdx.x & 63) == __ffsll((long long)__ballot(1)) - 1) *remaining = 1;
+}
+// with layers: a quad per group, polling colour[] itself
+__global__ __launch_bounds__(256) void k_colour_layered(int n_groups, const int* ga, const int* gb, const int* bflags,
+                                                        const int* inc_start, const int* inc_count,
+                                                        const int* inc_items, int* colour, int* remaining,
+                                                        const int* layer, int* blocker) {
+    const int quads = gridDim.x * (blockDim.x / 4), quad = (blockIdx.x * blockDim.x + threadIdx.x) / 4;
+    for (int polls = 0;; polls++) {
+        bool left = false;
+        for (int g = quad; g < n_groups; g += quads) {
+            if (ld_int(&colour[g]) >= 0) continue;
+            // the neighbour that kept this group waiting keeps it waiting while it is uncoloured
+            int bl = ld_int(&blocker[g]);
+            int c = -1;
+            if (bl < 0 || quad_max(ld_int(&colour[bl])) >= 0) {
+                const int a = ga[g], b = gb[g];
+                ColourLists l = {0, 0, 0, 0};
+                if (dynamic_body(bflags, a)) l.start_a = inc_start[a], l.n_a = inc_count[a];
+                if (dynamic_body(bflags, b)) l.start_b = inc_start[b], l.n_b = inc_count[b];
+                c = try_layered(
+                    g, l, [&](int h) { return ld_int(&colour[h]); }, [&](int i) { return inc_items[i]; },
+                    [&](int h) { return layer[h]; }, bl);
+                if (c >= 0) st_int(&colour[g], c);
+                else st_int(&blocker[g], bl);
+            }
+            left = left || c < 0;
+        }
+        if (!__any(left)) return;
+        if (polls >= kColourPolls) {
+            *remaining = 1;
+            return;
+        }
+    }
 }
 
 // Sort key of a group: colour, then (inside a parallel colour, where groups
@@ -268,37 +394,53 @@ __global__ void k_solve_order(int n_groups, const uint64_t* sorted, const int* g
 // is the incidence (2 q' + s') of the update of that body just before this
 // one: the group ranked one lower, or for rank 0 the body's last group, whose
 // update of the previous pass comes first.
-__global__ void k_flow_ranks(int n_ent, const int* bflags, const int* inc_start, const int* inc_count,
-                             const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n_ent || !dynamic_body(bflags, a)) return;
-    const int s = inc_start[a], d = inc_count[a];
-    auto incidence = [&](int q) { return 2 * q + (group_desc[4 * q + 2] == a ? 0 : 1); };
-    for (int i = 0; i < d; i++) {
-        const int qi = spos[inc_items[s + i]];
-        int r = 0, before = -1, last = -1;
-        for (int j = 0; j < d; j++) {
-            const int qj = spos[inc_items[s + j]];
-            if (qj < qi) {
-                r++;
-                before = max(before, qj);
+//
+// The rank of group q on a body, and the position of the one before it (for
+// rank 0 the body's last): spos_of(i) is the position of the body's i-th group.
+template <class Spos>
+AMD_INLINE int flow_rank(int q, int deg, Spos spos_of, int& pred) {
+    constexpr int kAhead = 4;
+    int rank = 0, before = -1, last = -1;
+    for (int i0 = 0; i0 < deg; i0 += kAhead) {
+        int qi[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) qi[u] = spos_of(min(i0 + u, deg - 1));
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            if (qi[u] < q) {
+                rank += i0 + u < deg ? 1 : 0;
+                before = max(before, qi[u]);
             }
-            last = max(last, qj);
+            last = max(last, qi[u]);
         }
-        const int side = group_desc[4 * qi + 2] == a ? 0 : 1;
-        flow[4 * qi + 2 * side] = r;
-        flow[4 * qi + 2 * side + 1] = d;
-        pred[2 * qi + side] = incidence(before >= 0 ? before : last);
     }
+    pred = before >= 0 ? before : last;
+    return rank;
+}
+// A thread per group and side: the lists are short, and the loads of several
+// entries are in flight together (a thread per body, one entry at a time, took
+// 193 us on the settled 20,000-box pile; this takes 17).
+__global__ void k_flow_ranks(int n_groups, const int* bflags, const int* inc_start, const int* inc_count,
+                             const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, q = i >> 1, side = i & 1;
+    if (q >= n_groups) return;
+    const int e = group_desc[4 * q + 2 + side];
+    int rank = 0, deg = 0, before = 0;
+    if (dynamic_body(bflags, e)) {
+        const int start = inc_start[e];
+        deg = inc_count[e];
+        int of;
+        rank = flow_rank(q, deg, [&](int k) { return spos[inc_items[start + k]]; }, of);
+        before = 2 * of + (group_desc[4 * of + 2] == e ? 0 : 1);
+    }
+    reinterpret_cast<int2*>(flow)[i] = make_int2(rank, deg);
+    pred[i] = before;
 }
 
-void launch_flow_ranks(hipStream_t s, int n_ent, int n_groups, const int* bflags, const int* inc_start,
-                       const int* inc_count, const int* inc_items, const int* spos, const int* group_desc,
-                       int* flow, int* pred) {
-    fill_int(s, flow, 4 * n_groups, 0);
-    fill_int(s, pred, 2 * n_groups, 0);
-    if (n_ent > 0 && n_groups > 0)
-        hipLaunchKernelGGL(k_flow_ranks, dim3((n_ent + 255) / 256), dim3(256), 0, s, n_ent, bflags, inc_start,
+void launch_flow_ranks(hipStream_t s, int n_groups, const int* bflags, const int* inc_start, const int* inc_count,
+                       const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred) {
+    if (n_groups > 0)
+        hipLaunchKernelGGL(k_flow_ranks, dim3((2 * n_groups + 255) / 256), dim3(256), 0, s, n_groups, bflags, inc_start,
                            inc_count, inc_items, spos, group_desc, flow, pred);
 }
 
@@ -1558,6 +1700,8 @@ enum { kSideDyn = 1, kSideSelf = 2, kSideRank0 = 4, kSideLast = 8 };
 
 struct ResidentSteps {
     int n[kMaxColours + 1], per[kMaxColours + 1], first[kMaxColours + 1];
+    int start[kMaxColours + 2];  // first sorted group of each colour
+    int colours;                 // up to the last one that has groups
 };
 struct ResidentLds {
     double2 region[kResDoubles / 2];       // the waves' groups, each wave as much as the plan counted for it
@@ -1582,30 +1726,43 @@ static_assert(sizeof(ResidentLds) <= 160 * 1024, "LDS of a CU");
 // 8 colours in a row then fall to different waves (27,000 contacts of 48 batched
 // scenes need 25,000 doubles in the fullest workgroup when they follow each
 // other, and fit like this).  A wave takes its steps colour by colour.
+// Called by a whole workgroup of more than kMaxColours threads.
 AMD_INLINE void resident_steps(const int* cs, int W, ResidentSteps& S) {
-    int total = 0;
-    for (int c = 0; c <= kMaxColours; c++) {
-        const int g = cs[c + 1] - cs[c];
-        S.per[c] = c < kMaxColours ? max(1, min(kQuads, (g + W - 1) / W)) : 1;
-        S.n[c] = (g + S.per[c] - 1) / S.per[c];
-        S.first[c] = total % W;
-        total += S.n[c];
+    const int c = threadIdx.x;
+    if (c <= kMaxColours) {
+        const int start = cs[c], g = cs[c + 1] - start;
+        const int per = c < kMaxColours ? max(1, min(kQuads, (g + W - 1) / W)) : 1;
+        S.start[c] = start;
+        if (c == kMaxColours) S.start[c + 1] = start + g;
+        S.per[c] = per;
+        S.n[c] = (g + per - 1) / per;
     }
-    if (total > W)
-        for (int c = 0; c <= kMaxColours; c++) S.first[c] = (int)((long)(c & 7) * 5 * W / 8) % W;
+    __syncthreads();
+    if (c <= kMaxColours) {
+        int before = 0, total = 0, used = 0;
+        for (int k = 0; k <= kMaxColours; k++) {
+            const int n = S.n[k];
+            before = k == c ? total : before;
+            used = n ? k + 1 : used;
+            total += n;
+        }
+        S.first[c] = total > W ? (int)((long)(c & 7) * 5 * W / 8) % W : before % W;
+        if (c == 0) S.colours = used;
+    }
+    __syncthreads();
 }
 struct StepWalk {
     int c = -1, i = 0;
     // the wave's next step: its first sorted group and its groups; false at the end
-    AMD_INLINE bool next(const ResidentSteps& S, const int* cs, int W, int w, int& q0, int& count) {
+    AMD_INLINE bool next(const ResidentSteps& S, int W, int w, int& q0, int& count) {
         if (c >= 0) i += W;
         while (c < 0 || i >= S.n[c]) {
-            if (++c > kMaxColours) return false;
+            if (++c >= S.colours) return false;
             i = w - S.first[c];
             if (i < 0) i += W;
         }
-        q0 = cs[c] + i * S.per[c];
-        count = min(S.per[c], cs[c + 1] - q0);
+        q0 = S.start[c] + i * S.per[c];
+        count = min(S.per[c], S.start[c + 1] - q0);
         return true;
     }
 };
@@ -1615,14 +1772,13 @@ struct StepWalk {
 __global__ __launch_bounds__(256) void k_resident_plan(const int* cs, const int* group_desc, int W, int* used,
                                                        int* plan) {
     __shared__ ResidentSteps S;
-    if (threadIdx.x == 0) resident_steps(cs, W, S);
-    __syncthreads();
+    resident_steps(cs, W, S);
     const int w = blockIdx.x * blockDim.x + threadIdx.x;
     if (w >= W) return;  // W is a multiple of kResWaves, which divides the wavefront
     const int4* gdesc = reinterpret_cast<const int4*>(group_desc);
     int sum = 0, steps = 0, q0, count;
     StepWalk walk;
-    while (walk.next(S, cs, W, w, q0, count)) {
+    while (walk.next(S, W, w, q0, count)) {
         const int contacts = gdesc[q0 + count - 1].y - gdesc[q0].x;
         sum += count * kResGroup + min(contacts, kResDoubles) * kResContact;
         steps++;
@@ -1641,11 +1797,378 @@ void launch_resident_plan(hipStream_t s, const int* colour_start, const int* gro
                        used, plan);
 }
 
+// LDS operations of one wave are performed in order: only the compiler is held back
+AMD_INLINE void lds_order() { asm volatile("" ::: "memory"); }
+// ---------------------------------------------------------------------------
+// The layout of a small contact set in one workgroup: incidence lists, colours,
+// sorted groups, sweep order, flow ranks and the resident kernel's plan, which
+// are some 20 launches otherwise (and were up to 100, with a launch per
+// colouring round).  What bounds it is latency: the colouring's chain of
+// groups, each waiting for a neighbour, runs in LDS (20 us for 3 groups, 56 for
+// 1,700).
+constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64;
+constexpr int kSmallBins = kMaxColours * 16 + 1;  // (colour, 15 - size), then the tail
+struct SmallLds {
+    short colour[kSmallLayout];             // then each group's sorted position
+    short sorted[kSmallLayout];             // with layers the group waited for; then the group at each sorted position
+    unsigned short item[2 * kSmallLayout];  // each body's groups
+    union {
+        struct {  // a body's, at the start of its groups (TakenColours)
+            unsigned long long set[2 * kSmallLayout];
+            unsigned short in_tail[2 * kSmallLayout];
+        };
+        struct {
+            unsigned short start_a, n_a, start_b, n_b;
+        } lists[kSmallLayout];
+        struct {
+            unsigned short hist[kSmallWaves][kSmallBins + 7];
+            int pos[kSmallLayout + 1];
+        };
+    };
+    int wave_sum[kSmallWaves];
+    int cs[kMaxColours + 2];
+    int n_items;
+    int plan[2];
+    ResidentSteps steps;
+};
+static_assert(sizeof(SmallLds) <= 160 * 1024, "LDS of a CU");
+
+// exclusive sum of v over the workgroup; wave_sum is scratch
+AMD_INLINE int small_exclusive(int v, int* wave_sum) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += t;
+    }
+    __syncthreads();
+    if (lane == 63) wave_sum[wave] = inc;
+    __syncthreads();
+    int before = 0;
+    for (int k = 0; k < kSmallWaves; k++) before += k < wave ? wave_sum[k] : 0;
+    return before + inc - v;
+}
+// the lanes of the wave with this lane's key (of 11 bits) that are in
+AMD_INLINE unsigned long long same_key(int key, bool in) {
+    unsigned long long m = __ballot(in);
+#pragma unroll
+    for (int b = 0; b < 11; b++) {
+        const unsigned long long v = __ballot((key >> b) & 1);
+        m &= (key >> b) & 1 ? v : ~v;
+    }
+    return m;
+}
+static_assert(kSmallBins <= 1 << 11, "same_key");
+
+__global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs A) {
+    __shared__ SmallLds L;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, n = A.n_groups;
+    constexpr int kPer = kSmallLayout / kSmallThreads;
+
+    // incidence lists: a body's groups in any order
+    for (int e = t; e < A.n_ent; e += kSmallThreads) st_int(&A.inc_count[e], 0);
+    if (t == 0) L.n_items = 0;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    int body[kPer][2], at[kPer][2], count[kPer][2];  // this thread's groups; -1: a pinned body
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int g = t + k * kSmallThreads;
+        body[k][0] = g < n ? A.ga[g] : -1;
+        body[k][1] = g < n ? A.gb[g] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            if (body[k][s] >= 0 && !dynamic_body(A.bflags, body[k][s])) body[k][s] = -1;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int g = t + k * kSmallThreads;
+#pragma unroll
+        for (int s = 0; s < 2; s++) at[k][s] = body[k][s] >= 0 ? atomicAdd(&A.inc_count[body[k][s]], 1) : 0;
+        if (g < n) {
+            L.colour[g] = -1;
+            L.sorted[g] = -1;
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    for (int e = t; e < A.n_ent; e += kSmallThreads) {
+        const int c = ld_int(&A.inc_count[e]);
+        if (c > 0) {
+            const int start = atomicAdd(&L.n_items, c);
+            st_int(&A.inc_start[e], start);
+            if (!A.layer) {
+                L.set[start] = 0;
+                L.in_tail[start] = 0;
+            }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    int start[kPer][2];
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            start[k][s] = body[k][s] >= 0 ? ld_int(&A.inc_start[body[k][s]]) : 0;
+            count[k][s] = body[k][s] >= 0 ? ld_int(&A.inc_count[body[k][s]]) : 0;
+        }
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int g = t + k * kSmallThreads;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            if (body[k][s] >= 0) L.item[start[k][s] + at[k][s]] = (unsigned short)g;
+        if (A.layer && g < n) {
+            L.lists[g].start_a = (unsigned short)start[k][0];
+            L.lists[g].n_a = (unsigned short)count[k][0];
+            L.lists[g].start_b = (unsigned short)start[k][1];
+            L.lists[g].n_b = (unsigned short)count[k][1];
+        }
+    }
+    __syncthreads();
+
+    // colours
+    if (!A.layer) {
+        // as k_colour
+        int rank[kPer][2];
+        bool done[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int g = t + k * kSmallThreads;
+            done[k] = g >= n;
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+                rank[k][s] = body[k][s] >= 0 ? colour_rank(g, count[k][s],
+                                                           [&](int i) { return (int)L.item[start[k][s] + i]; })
+                                             : 0;
+        }
+        bool left = true;
+        while (left) {
+            left = false;
+#pragma unroll
+            for (int k = 0; k < kPer; k++) {
+                unsigned long long set[2] = {0, 0};
+                int tail[2] = {0, 0};
+                bool ready = !done[k];
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+                    if (!done[k] && body[k][s] >= 0) {
+                        set[s] = __hip_atomic_load(&L.set[start[k][s]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        tail[s] = __hip_atomic_load(&L.in_tail[start[k][s]], __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+                        ready = ready && __popcll(set[s]) + tail[s] == rank[k][s];
+                    }
+                if (ready) {
+                    const int c = free_colour(set[0] | set[1]);
+                    L.colour[t + k * kSmallThreads] = (short)c;
+#pragma unroll
+                    for (int s = 0; s < 2; s++) {
+                        if (body[k][s] < 0) continue;
+                        if (c < kMaxColours)
+                            __hip_atomic_store(&L.set[start[k][s]], set[s] | 1ull << c, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+                        else
+                            __hip_atomic_store(&L.in_tail[start[k][s]], (unsigned short)(tail[s] + 1), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                    done[k] = true;
+                }
+                left = left || __any(!done[k]);
+            }
+        }
+    } else {
+        auto get = [](const short* p) {
+            return (int)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        auto set = [](short* p, int v) {
+            __hip_atomic_store(p, (short)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        bool left = true;
+        while (__any(left)) {
+            left = false;
+            for (int g = t / 4; g < n; g += kSmallThreads / 4) {
+                if (get(&L.colour[g]) >= 0) continue;
+                int bl = get(&L.sorted[g]);
+                int c = -1;
+                if (bl < 0 || get(&L.colour[bl]) >= 0) {
+                    const auto l = L.lists[g];
+                    c = try_layered(
+                        g, ColourLists{l.start_a, l.n_a, l.start_b, l.n_b}, [&](int h) { return get(&L.colour[h]); },
+                        [&](int i) { return (int)L.item[i]; }, [&](int h) { return A.layer[h]; }, bl);
+                    if (c >= 0) set(&L.colour[g], c);
+                    else set(&L.sorted[g], bl);
+                }
+                left = left || c < 0;
+            }
+        }
+    }
+    __syncthreads();
+
+    // sorted positions: a stable counting sort over (colour, larger groups first)
+    for (int i = t; i < kSmallWaves * (kSmallBins + 7); i += kSmallThreads) (&L.hist[0][0])[i] = 0;
+    __syncthreads();
+    const int chunk = ((n + kSmallThreads - 1) / kSmallThreads) * 64;  // of a wave
+    auto bin_of = [&](int g) {
+        const int c = L.colour[g];
+        return c < kMaxColours ? c * 16 + 15 - min(A.group_start[g + 1] - A.group_start[g], 15) : kSmallBins - 1;
+    };
+    int bin[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int g = wave * chunk + 64 * k + lane;
+        const bool in = 64 * k < chunk && g < n;
+        bin[k] = in ? bin_of(g) : 0;
+        const unsigned long long m = same_key(bin[k], in);
+        if (in && __ffsll((long long)m) - 1 == lane) L.hist[wave][bin[k]] += (unsigned short)__popcll(m);
+        lds_order();
+    }
+    __syncthreads();
+    {
+        int sum = 0;
+        for (int v = 0; v < kSmallWaves; v++) sum += L.hist[v][t];
+        const int base = small_exclusive(sum, L.wave_sum);
+        int run = base;
+        for (int v = 0; v < kSmallWaves; v++) {
+            const int count = L.hist[v][t];
+            L.hist[v][t] = (unsigned short)run;
+            run += count;
+        }
+        if (t % 16 == 0) L.cs[t / 16] = base;
+        if (t == kSmallThreads - 1) {  // the tail's bin
+            L.cs[kMaxColours] = run;
+            L.cs[kMaxColours + 1] = n;
+            for (int v = 0; v < kSmallWaves; v++) {
+                const int count = L.hist[v][kSmallBins - 1];
+                L.hist[v][kSmallBins - 1] = (unsigned short)run;
+                run += count;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int g = wave * chunk + 64 * k + lane;
+        const bool in = 64 * k < chunk && g < n;
+        const unsigned long long m = same_key(bin[k], in);
+        const int q = L.hist[wave][bin[k]] + __popcll(m & ((1ull << lane) - 1));
+        lds_order();
+        if (in && __ffsll((long long)m) - 1 == lane) L.hist[wave][bin[k]] += (unsigned short)__popcll(m);
+        lds_order();
+        if (in) L.sorted[q] = (short)g;
+    }
+    __syncthreads();
+    // the tail in the order of its colours
+    const int tail = L.cs[kMaxColours], n_tail = n - tail;
+    if (A.layer && n_tail > 1) {
+        int to[kPer], who[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int i = t + k * kSmallThreads;
+            if (i >= n_tail) continue;
+            who[k] = L.sorted[tail + i];
+            const int c = L.colour[who[k]];
+            int before = 0;
+            for (int j = 0; j < n_tail; j++) {
+                const int cj = L.colour[L.sorted[tail + j]];
+                before += cj < c || (cj == c && j < i) ? 1 : 0;
+            }
+            to[k] = before;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kPer; k++)
+            if (t + k * kSmallThreads < n_tail) L.sorted[tail + to[k]] = (short)who[k];
+        __syncthreads();
+    }
+
+    // positions of the groups and their contacts
+    {
+        int size[kPer], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int q = t * kPer + k;
+            size[k] = 0;
+            if (q < n) {
+                const int g = L.sorted[q];
+                L.colour[g] = (short)q;
+                size[k] = A.group_start[g + 1] - A.group_start[g];
+            }
+            sum += size[k];
+        }
+        int run = small_exclusive(sum, L.wave_sum);
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int q = t * kPer + k;
+            if (q <= n) {
+                L.pos[q] = run;
+                A.pos_start[q] = run;
+            }
+            run += size[k];
+        }
+        if (t == kSmallThreads - 1 && n == kSmallLayout) {
+            L.pos[n] = run;
+            A.pos_start[n] = run;
+        }
+    }
+    if (t <= kMaxColours + 1) A.colour_start[t] = L.cs[t];
+    if (t < 2) L.plan[t] = 0;
+    __syncthreads();
+    for (int q = t / 4; q < n; q += kSmallThreads / 4) {
+        const int g = L.sorted[q], o = L.pos[q], size = L.pos[q + 1] - o, k0 = A.group_start[g];
+        const int a = A.ga[g], b = A.gb[g];
+        for (int k = t & 3; k < size; k += 4) {
+            A.order[o + k] = k0 + k;
+            A.pos_a[o + k] = a;
+        }
+        if ((t & 3) == 0) reinterpret_cast<int4*>(A.group_desc)[q] = make_int4(o, o + size, a, b);
+    }
+    // flow ranks (k_flow_ranks): a thread per group and side
+    for (int i = t; i < 2 * n; i += kSmallThreads) {
+        const int q = i >> 1, g = L.sorted[q], e = (i & 1) ? A.gb[g] : A.ga[g];
+        int rank = 0, deg = 0, pred = 0;
+        if (dynamic_body(A.bflags, e)) {
+            const int s0 = ld_int(&A.inc_start[e]);
+            deg = ld_int(&A.inc_count[e]);
+            int of;
+            rank = flow_rank(q, deg, [&](int k) { return (int)L.colour[L.item[s0 + k]]; }, of);
+            pred = 2 * of + (A.ga[L.sorted[of]] == e ? 0 : 1);
+        }
+        reinterpret_cast<int2*>(A.flow)[i] = make_int2(rank, deg);
+        A.pred[i] = pred;
+    }
+    // the resident kernel's plan
+    if (A.waves > 0) {
+        resident_steps(L.cs, A.waves, L.steps);
+        if (t < A.waves) {
+            int sum = 0, steps = 0, q0, count;
+            StepWalk walk;
+            while (walk.next(L.steps, A.waves, t, q0, count)) {
+                sum += count * kResGroup + min(L.pos[q0 + count] - L.pos[q0], kResDoubles) * kResContact;
+                steps++;
+                if (sum > kResDoubles || steps > kResidentSteps) break;
+            }
+            A.used[t] = sum;
+            int total = sum;
+#pragma unroll
+            for (int o = 1; o < kResWaves; o <<= 1) total += __shfl_xor(total, o, 64);
+            atomicMax(&L.plan[0], total);
+            atomicMax(&L.plan[1], steps);
+        }
+    }
+    __syncthreads();
+    if (t < 2) A.colour_start[kMaxColours + 2 + t] = L.plan[t];
+}
+void launch_layout_small(hipStream_t s, const SmallLayoutArgs& A) {
+    hipLaunchKernelGGL(k_layout_small, dim3(1), dim3(kSmallThreads), 0, s, A);
+}
+
 AMD_INLINE int lds_int(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 AMD_INLINE void set_lds_int(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 AMD_INLINE void lds_landed() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0)
-// LDS operations of one wave are performed in order: only the compiler is held back
-AMD_INLINE void lds_order() { asm volatile("" ::: "memory"); }
 
 // One contact as a lane of its quad needs it: its three J entries and update
 // coefficients per row, and the contact's scalars.
@@ -1712,7 +2235,6 @@ AMD_INLINE void resident_places(int d, int& first, int& second) {
     }
 }
 static_assert(kRecB == 3 && kRecD == 7 && kRecDen == 11 && kRecY == 15 && kRecMu == 19, "resident_places");
-constexpr int kQuadSwap1 = 0xB1, kQuadSwap2 = 0x4E;  // quad_perm: lanes 0-1 and 2-3, then the pairs
 // Contact.getJdv (Contact.java:362-378), the same sum in every lane of the
 // quad.  kExact flips the A.v lanes' entries; otherwise their sum is flipped,
 // which differs only in the sign of a zero.
@@ -1896,11 +2418,10 @@ __global__ __launch_bounds__((kResWaves + 1) * 64) __attribute__((amdgpu_waves_p
     const int W = gridDim.x * kResWaves;
     const int wave = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (threadIdx.x == 0) {
-        resident_steps(cs, W, L.steps);
         L.published = L.known = L.stop = L.failed = 0;
         for (int i = 0; i < kResWaves; i++) L.done[i] = 0;
     }
-    __syncthreads();
+    resident_steps(cs, W, L.steps);
     if (wave == kResWaves) {
         keep_passes(F, L, lane);
         return;
@@ -1940,7 +2461,7 @@ __global__ __launch_bounds__((kResWaves + 1) * 64) __attribute__((amdgpu_waves_p
         int4 gd = make_int4(0, 0, 0, 0), fd = gd;
         int2 pr = make_int2(0, 0);
         auto fetch = [&]() -> bool {
-            if (!walk.next(L.steps, cs, W, w, q0, count)) return false;
+            if (!walk.next(L.steps, W, w, q0, count)) return false;
             const int q = q0 + (quad < count ? quad : 0);
             gd = gdesc[q];
             fd = fdesc[q];
@@ -3020,12 +3541,22 @@ void launch_incidence(hipStream_t s, bool fill, int n_groups, const int* ga, con
     if (!fill) hipLaunchKernelGGL(k_incidence_count, g, b, 0, s, n_groups, ga, gb, bflags, inc_count);
     else hipLaunchKernelGGL(k_incidence_fill, g, b, 0, s, n_groups, ga, gb, bflags, inc_start, inc_cursor, inc_items);
 }
-void launch_colour_round(hipStream_t s, int n_groups, const int* ga, const int* gb, const int* bflags,
-                         const int* inc_start, const int* inc_count, const int* inc_items, const int* col_in,
-                         int* col_out, int* remaining, const int* layer, int* blocker) {
+void launch_colour(hipStream_t s, int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
+                   const int* inc_count, const int* inc_items, int* colour, TakenColours* taken, int* rank,
+                   int* remaining, const int* layer, int* blocker, bool again) {
     if (n_groups <= 0) return;
-    hipLaunchKernelGGL(k_colour_round, dim3((n_groups + 255) / 256), dim3(256), 0, s, n_groups, ga, gb, bflags,
-                       inc_start, inc_count, inc_items, col_in, col_out, remaining, layer, blocker);
+    // at most 8 workgroups on each of 256 CUs: as many as can run at once
+    const int per = layer ? 64 : 256;
+    const dim3 g(std::min((n_groups + per - 1) / per, 2048)), b(256);
+    if (layer) {
+        hipLaunchKernelGGL(k_colour_layered, g, b, 0, s, n_groups, ga, gb, bflags, inc_start, inc_count, inc_items,
+                           colour, remaining, layer, blocker);
+        return;
+    }
+    if (!again)
+        hipLaunchKernelGGL(k_colour_ranks, dim3((2 * n_groups + 255) / 256), b, 0, s, n_groups, ga, gb, bflags,
+                           inc_start, inc_count, inc_items, rank);
+    hipLaunchKernelGGL(k_colour, g, b, 0, s, n_groups, ga, gb, rank, colour, taken, remaining);
 }
 void launch_colour_keys(hipStream_t s, int n_groups, const int* colour, const int* group_start, uint64_t* keys) {
     if (n_groups > 0)

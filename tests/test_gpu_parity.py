@@ -101,6 +101,66 @@ def test_colouring_valid(gpu_lib):
     print("colours", ncol, flush=True)
 
 
+def _priority(g):
+    h = (g * 0x9E3779B1) & 0xFFFFFFFF
+    h ^= h >> 16
+    h = (h * 0x85EBCA6B) & 0xFFFFFFFF
+    h ^= h >> 13
+    return h
+
+
+@pytest.mark.parametrize("pairs,on_platform", [(1, 0), (64, 1), (1025, 63), (500, 200), (4025, 70),
+                                                 (4026, 70), (4096, 0), (4097, 0), (20000, 300)])
+def test_sweep_order_is_the_greedy_colouring(gpu_lib, pairs, on_platform):
+    """The exported order against a plain greedy colouring: groups in order of
+    priority take the smallest colour free at their dynamic bodies (64: the
+    sequential tail), then order by colour, larger groups first, index.
+    `pairs` body pairs of spheres (a chain on a plane, then some alone) and a
+    platform under on_platform boxes (more than 64 of them fill the tail),
+    below, at and above the 4,096 groups that one workgroup lays out."""
+    from adaptivemerging_amd.context import Context
+    from adaptivemerging_amd.scene import Scene
+
+    s = Scene()
+    s.add_plane([0, 0, 0], [0, 1, 0])
+    chain = max(1, pairs // 3)
+    for i in range(chain):  # each touches the plane and the one before it
+        s.add_sphere(0.101, [0.2 * i, 0.1, -30.0])
+    for i in range(pairs - (2 * chain - 1)):
+        s.add_sphere(0.101, [0.5 * (i % 200), 0.1, -40.0 - 0.5 * (i // 200)])
+    if on_platform:
+        s.add_box([40.0, 0.5, 40.0], [100.0, 0.249, 0.0])
+        for i in range(on_platform):
+            s.add_box([0.2, 0.2, 0.2], [100.0 - 10 + (i % 30) * 0.5, 0.598, (i // 30) * 0.5])
+    ctx = Context()
+    ctx.upload(s)
+    ctx.set_params()
+    ctx.detect(0.01)
+    c = ctx.contacts()
+    b, _, _, _, _, _ = s.arrays()
+    pinned = (b["flags"] & 1) != 0
+    key = np.sort(np.stack([c["body1"], c["body2"]], axis=1), axis=1)
+    start = np.concatenate([[0], 1 + np.flatnonzero(np.any(np.diff(key, axis=0) != 0, axis=1)), [len(key)]])
+    n = len(start) - 1
+    assert n == pairs + (on_platform + 1 if on_platform else 0)
+    used, colour = {}, np.zeros(n, int)
+    for g in sorted(range(n), key=lambda g: (_priority(g), g), reverse=True):
+        mine = [used.setdefault(int(e), set()) for e in key[start[g]] if not pinned[e]]
+        col = next(k for k in range(65) if k == 64 or not any(k in u for u in mine))
+        colour[g] = col
+        for u in mine:
+            u.add(col)
+    size = np.minimum(np.diff(start), 15)
+    order = sorted(range(n), key=lambda g: (colour[g], 15 - size[g] if colour[g] < 64 else 0, g))
+    expect = np.concatenate([np.arange(start[g], start[g + 1]) for g in order])
+    print("groups", n, "colours", colour.max() + 1, flush=True)
+    assert np.array_equal(ctx.solve_order(), expect)
+    got, ncol = ctx.colours()
+    assert np.array_equal(got, np.repeat(colour, np.diff(start)))
+    assert ncol == len(set(colour))
+    ctx.close()
+
+
 def test_steps_jenga(gpu_lib):
     scene = workloads.jenga_tower(seed=7, layers=8, overlap=0.001)
     ctx, orc = twin(scene, iterations=50, gravity_amount=9.81, friction_override=1, friction=0.6)
