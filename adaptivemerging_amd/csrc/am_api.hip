@@ -612,8 +612,15 @@ int do_detect(am_ctx* c) {
         launch_pairs_impl(s, true, A, nullptr, c->d_pair_offsets.p, c->d_keys_unsorted.p, (int)c->d_keys.n, sc + 4);
         sort_u64(s, c->d_keys_unsorted.p, c->d_keys.p, np, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
         fill_int(s, sc + 0, 1, np);
+        int* trees = nullptr;
+        if (c->big_trees) {
+            AM_HIP(c, c->d_tree_pairs.ensure(c->d_keys.n));
+            trees = c->d_tree_pairs.p;
+            fill_int(s, sc + 13, 1, 0);
+        }
         launch_narrow(s, false, B, T, c->d_keys.p, sc + 0, np, c->d_slot_entity.p, c->d_member_first.p,
-                      c->d_members.p, c->d_narrow_counts.p, nullptr, contacts_view(c), sc + 4);
+                      c->d_members.p, c->d_narrow_counts.p, nullptr, contacts_view(c), sc + 4, trees,
+                      sc + 13);
         exclusive_scan(s, c->d_narrow_counts.p, c->d_narrow_offsets.p, np, sc + 1, c->d_scan_temp.p);
         AM_HIP(c, hipGetLastError());
         r = read_scalars(c, 1, 1);
@@ -624,7 +631,8 @@ int do_detect(am_ctx* c) {
         c->n_contacts = nc;
         if (nc > 0)
             launch_narrow(s, true, B, T, c->d_keys.p, sc + 0, np, c->d_slot_entity.p, c->d_member_first.p,
-                          c->d_members.p, nullptr, c->d_narrow_offsets.p, contacts_view(c), sc + 4);
+                          c->d_members.p, nullptr, c->d_narrow_offsets.p, contacts_view(c), sc + 4, trees,
+                          sc + 13);
     } else {
         c->n_contacts = 0;
         fill_int(s, sc + 1, 1, 0);
@@ -1106,9 +1114,11 @@ int am_scene_upload_ex(am_ctx* c, const am_body_desc* bodies, int32_t n_bodies, 
         c->n_bpc = c->n_bpc_prev = 0;
         c->ibpc.clear();
         c->n_ic = 0;
+        c->big_trees = false;
         for (int i = 0; i < n_bodies; i++) {
             const am_body_desc& d = bodies[i];
             c->n_phys = i + 1;
+            c->big_trees = c->big_trees || (d.geom == AM_GEOM_TREE && d.tree_count > kWaveTree);
             if (d.geom == AM_GEOM_TREE) {
                 if (d.tree_first < 0 || d.tree_count <= 0 || d.tree_first + d.tree_count > n_nodes)
                     return fail(c, AM_ERR_INVALID, "tree node range out of bounds");

@@ -156,7 +156,8 @@ struct am_ctx {
     int cap_c = 0;
     DBuf<int> c_b1, c_b2, c_bv1, c_bv2, c_info, c_state, c_new;
     DBuf<double> c_pB1, c_nB1, c_t1B1, c_t2B1, c_viol, c_prev, c_J, c_lam, c_lamw, c_b, c_D;
-    DBuf<int> d_narrow_counts, d_narrow_offsets;
+    DBuf<int> d_narrow_counts, d_narrow_offsets, d_tree_pairs;
+    bool big_trees = false;  // some body is a sphere tree of more than kWaveTree nodes
 
     // old contacts (warm start)
     int n_old = 0, table_mask = 0;

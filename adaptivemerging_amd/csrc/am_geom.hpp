@@ -509,9 +509,16 @@ AMD_INLINE bool box_sphere_test(const Shape& box, d3 c, double r) {
 }
 
 // ---------------------------------------------------------------------------
-// Sphere trees: depth-first traversals with an explicit stack that visits
-// children in stored order, i.e. the reference recursion order
-// (CollisionProcessor.java:793-850, 975-1056).
+// Sphere trees: depth-first traversals that visit children in stored order,
+// i.e. the reference recursion order (CollisionProcessor.java:793-850,
+// 975-1056).  A walk says what becomes of an entry (a node, or a pair of
+// nodes): dropped, followed by `count` entries from `first` on, `stride` apart,
+// or a leaf, whose contact (if any) leaf() reports.
+enum { kDrop, kLeaf, kDescend };
+struct WalkStep {
+    int kind;
+    int first, stride, count;
+};
 struct NodeRef {
     d3 c;
     double r;
@@ -524,98 +531,95 @@ AMD_INLINE NodeRef node_ref(const TreeView& T, int g) {
 
 // collideSphereTreeAndPlane: contacts body1 = tree body, body2 = plane,
 // bv2 = the plane's dummy volume, violation = d.
-template <class Sink>
-AMD_INLINE void tree_plane(const TreeView& T, const Shape& body, const Shape& plane, Sink& sink, int* overflow) {
-    const am_body_desc& bd = *body.d;
-    const am_body_desc& pd = *plane.d;
-    d3 n = ld3(pd.plane_n);
-    d3 pp = ld3(pd.plane_p);
-    int stack[kTreeStack];
-    int sp = 0;
-    stack[sp++] = 0;
-    while (sp > 0) {
-        int node = stack[--sp];
-        NodeRef s = node_ref(T, bd.tree_first + node);
-        double d = n.x * s.c.x + n.y * s.c.y + n.z * s.c.z + pd.plane_d - s.r;
-        if (d < 0) {
-            if (s.count == 0) {
-                d3 nm = sub(s.c, pp);
-                double val = dot(nm, n);
-                nm = scale(val, n);
-                d3 cw = sub(s.c, nm);
-                d3 nn = mk(-1.0 * n.x, -1.0 * n.y, -1.0 * n.z);
-                sink.emit(body.body, plane.body, cw, nn, enc_bv(body, node), AM_BV_PLANE, 0, d);
-            } else {
-                if (sp + s.count > kTreeStack) {
-                    atomicOr(overflow, 2);
-                    return;
-                }
-                for (int k = s.count - 1; k >= 0; k--) stack[sp++] = s.first + k;
-            }
-        }
+struct TreePlaneWalk {
+    const TreeView& T;
+    const Shape &body, &plane;
+    AMD_INLINE double distance_to(const NodeRef& s) const {
+        const d3 n = ld3(plane.d->plane_n);
+        return n.x * s.c.x + n.y * s.c.y + n.z * s.c.z + plane.d->plane_d - s.r;
     }
-}
+    AMD_INLINE WalkStep step(int node) const {
+        const NodeRef s = node_ref(T, body.d->tree_first + node);
+        if (!(distance_to(s) < 0)) return {kDrop, 0, 0, 0};
+        return {s.count == 0 ? kLeaf : kDescend, s.first, 1, s.count};
+    }
+    template <class Sink>
+    AMD_INLINE void leaf(int node, Sink& sink) const {
+        const NodeRef s = node_ref(T, body.d->tree_first + node);
+        const double d = distance_to(s);
+        const d3 n = ld3(plane.d->plane_n);
+        d3 nm = sub(s.c, ld3(plane.d->plane_p));
+        double val = dot(nm, n);
+        nm = scale(val, n);
+        d3 cw = sub(s.c, nm);
+        d3 nn = mk(-1.0 * n.x, -1.0 * n.y, -1.0 * n.z);
+        sink.emit(body.body, plane.body, cw, nn, enc_bv(body, node), AM_BV_PLANE, 0, d);
+    }
+};
 
 // collideBoxAndSphereTree: contacts body1 = box, body2 = tree body.
-template <class Sink>
-AMD_INLINE void box_tree(const TreeView& T, const Shape& box, const Shape& body2, Sink& sink, int* overflow) {
-    const am_body_desc& bd = *body2.d;
+struct BoxTreeWalk {
+    const TreeView& T;
+    const Shape &box, &body2;
+    AMD_INLINE WalkStep step(int node) const {
+        const NodeRef s = node_ref(T, body2.d->tree_first + node);
+        if (!box_sphere_test(box, s.c, s.r)) return {kDrop, 0, 0, 0};
+        return {s.count == 0 ? kLeaf : kDescend, s.first, 1, s.count};
+    }
+    template <class Sink>
+    AMD_INLINE void leaf(int node, Sink& sink) const {
+        const NodeRef s = node_ref(T, body2.d->tree_first + node);
+        box_sphere(box, body2, s.c, s.r, node, sink);
+    }
+};
+
+// collideSphereTrees + processCollision.  Entries pack node1 (low 16 bits) and
+// node2 (high 16 bits).
+struct TreeTreeWalk {
+    const TreeView& T;
+    const Shape &S1, &S2;
+    AMD_INLINE WalkStep step(int e) const {
+        const int n1 = e & 0xffff, n2 = (e >> 16) & 0xffff;
+        const NodeRef s1 = node_ref(T, S1.d->tree_first + n1), s2 = node_ref(T, S2.d->tree_first + n2);
+        if (!(distance_sq(s1.c, s2.c) < (s1.r + s2.r) * (s1.r + s2.r))) return {kDrop, 0, 0, 0};
+        const bool l1 = s1.count == 0, l2 = s2.count == 0;
+        if (l1 && l2) return {kLeaf, 0, 0, 0};
+        if (l1 || (!l2 && s1.r <= s2.r)) return {kDescend, n1 | (s2.first << 16), 1 << 16, s2.count};
+        return {kDescend, s1.first | (n2 << 16), 1, s1.count};
+    }
+    template <class Sink>
+    AMD_INLINE void leaf(int e, Sink& sink) const {
+        const int n1 = e & 0xffff, n2 = (e >> 16) & 0xffff;
+        const NodeRef s1 = node_ref(T, S1.d->tree_first + n1), s2 = node_ref(T, S2.d->tree_first + n2);
+        double dist = distance(s1.c, s2.c);
+        double sum = s2.r + s1.r;
+        if (dist < sum) {
+            double alpha = (s1.r - s2.r + dist) / (2 * dist);
+            d3 p = mk((1 - alpha) * s1.c.x + alpha * s2.c.x, (1 - alpha) * s1.c.y + alpha * s2.c.y,
+                      (1 - alpha) * s1.c.z + alpha * s2.c.z);
+            d3 nrm = normalized(sub(s2.c, s1.c));
+            sink.emit(S1.body, S2.body, p, nrm, enc_bv(S1, n1), enc_bv(S2, n2), 0, dist - sum);
+        }
+    }
+};
+
+// A walk by one thread, with an explicit stack.
+template <class Walk, class Sink>
+AMD_INLINE void walk_thread(const Walk& w, Sink& sink, int* overflow) {
     int stack[kTreeStack];
     int sp = 0;
     stack[sp++] = 0;
     while (sp > 0) {
-        int node = stack[--sp];
-        NodeRef s = node_ref(T, bd.tree_first + node);
-        if (!box_sphere_test(box, s.c, s.r)) continue;
-        if (s.count != 0) {
-            if (sp + s.count > kTreeStack) {
+        const int e = stack[--sp];
+        const WalkStep t = w.step(e);
+        if (t.kind == kLeaf) {
+            w.leaf(e, sink);
+        } else if (t.kind == kDescend) {
+            if (sp + t.count > kTreeStack) {
                 atomicOr(overflow, 2);
                 return;
             }
-            for (int k = s.count - 1; k >= 0; k--) stack[sp++] = s.first + k;
-        } else {
-            box_sphere(box, body2, s.c, s.r, node, sink);
-        }
-    }
-}
-
-// collideSphereTrees + processCollision.
-template <class Sink>
-AMD_INLINE void tree_tree(const TreeView& T, const Shape& S1, const Shape& S2, Sink& sink, int* overflow) {
-    const int f1 = S1.d->tree_first, f2 = S2.d->tree_first;
-    // stack entries pack node1 (low 16 bits) and node2 (high 16 bits)
-    int stack[kTreeStack];
-    int sp = 0;
-    stack[sp++] = 0;
-    while (sp > 0) {
-        int e = stack[--sp];
-        int n1 = e & 0xffff, n2 = (e >> 16) & 0xffff;
-        NodeRef s1 = node_ref(T, f1 + n1);
-        NodeRef s2 = node_ref(T, f2 + n2);
-        if (!(distance_sq(s1.c, s2.c) < (s1.r + s2.r) * (s1.r + s2.r))) continue;
-        bool l1 = s1.count == 0, l2 = s2.count == 0;
-        if (l1 && l2) {
-            double dist = distance(s1.c, s2.c);
-            double sum = s2.r + s1.r;
-            if (dist < sum) {
-                double alpha = (s1.r - s2.r + dist) / (2 * dist);
-                d3 p = mk((1 - alpha) * s1.c.x + alpha * s2.c.x, (1 - alpha) * s1.c.y + alpha * s2.c.y,
-                          (1 - alpha) * s1.c.z + alpha * s2.c.z);
-                d3 nrm = normalized(sub(s2.c, s1.c));
-                sink.emit(S1.body, S2.body, p, nrm, enc_bv(S1, n1), enc_bv(S2, n2), 0, dist - sum);
-            }
-            continue;
-        }
-        bool down2 = l1 || (!l2 && s1.r <= s2.r);
-        int cnt = down2 ? s2.count : s1.count;
-        if (sp + cnt > kTreeStack) {
-            atomicOr(overflow, 2);
-            return;
-        }
-        if (down2) {
-            for (int k = cnt - 1; k >= 0; k--) stack[sp++] = n1 | ((s2.first + k) << 16);
-        } else {
-            for (int k = cnt - 1; k >= 0; k--) stack[sp++] = (s1.first + k) | (n2 << 16);
+            for (int k = t.count - 1; k >= 0; k--) stack[sp++] = t.first + k * t.stride;
         }
     }
 }
@@ -627,15 +631,15 @@ AMD_INLINE void shape_dispatch(const TreeView& T, const Shape& s1, const Shape& 
     if (g1 == AM_GEOM_PLANE) {
         if (g2 == AM_GEOM_PLANE) return;
         if (g2 == AM_GEOM_BOX) box_plane(s2, s1, sink);
-        else tree_plane(T, s2, s1, sink, overflow);
+        else walk_thread(TreePlaneWalk{T, s2, s1}, sink, overflow);
     } else if (g1 == AM_GEOM_BOX) {
         if (g2 == AM_GEOM_PLANE) box_plane(s1, s2, sink);
         else if (g2 == AM_GEOM_BOX) box_box(s1, s2, sink);
-        else box_tree(T, s1, s2, sink, overflow);
+        else walk_thread(BoxTreeWalk{T, s1, s2}, sink, overflow);
     } else {
-        if (g2 == AM_GEOM_PLANE) tree_plane(T, s1, s2, sink, overflow);
-        else if (g2 == AM_GEOM_BOX) box_tree(T, s2, s1, sink, overflow);
-        else tree_tree(T, s1, s2, sink, overflow);
+        if (g2 == AM_GEOM_PLANE) walk_thread(TreePlaneWalk{T, s1, s2}, sink, overflow);
+        else if (g2 == AM_GEOM_BOX) walk_thread(BoxTreeWalk{T, s2, s1}, sink, overflow);
+        else walk_thread(TreeTreeWalk{T, s1, s2}, sink, overflow);
     }
 }
 

@@ -44,6 +44,71 @@ def test_detect_sphere_trees(gpu_lib):
     assert_contacts_equal(ctx.contacts(), orc.contacts())
 
 
+def _tree(rng, fanouts, radius=0.05, size=0.4):
+    """A sphere tree with fanouts[k] children for every node of level k."""
+    centres, radii, children = [], [], []
+
+    def build(level):
+        node = len(centres)
+        centres.append(rng.uniform(-size / 2, size / 2, 3).tolist())
+        radii.append(radius)
+        children.append([])
+        if level < len(fanouts):
+            children[node] = [build(level + 1) for _ in range(fanouts[level])]
+            radii[node] = 0.9  # encloses everything below it
+        return node
+
+    build(0)
+    return centres, radii, children
+
+
+@pytest.mark.parametrize("fanouts", [[], [6], [7], [8], [1] * 60, [64], [65], [127], [128], [8, 8], [16, 3, 5], [2] * 8])
+def test_detect_trees_walked_by_waves(gpu_lib, fanouts):
+    """Overlapping trees of every shape a wave's stack meets, each against the
+    others, boxes, spheres and a plane: no more nodes than a thread takes (8),
+    long chains, 64 and 65 children, as many as a thread's stack holds.  Same
+    contacts, in the same order, as the oracle's recursion."""
+    from adaptivemerging_amd.scene import Scene
+
+    rng = np.random.default_rng(len(fanouts) + sum(fanouts))
+    s = Scene()
+    s.add_plane([0, 0, 0], [0, 1, 0])
+    for i in range(4 if max(fanouts, default=0) <= 64 else 1):  # two trees of 65 children are refused (below)
+        c, r, ch = _tree(rng, fanouts)
+        s.add_tree(c, r, ch, rng.uniform(-0.1, 0.1, 3) + [0, 0.1, 0])
+    s.add_box([0.3, 0.2, 0.3], [0.1, 0.1, 0.0])
+    s.add_sphere(0.15, [0.0, 0.2, 0.1])
+    s.add_tree([[0, 0, 0], [0.1, 0, 0]], [0.3, 0.1], [[1], []], [0.0, 0.1, 0.0])
+    ctx, orc = twin(s)
+    n_g = ctx.detect(0.01)
+    n_o = orc.detect()
+    print("contacts", n_g, n_o, flush=True)
+    assert n_g == n_o and n_g > 0
+    assert_contacts_equal(ctx.contacts(), orc.contacts())
+    ctx.close()
+
+
+@pytest.mark.parametrize("fanouts,trees", [([2, 128], 1), ([65], 2)])
+def test_detect_refuses_trees_too_wide_for_a_walk(gpu_lib, fanouts, trees):
+    """A thread's stack holds 128 entries: one sibling and 128
+    children, or 64 siblings and the 65 children of the other tree, do not fit."""
+    from adaptivemerging_amd import _lib
+    from adaptivemerging_amd.context import Context
+    from adaptivemerging_amd.scene import Scene
+
+    s = Scene()
+    s.add_plane([0, 0, 0], [0, 1, 0])
+    for _ in range(trees):
+        c, r, ch = _tree(np.random.default_rng(1), fanouts)
+        s.add_tree(c, r, ch, [0.0, 0.1, 0.0])
+    ctx = Context()
+    ctx.upload(s)
+    with pytest.raises(_lib.AMError) as e:
+        ctx.detect(0.01)
+    assert e.value.code == _lib.AM_ERR_CAPACITY
+    ctx.close()
+
+
 @pytest.mark.parametrize("schedule", [0, 1])
 @pytest.mark.parametrize("iterations", [1, 7, 100])
 def test_pgs_jenga_bit_exact(gpu_lib, iterations, schedule):
