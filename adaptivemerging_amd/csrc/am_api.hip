@@ -357,12 +357,12 @@ int am_ctx_create(int32_t device, am_ctx** out) {
         return AM_ERR_HIP;
     }
     default_params(&c->params);
-    if (c->d_scalars.ensure(32) != hipSuccess || hipHostMalloc((void**)&c->h_scalars, 32 * sizeof(int)) != hipSuccess) {
+    if (c->d_scalars.ensure(32) != hipSuccess || hipHostMalloc((void**)&c->h_scalars, kHostInts * sizeof(int)) != hipSuccess) {
         (void)hipStreamDestroy(c->stream);
         delete c;
         return AM_ERR_HIP;
     }
-    std::memset(c->h_scalars, 0, 32 * sizeof(int));
+    std::memset(c->h_scalars, 0, kHostInts * sizeof(int));
     *out = c;
     return AM_OK;
 }
@@ -372,6 +372,7 @@ int am_ctx_destroy(am_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     if (c->h_scalars) (void)hipHostFree(c->h_scalars);
+    if (c->h_sweeps) (void)hipHostFree(c->h_sweeps);
     for (auto& e : c->kev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : c->lev)
@@ -424,7 +425,7 @@ int build_layout(am_ctx* c) {
     if (ng >= (1 << 28)) return fail(c, AM_ERR_INVALID, "more than 2^28 contact groups");
     hipStream_t s = c->stream;
     int* sc = c->d_scalars.p;
-    AM_HIP(c, c->s_colour_start.ensure(kMaxColours + 4));
+    AM_HIP(c, c->s_colour_start.ensure(kMaxColours + 5));
     AM_HIP(c, c->s_group_desc.ensure((size_t)std::max(ng, 1) * 4));
     AM_HIP(c, c->s_flow.ensure((size_t)std::max(ng, 1) * 4));
     AM_HIP(c, c->s_pred.ensure((size_t)std::max(ng, 1) * 2));
@@ -476,14 +477,15 @@ int build_layout(am_ctx* c) {
             fill_u64(s, c->g_taken.p, 2 * (size_t)c->n_ent, 0);
         }
     }
-    int cs[kMaxColours + 4];
+    int* left = c->s_colour_start.p + kMaxColours + 4;
+    const int* cs = c->h_scalars + kHostLayout;
     // again if groups were left without a colour (launch_colour)
     for (int round = 0;; round++) {
         if (!small) {
             if (ng > 0) {
-                fill_int(s, sc + 5, 1, 0);
+                fill_int(s, left, 1, 0);
                 launch_colour(s, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_start.p, c->inc_count.p,
-                              c->inc_items.p, c->g_colour.p, c->g_taken.p, c->g_rank.p, sc + 5, c->layout_layer,
+                              c->inc_items.p, c->g_colour.p, c->g_taken.p, c->g_rank.p, left, c->layout_layer,
                               c->g_blocker.p, round > 0);
                 launch_colour_keys(s, ng, c->g_colour.p, c->g_start.p, c->g_keys.p);
                 sort_u64(s, c->g_keys.p, c->g_keys_sorted.p, ng, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
@@ -498,10 +500,10 @@ int build_layout(am_ctx* c) {
                                      c->s_colour_start.p + kMaxColours + 2);
         }
         AM_HIP(c, hipGetLastError());
-        AM_HIP(c, hipMemcpyAsync(cs, c->s_colour_start.p, sizeof cs, hipMemcpyDeviceToHost, s));
-        int r = read_scalars(c, 5, 1);
-        if (r) return r;
-        if (small || ng == 0 || c->h_scalars[5] == 0) break;
+        AM_HIP(c, hipMemcpyAsync(c->h_scalars + kHostLayout, c->s_colour_start.p, (kMaxColours + 5) * sizeof(int),
+                                 hipMemcpyDeviceToHost, s));
+        AM_HIP(c, hipStreamSynchronize(s));
+        if (small || ng == 0 || cs[kMaxColours + 4] == 0) break;
         if (round == 1000) return fail(c, AM_ERR_HIP, "colouring stopped making progress");
     }
     const bool fits = rgrid > 0 && cs[kMaxColours + 2] <= kResidentDoubles && cs[kMaxColours + 3] <= kResidentSteps;
@@ -545,13 +547,20 @@ int groups_after_contacts(am_ctx* c) {
                       c->g_flags.p, c->g_scanned.p, c->g_start.p, c->g_a.p, c->g_b.p, c->d_scalars.p + 2,
                       c->d_scan_temp.p);
         AM_HIP(c, hipGetLastError());
-        int r = read_scalars(c, 2, 1);
+        int r = read_scalars(c, 2, 3);
         if (r) return r;
         c->n_groups = c->h_scalars[2];
     } else {
         c->n_groups = 0;
     }
     c->layout_valid = false;
+    return AM_OK;
+}
+
+// The overflow flags, as last read
+int detect_flags(am_ctx* c) {
+    if (c->h_scalars[4] & 2) return fail(c, AM_ERR_CAPACITY, "sphere-tree traversal stack overflow (tree too deep)");
+    if (c->h_scalars[4] & 1) return fail(c, AM_ERR_CAPACITY, "contact or pair buffer overflow");
     return AM_OK;
 }
 
@@ -566,8 +575,12 @@ int do_detect(am_ctx* c) {
     const int tsize = c->hash_mask + 1;
     launch_bounds(s, B, T, c->d_grid.p, ng, c->d_sphere.p, c->cell_size, c->d_cell.p, c->hash_mask,
                   c->d_grid_is_large.p);
-    fill_int(s, c->d_bucket_count.p, tsize, 0);
-    fill_int(s, c->d_bucket_cursor.p, tsize, 0);
+    MemBatch m(s);
+    m.fill_int(c->d_bucket_count.p, tsize, 0);
+    m.fill_int(c->d_bucket_cursor.p, tsize, 0);
+    m.fill_int(sc + 4, 1, 0);
+    m.fill_int(sc + 13, 1, 0);
+    m.run();
     launch_buckets(s, c->d_cell.p, ng, c->d_bucket_count.p, nullptr, nullptr, nullptr, false);
     exclusive_scan(s, c->d_bucket_count.p, c->d_bucket_start.p, tsize, sc + 3, c->d_scan_temp.p);
     launch_buckets(s, c->d_cell.p, ng, c->d_bucket_count.p, c->d_bucket_start.p, c->d_bucket_cursor.p,
@@ -589,7 +602,6 @@ int do_detect(am_ctx* c) {
     A.top_sleeping = c->d_top_sleeping.p;
     A.large = c->d_grid_large.p;
     A.n_large = (int)c->grid_large.size();
-    fill_int(s, sc + 4, 1, 0);
     launch_pairs_impl(s, false, A, c->d_pair_counts.p, nullptr, nullptr, 0, sc + 4);
     exclusive_scan(s, c->d_pair_counts.p, c->d_pair_offsets.p, pair_tasks(ng), sc + 0, c->d_scan_temp.p);
     AM_HIP(c, hipGetLastError());
@@ -611,21 +623,20 @@ int do_detect(am_ctx* c) {
         }
         launch_pairs_impl(s, true, A, nullptr, c->d_pair_offsets.p, c->d_keys_unsorted.p, (int)c->d_keys.n, sc + 4);
         sort_u64(s, c->d_keys_unsorted.p, c->d_keys.p, np, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
-        fill_int(s, sc + 0, 1, np);
         int* trees = nullptr;
         if (c->big_trees) {
             AM_HIP(c, c->d_tree_pairs.ensure(c->d_keys.n));
             trees = c->d_tree_pairs.p;
-            fill_int(s, sc + 13, 1, 0);
         }
         launch_narrow(s, false, B, T, c->d_keys.p, sc + 0, np, c->d_slot_entity.p, c->d_member_first.p,
                       c->d_members.p, c->d_narrow_counts.p, nullptr, contacts_view(c), sc + 4, trees,
                       sc + 13);
         exclusive_scan(s, c->d_narrow_counts.p, c->d_narrow_offsets.p, np, sc + 1, c->d_scan_temp.p);
         AM_HIP(c, hipGetLastError());
-        r = read_scalars(c, 1, 1);
+        r = read_scalars(c, 1, 4);
         if (r) return r;
         int nc = c->h_scalars[1];
+        if ((r = detect_flags(c))) return r;
         r = ensure_contact_capacity(c, nc);
         if (r) return r;
         c->n_contacts = nc;
@@ -636,13 +647,11 @@ int do_detect(am_ctx* c) {
     } else {
         c->n_contacts = 0;
         fill_int(s, sc + 1, 1, 0);
+        if ((r = read_scalars(c, 4, 1)) || (r = detect_flags(c))) return r;
     }
-    r = read_scalars(c, 4, 1);
-    if (r) return r;
-    if (c->h_scalars[4] & 2) return fail(c, AM_ERR_CAPACITY, "sphere-tree traversal stack overflow (tree too deep)");
-    if (c->h_scalars[4] & 1) return fail(c, AM_ERR_CAPACITY, "contact or pair buffer overflow");
     if (c->n_contacts == 0) c->n_old = 0;  // CollisionProcessor.java:99-101
-    return groups_after_contacts(c);
+    if ((r = groups_after_contacts(c))) return r;
+    return np > 0 && c->n_contacts > 0 ? detect_flags(c) : AM_OK;  // of the pass that wrote the contacts
 }
 
 // ---- learned warm start helpers ------------------------------------------
@@ -766,7 +775,7 @@ int start_residual(am_ctx* c, PgsArgs G, double* out) {
     AM_HIP(c, hipMemcpyAsync(c->d_dv.p, c->dv_save.p, (size_t)c->n_ent * 48, hipMemcpyDeviceToDevice, s));
     G.iterations = 0;
     G.warm_start = 1;
-    fill_int(s, c->d_barrier.p, 2, 0);
+    fill_int(s, c->d_barrier.p, 1, 0);
     // the warm-start pass alone, by the coloured kernel at its automatic
     // shape (its bits do not depend on the shape)
     am_params pc = c->params;
@@ -868,7 +877,8 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
     S.iters_used = nullptr;
     S.scene_used = nullptr;
     const bool flow = P.pgs_schedule == 0;
-    fill_int(s, c->d_scalars.p + 1, 1, c->n_contacts);
+    MemBatch m(s);
+    m.fill_int(c->d_scalars.p + 1, 1, c->n_contacts);
     for (auto& e : c->kev)
         if (!e) AM_HIP(c, hipEventCreate(&e));
     for (auto& e : c->lev)
@@ -881,14 +891,16 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
     c->ms_learned = 0;
     AM_HIP(c, hipEventRecord(c->lev[0], s));
     if (learned || collect) {
+        m.run();
         r = compute_features(c, dt);
         if (r) return r;
     }
     AM_HIP(c, hipEventRecord(c->kev[0], s));
-    launch_setup(s, S, c->n_contacts);
     const int iterations = main_solve ? P.iterations : P.iterations_in_collection;
-    AM_HIP(c, c->s_iter_max.ensure(std::max(iterations, 1)));
-    fill_int(s, (int*)c->s_iter_max.p, 2 * std::max(iterations, 1), 0);
+    // what the host reads back at the end lies together: sweeps used and the
+    // error flag, then every sweep's max
+    AM_HIP(c, c->s_iter_max.ensure((size_t)iterations + 1));
+    m.fill_u64(c->s_iter_max.p, (size_t)iterations + 1, 0);
     PgsArgs G;
     G.colour_start = c->s_colour_start.p;
     G.group_desc = c->s_group_desc.p;
@@ -906,12 +918,12 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
     G.omega = P.omega;
     G.sliding = P.sliding_threshold;
     G.compliance = S.compliance;
-    AM_HIP(c, c->d_barrier.ensure(2));
-    fill_int(s, c->d_barrier.p, 2, 0);
+    AM_HIP(c, c->d_barrier.ensure(1));
+    m.fill_int(c->d_barrier.p, 1, 0);
     G.barrier = (unsigned*)c->d_barrier.p;
-    G.error = c->d_barrier.p + 1;
-    G.iter_max = c->s_iter_max.p;
-    G.iters_used = c->d_scalars.p + 6;
+    G.iters_used = (int*)c->s_iter_max.p;
+    G.error = (int*)c->s_iter_max.p + 1;
+    G.iter_max = c->s_iter_max.p + 1;
     // several scenes in one context stop one by one, as each would alone
     G.per_scene = main_solve && c->n_scenes > 1 && P.tolerance > 0 ? 1 : 0;
     G.n_scenes = c->n_scenes;
@@ -928,9 +940,10 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         AM_HIP(c, c->scene_groups.ensure(ns));
         AM_HIP(c, c->scene_max.ensure(ns * iterations));
         AM_HIP(c, c->scene_done.ensure(ns * (iterations + 1)));
-        fill_int(s, (int*)c->scene_groups.p, (int)ns, 0);
-        fill_int(s, (int*)c->scene_max.p, (int)(2 * ns * iterations), 0);
-        fill_int(s, (int*)c->scene_done.p, (int)(2 * ns * (iterations + 1)), 0);
+        m.fill_int((int*)c->scene_groups.p, ns, 0);
+        m.fill_u64(c->scene_max.p, ns * iterations, 0);
+        m.fill_u64(c->scene_done.p, ns * (iterations + 1), 0);
+        m.run();
         launch_group_scene(s, c->s_group_desc.p, c->n_groups, c->s_order.p, c->c_b1.p, c->d_desc.p, c->n_scenes,
                            c->g_scene.p, c->scene_groups.p);
         G.g_scene = c->g_scene.p;
@@ -946,6 +959,27 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         c->last_grid = grid;
         c->last_block = block;
     }
+    const size_t n_dv = (size_t)c->n_ent * 6;
+    auto prepare_flow = [&]() -> int {
+        AM_HIP(c, c->s_start.ensure((size_t)std::max(c->n_contacts, 1) * 3));
+        m.copy(c->s_start.p, c->c_lam.p, (size_t)c->n_contacts * 24);
+        if (!flow) return AM_OK;
+        AM_HIP(c, c->s_lam_alt.ensure((size_t)c->n_contacts * 4));
+        AM_HIP(c, c->dv_alt.ensure(std::max(n_dv, (size_t)6)));
+        const size_t n_slot = (size_t)2 * 2 * std::max(c->n_groups, 1) * kSlotDoubles;
+        AM_HIP(c, c->f_slot.ensure(n_slot));
+        const size_t n_pass = block == kResidentThreads ? ((size_t)(iterations + 1) * kPassWords + 1) * kPassStride
+                                                        : (size_t)(iterations + 2) * kPassWords;
+        AM_HIP(c, c->d_pass_done.ensure(n_pass));
+        m.fill_u64(c->f_slot.p, n_slot, kSlotEmpty);
+        m.fill_u64(c->d_pass_done.p, n_pass, 0);
+        m.copy(c->dv_alt.p, c->d_dv.p, n_dv * sizeof(double));
+        return AM_OK;
+    };
+    // a learned start may still change the lambdas
+    if (!learned && (r = prepare_flow())) return r;
+    m.run();
+    launch_setup(s, S, c->n_contacts);
     if (learned) {
         // plain start residual, predicted start residual; keep the better
         AM_HIP(c, c->dv_save.ensure((size_t)c->n_ent * 6));
@@ -965,23 +999,14 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         } else {
             launch_rec_lambda(s, c->s_rec.p, c->s_order.p, c->c_lam.p, c->n_contacts);
         }
-        fill_int(s, c->d_barrier.p, 2, 0);
+        fill_int(s, c->d_barrier.p, 1, 0);
     }
     AM_HIP(c, hipEventRecord(c->lev[1], s));
-    AM_HIP(c, c->s_start.ensure((size_t)std::max(c->n_contacts, 1) * 3));
-    AM_HIP(c, hipMemcpyAsync(c->s_start.p, c->c_lam.p, (size_t)c->n_contacts * 24, hipMemcpyDeviceToDevice, s));
+    if (learned) {
+        if ((r = prepare_flow())) return r;
+        m.run();
+    }
     if (flow) {
-        const size_t n_dv = (size_t)c->n_ent * 6;
-        AM_HIP(c, c->s_lam_alt.ensure((size_t)c->n_contacts * 4));
-        AM_HIP(c, c->dv_alt.ensure(std::max(n_dv, (size_t)6)));
-        const size_t n_slot = (size_t)2 * 2 * std::max(c->n_groups, 1) * kSlotDoubles;
-        AM_HIP(c, c->f_slot.ensure(n_slot));
-        const size_t n_pass = block == kResidentThreads ? ((size_t)(iterations + 1) * kPassWords + 1) * kPassStride
-                                                        : (size_t)(iterations + 2) * kPassWords;
-        AM_HIP(c, c->d_pass_done.ensure(n_pass));
-        fill_u64(s, c->f_slot.p, n_slot, kSlotEmpty);
-        fill_u64(s, c->d_pass_done.p, n_pass, 0);
-        AM_HIP(c, hipMemcpyAsync(c->dv_alt.p, c->d_dv.p, n_dv * sizeof(double), hipMemcpyDeviceToDevice, s));
         const int fgrid = grid;
         FlowArgs F;
         F.P = G;
@@ -997,28 +1022,31 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         S.lam_alt = c->s_lam_alt.p;
         S.iters_used = G.iters_used;
         AM_HIP(c, hipEventRecord(c->kev[1], s));
-        AM_HIP(c, launch_pgs_flow(s, F, fgrid, block, P.pgs_plain_launch != 0, (int)n_dv, bodies_view(c)));
+        AM_HIP(c, launch_pgs_flow(s, F, fgrid, block, P.pgs_plain_launch != 0));
         AM_HIP(c, hipEventRecord(c->kev[2], s));
+        launch_flow_end(s, F, S, c->n_contacts, (int)n_dv);
     } else {
         AM_HIP(c, hipEventRecord(c->kev[1], s));
         AM_HIP(c, launch_pgs(s, G, grid, block, P.pgs_plain_launch != 0));
         AM_HIP(c, hipEventRecord(c->kev[2], s));
         launch_scene_finish(s, G);
+        launch_unpack(s, S, c->n_contacts);
     }
     if (G.per_scene) {
         c->scene_solve_valid = true;
         c->scene_iters = iterations;
     }
-    launch_unpack(s, S, c->n_contacts);
     AM_HIP(c, hipGetLastError());
-    r = read_scalars(c, 6, 1);
-    if (r) return r;
+    const size_t n_back = (size_t)std::min(iterations, kSweepsRead) + 1;
+    if (!c->h_sweeps)
+        AM_HIP(c, hipHostMalloc((void**)&c->h_sweeps, (kSweepsRead + 1) * sizeof(unsigned long long)));
+    AM_HIP(c, hipMemcpyAsync(c->h_sweeps, c->s_iter_max.p, n_back * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    AM_HIP(c, hipStreamSynchronize(s));
+    const int used = (int)(unsigned)c->h_sweeps[0], berr = (int)(c->h_sweeps[0] >> 32);
     {
         float lms = 0;
         (void)hipEventElapsedTime(&lms, c->lev[0], c->lev[1]);
         c->ms_learned = learned ? lms : 0.0;
-        int berr = 0;
-        AM_HIP(c, hipMemcpy(&berr, c->d_barrier.p + 1, sizeof(int), hipMemcpyDeviceToHost));
         if (berr)
             return fail(c, AM_ERR_HIP, flow ? "PGS dataflow kernel stopped making progress (workgroups not co-resident?)"
                                             : "PGS grid barrier did not complete (blocks not co-resident)");
@@ -1028,10 +1056,13 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         (void)hipEventElapsedTime(&ms, c->kev[0], c->kev[1]);
         c->ms_setup_kernel = ms;
     }
-    int used = c->h_scalars[6];
-    std::vector<unsigned long long> im(std::max(used, 1));
-    if (used > 0)
-        AM_HIP(c, hipMemcpy(im.data(), c->s_iter_max.p, used * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    std::vector<unsigned long long> more;  // past kSweepsRead sweeps
+    const unsigned long long* im = c->h_sweeps + 1;
+    if (used > kSweepsRead) {
+        more.resize(used);
+        AM_HIP(c, hipMemcpy(more.data(), c->s_iter_max.p + 1, (size_t)used * 8, hipMemcpyDeviceToHost));
+        im = more.data();
+    }
     double lc = 0;
     for (int i = 0; i < used; i++) {
         double m;
@@ -1598,19 +1629,19 @@ int am_update_contacts_map(am_ctx* c) {
     r = ensure_old_capacity(c, n);
     if (r) return r;
     hipStream_t s = c->stream;
-    if (n > 0) {
-        AM_HIP(c, hipMemcpyAsync(c->o_b1.p, c->c_b1.p, n * 4, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_b2.p, c->c_b2.p, n * 4, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_bv1.p, c->c_bv1.p, n * 4, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_bv2.p, c->c_bv2.p, n * 4, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_info.p, c->c_info.p, n * 4, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_pB1.p, c->c_pB1.p, (size_t)n * 24, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_lam.p, c->c_lam.p, (size_t)n * 24, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_viol.p, c->c_viol.p, (size_t)n * 8, hipMemcpyDeviceToDevice, s));
-        AM_HIP(c, hipMemcpyAsync(c->o_prev.p, c->c_prev.p, (size_t)n * 8, hipMemcpyDeviceToDevice, s));
-    }
+    MemBatch m(s);
+    m.copy(c->o_b1.p, c->c_b1.p, (size_t)n * 4);
+    m.copy(c->o_b2.p, c->c_b2.p, (size_t)n * 4);
+    m.copy(c->o_bv1.p, c->c_bv1.p, (size_t)n * 4);
+    m.copy(c->o_bv2.p, c->c_bv2.p, (size_t)n * 4);
+    m.copy(c->o_info.p, c->c_info.p, (size_t)n * 4);
+    m.copy(c->o_pB1.p, c->c_pB1.p, (size_t)n * 24);
+    m.copy(c->o_lam.p, c->c_lam.p, (size_t)n * 24);
+    m.copy(c->o_viol.p, c->c_viol.p, (size_t)n * 8);
+    m.copy(c->o_prev.p, c->c_prev.p, (size_t)n * 8);
+    m.fill_int(c->o_table.p, c->table_mask + 1, -1);
+    m.run();
     c->n_old = n;
-    fill_int(s, c->o_table.p, c->table_mask + 1, -1);
     launch_map_insert(s, old_view(c), c->o_table.p);
     AM_HIP(c, hipGetLastError());
     return AM_OK;
@@ -1738,9 +1769,11 @@ int am_lambdas_push(am_ctx* c, const double* lambda, int32_t n) {
 int am_warm_start(am_ctx* c, int32_t post, int32_t* bad, int32_t* repaired) {
     int r = check_ctx(c);
     if (r) return r;
-    fill_int(c->stream, c->d_scalars.p + 7, 2, 0);
+    MemBatch m(c->stream);
+    m.fill_int(c->d_scalars.p + 7, 2, 0);
+    if (c->n_contacts > 0) m.fill_int(c->d_scalars.p + 2, 1, c->n_groups);
+    m.run();
     if (c->n_contacts > 0) {
-        fill_int(c->stream, c->d_scalars.p + 2, 1, c->n_groups);
         launch_warm_start(c->stream, bodies_view(c), contacts_view(c), old_view(c), c->d_scalars.p + 2, c->n_groups,
                           c->g_start.p, post, c->d_scalars.p + 7);
         AM_HIP(c, hipGetLastError());

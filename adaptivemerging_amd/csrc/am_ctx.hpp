@@ -113,6 +113,12 @@ struct ContactStore {
 
 }  // namespace am_rt
 
+namespace am_rt {
+// Words of the pinned mirror: the scalars, then the layout's colour starts, plan and flag
+constexpr int kHostLayout = 32, kHostInts = kHostLayout + am::kMaxColours + 5;
+constexpr int kSweepsRead = 4096;  // a solve's sweeps read back with its result
+}  // namespace am_rt
+
 struct am_ctx {
     template <class T>
     using DBuf = am_rt::DBuf<T>;
@@ -210,6 +216,7 @@ struct am_ctx {
     // 6 iters_used, 7 bad, 8 repaired, 9 n_sweep
     DBuf<int> d_scalars;
     int* h_scalars = nullptr;  // pinned mirror
+    unsigned long long* h_sweeps = nullptr;  // pinned: sweeps used, error flag, the sweeps' max |dl| (kSweepsRead + 1)
 
     int n_pairs = 0, n_contacts = 0, n_groups = 0, n_colours = 0, max_colour_groups = 0;
     bool layout_valid = false;

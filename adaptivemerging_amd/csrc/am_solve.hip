@@ -40,54 +40,142 @@ void fill_u64(hipStream_t s, void* p, size_t n, unsigned long long v) {
                            v);
 }
 
+constexpr unsigned kMemWords = 1024;  // of a workgroup: 16 bytes a thread
+__global__ __launch_bounds__(256) void k_mem_batch(MemBatch::Jobs J) {
+    int k = 0;
+    unsigned first = 0;
+    while (blockIdx.x >= J.job[k].end) first = J.job[k++].end;
+    const MemBatch::Job& j = J.job[k];
+    const size_t w0 = (size_t)(blockIdx.x - first) * kMemWords + 4 * threadIdx.x;
+    unsigned* dst = (unsigned*)j.dst;
+    const unsigned* src = (const unsigned*)j.src;
+    const unsigned lo = (unsigned)j.value, hi = (unsigned)(j.value >> 32);
+    if (w0 + 4 <= j.words && (((uintptr_t)dst | (uintptr_t)src) & 15) == 0) {
+        *(uint4*)(dst + w0) = src ? *(const uint4*)(src + w0) : make_uint4(lo, hi, lo, hi);
+        return;
+    }
+    for (size_t w = w0; w < w0 + 4 && w < j.words; w++) dst[w] = src ? src[w] : (w & 1) ? hi : lo;
+}
+void MemBatch::add(void* dst, const void* src, unsigned long long v, size_t words) {
+    if (words == 0) return;
+    if (j_.n == kMax) run();
+    const unsigned first = j_.n ? j_.job[j_.n - 1].end : 0;
+    j_.job[j_.n++] = Job{dst, src, v, words, first + (unsigned)((words + kMemWords - 1) / kMemWords)};
+}
+void MemBatch::run() {
+    if (j_.n) hipLaunchKernelGGL(k_mem_batch, dim3(j_.job[j_.n - 1].end), dim3(256), 0, s_, j_);
+    j_.n = 0;
+}
+
 // ---------------------------------------------------------------------------
 // Groups: runs of contacts with the same unordered slot pair (solve bodies are
 // the top-level entities), or with the same unordered physical body pair when
 // slot and parent are null (the single sweep inside collections).
-__global__ void k_group_flags(int cap, const int* n_contacts, const int* cb1, const int* cb2, const int* slot,
-                              int* flags) {
+// slot == nullptr: physical body pairs (computeInCollection)
+AMD_INLINE int starts_group(int k, const int* cb1, const int* cb2, const int* slot) {
+    if (k == 0) return 1;
+    const int a = slot ? slot[cb1[k]] : cb1[k], b = slot ? slot[cb2[k]] : cb2[k];
+    const int pa = slot ? slot[cb1[k - 1]] : cb1[k - 1], pb = slot ? slot[cb2[k - 1]] : cb2[k - 1];
+    return min(a, b) != min(pa, pb) || max(a, b) != max(pa, pb) ? 1 : 0;
+}
+struct GroupArgs {
+    int cap;
+    const int *n_contacts, *cb1, *cb2, *slot, *parent;
+    int *flags, *scanned, *group_start, *group_a, *group_b, *d_n_groups;
+};
+AMD_INLINE void begin_group(const GroupArgs& A, int g, int k) {
+    A.group_start[g] = k;
+    const int a = A.cb1[k], b = A.cb2[k];
+    if (A.group_a) A.group_a[g] = (A.parent && A.parent[a] >= 0) ? A.parent[a] : a;
+    if (A.group_b) A.group_b[g] = (A.parent && A.parent[b] >= 0) ? A.parent[b] : b;
+}
+__global__ void k_group_flags(GroupArgs A) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = *n_contacts;
-    if (k >= cap) return;
-    if (k >= n) {
-        flags[k] = 0;
-        return;
-    }
-    int f = 1;
-    if (k > 0) {
-        // slot == nullptr: physical body pairs (computeInCollection)
-        int a = slot ? slot[cb1[k]] : cb1[k], b = slot ? slot[cb2[k]] : cb2[k];
-        int pa = slot ? slot[cb1[k - 1]] : cb1[k - 1], pb = slot ? slot[cb2[k - 1]] : cb2[k - 1];
-        int lo = min(a, b), hi = max(a, b), plo = min(pa, pb), phi = max(pa, pb);
-        f = (lo != plo || hi != phi) ? 1 : 0;
-    }
-    flags[k] = f;
+    if (k < A.cap) A.flags[k] = k < *A.n_contacts ? starts_group(k, A.cb1, A.cb2, A.slot) : 0;
 }
 
-__global__ void k_group_build(const int* n_contacts, const int* flags, const int* scanned, const int* cb1,
-                              const int* cb2, const int* parent, int* group_start, int* group_a, int* group_b) {
+__global__ void k_group_build(GroupArgs A) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
-    int n = *n_contacts;
+    int n = *A.n_contacts;
     if (k >= n) return;
-    if (flags[k]) {
-        int g = scanned[k];
-        group_start[g] = k;
-        int a = cb1[k], b = cb2[k];
-        if (group_a) group_a[g] = (parent && parent[a] >= 0) ? parent[a] : a;
-        if (group_b) group_b[g] = (parent && parent[b] >= 0) ? parent[b] : b;
+    if (A.flags[k]) begin_group(A, A.scanned[k], k);
+    if (k == n - 1) A.group_start[A.scanned[k] + A.flags[k]] = n;
+}
+// All of it by one workgroup, 4,096 contacts at a time (8 us each): one launch for three
+// that take 10 us for 5,000 contacts and cost the host 5 each.
+constexpr int kGroupsAtOnce = 8192;
+__global__ __launch_bounds__(1024) void k_groups_small(GroupArgs A) {
+    constexpr int kItems = 4;
+    __shared__ int wave_sum[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = min(*A.n_contacts, A.cap);
+    if (n <= 0) {
+        for (int k = threadIdx.x; k < A.cap; k += blockDim.x) A.flags[k] = 0, A.scanned[k] = 0;
+        if (threadIdx.x == 0) *A.d_n_groups = 0;
+        return;
     }
-    if (k == n - 1) group_start[scanned[k] + flags[k]] = n;
+    int before = 0;  // groups of the contacts before this turn's
+    for (int k0 = 0; k0 < A.cap; k0 += 1024 * kItems) {
+        const int k = k0 + threadIdx.x * kItems;
+        // the pairs of the contacts from k - 1 on, loaded without a branch between them
+        int a[kItems + 1], b[kItems + 1], f[kItems], sum = 0;
+#pragma unroll
+        for (int u = 0; u <= kItems; u++) {
+            const int i = max(0, min(k + u - 1, n - 1));
+            a[u] = A.cb1[i];
+            b[u] = A.cb2[i];
+        }
+        if (A.slot)
+#pragma unroll
+            for (int u = 0; u <= kItems; u++) {
+                a[u] = A.slot[a[u]];
+                b[u] = A.slot[b[u]];
+            }
+#pragma unroll
+        for (int u = 0; u < kItems; u++) {
+            const bool same = min(a[u], b[u]) == min(a[u + 1], b[u + 1]) && max(a[u], b[u]) == max(a[u + 1], b[u + 1]);
+            f[u] = k + u < n && (k + u == 0 || !same) ? 1 : 0;
+            sum += f[u];
+        }
+        int inc = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
+        }
+        if (lane == 63) wave_sum[wave] = inc;
+        __syncthreads();
+        int at = before + inc - sum;
+        for (int v = 0; v < 16; v++) {
+            at += v < wave ? wave_sum[v] : 0;
+            before += wave_sum[v];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kItems; u++) {
+            if (k + u >= A.cap) break;
+            A.flags[k + u] = f[u];
+            A.scanned[k + u] = at;
+            if (f[u]) begin_group(A, at, k + u);
+            at += f[u];
+            if (k + u == n - 1) A.group_start[at] = n;
+        }
+    }
+    if (threadIdx.x == 0) *A.d_n_groups = before;
 }
 
 void launch_groups(hipStream_t s, int cap, const int* n_contacts, const int* cb1, const int* cb2, const int* slot,
                    const int* parent, int* flags, int* scanned, int* group_start, int* group_a, int* group_b,
                    int* d_n_groups, void* scan_temp) {
     if (cap <= 0) return;
+    const GroupArgs A{cap, n_contacts, cb1, cb2, slot, parent, flags, scanned, group_start, group_a, group_b, d_n_groups};
+    if (cap <= kGroupsAtOnce) {
+        hipLaunchKernelGGL(k_groups_small, dim3(1), dim3(1024), 0, s, A);
+        return;
+    }
     dim3 g((cap + 255) / 256), b(256);
-    hipLaunchKernelGGL(k_group_flags, g, b, 0, s, cap, n_contacts, cb1, cb2, slot, flags);
+    hipLaunchKernelGGL(k_group_flags, g, b, 0, s, A);
     exclusive_scan(s, flags, scanned, cap, d_n_groups, scan_temp);
-    hipLaunchKernelGGL(k_group_build, g, b, 0, s, n_contacts, flags, scanned, cb1, cb2, parent, group_start, group_a,
-                       group_b);
+    hipLaunchKernelGGL(k_group_build, g, b, 0, s, A);
 }
 
 // ---------------------------------------------------------------------------
@@ -625,13 +713,11 @@ void launch_setup(hipStream_t s, const SetupArgs& S, int cap) {
 }
 
 // Results back to list order.
-__global__ void k_unpack(SetupArgs S) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= *S.n_contacts) return;
+AMD_INLINE void unpack(const SetupArgs& S, int k, int iters_used) {
     int c = S.order[k];
     double* rec = &S.rec[(size_t)k * kRecDoubles];
     ContactsView C = S.C;
-    const int used = S.scene_used ? S.scene_used[S.B.desc[S.C.b1[c]].scene] : *S.iters_used;
+    const int used = S.scene_used ? S.scene_used[S.B.desc[S.C.b1[c]].scene] : iters_used;
     if (S.lam_alt && (used & 1)) {
         // dataflow schedule: an odd last sweep left lambda in the odd-sweep buffer
 #pragma unroll
@@ -644,6 +730,10 @@ __global__ void k_unpack(SetupArgs S) {
         C.D[c * 3 + r] = rec[r * kRecRow + kRecD];
     }
     C.state[c] = S.sstate[k];
+}
+__global__ void k_unpack(SetupArgs S) {
+    int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < *S.n_contacts) unpack(S, k, S.lam_alt ? *S.iters_used : 0);
 }
 
 void launch_unpack(hipStream_t s, const SetupArgs& S, int cap) {
@@ -2850,25 +2940,43 @@ int pgs_resident_max_blocks(bool* ok) {
     return n_cu * std::min(a, b);
 }
 
-// Sweeps used (the first converged sweep, else all), then the buffers of the
-// last pass become the results.
-__global__ void k_flow_finish(PgsArgs P) {
+// Sweeps used: the first converged sweep, else all (threads that fall below it find nothing)
+AMD_INLINE int first_converged(const PgsArgs& P) {
     int used = P.iterations;
     if (P.check_tolerance)
-        for (int t = 1 + (int)threadIdx.x; t <= P.iterations; t += 64)
+        for (int t = 1 + (int)threadIdx.x; t <= P.iterations; t += blockDim.x)
             if (__longlong_as_double((long long)P.iter_max[t - 1]) < P.tolerance) {
                 used = t;
                 break;
             }
     for (int o = 32; o > 0; o >>= 1) used = min(used, __shfl_xor(used, o, 64));
+    return used;
+}
+__global__ void k_flow_finish(PgsArgs P) {
+    const int used = first_converged(P);
     if (threadIdx.x == 0) *P.iters_used = used;
 }
-__global__ void k_flow_select_dv(double* dv, const double* dv_alt, int n, const int* iters_used,
-                                 const int* scene_used, const am_body_desc* desc) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int used = scene_used ? scene_used[desc[i / 6].scene] : *iters_used;
-    if (used & 1) dv[i] = dv_alt[i];
+// The buffers of the last pass become the results.  With find, every workgroup
+// looks the sweeps up by itself (up to kFindSweeps of them), which saves a launch.
+constexpr int kFindSweeps = 4096;
+__global__ __launch_bounds__(256) void k_flow_end(FlowArgs F, SetupArgs S, int n_dv, int cap, int find) {
+    __shared__ int wave_used[4];
+    int used;
+    if (find) {
+        used = first_converged(F.P);
+        if ((threadIdx.x & 63) == 0) wave_used[threadIdx.x >> 6] = used;
+        __syncthreads();
+        used = min(min(wave_used[0], wave_used[1]), min(wave_used[2], wave_used[3]));
+        if (blockIdx.x == 0 && threadIdx.x == 0) *F.P.iters_used = used;
+    } else {
+        used = *F.P.iters_used;
+    }
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_dv) {
+        const int u = S.scene_used ? S.scene_used[S.B.desc[i / 6].scene] : used;
+        if (u & 1) F.P.dv[i] = F.dv_alt[i];
+    }
+    if (i < cap) unpack(S, i, used);
 }
 
 // Sweeps used per scene: the first sweep whose max |dl| over the scene was
@@ -2931,8 +3039,7 @@ int pgs_flow_max_blocks(bool* ok) {
     return n_cu * (per_cu > 0 ? per_cu : 1);
 }
 
-hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain, int n_dv,
-                           const BodiesView& B) {
+hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain) {
     const bool resident = block != 64;
     void (*kernel)(FlowArgs) = resident ? (F.P.per_scene ? k_pgs_resident<true> : k_pgs_resident<false>)
                                         : (F.P.per_scene ? k_pgs_flow<true> : k_pgs_flow<false>);
@@ -2943,12 +3050,14 @@ hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block
         hipError_t e = hipLaunchCooperativeKernel((const void*)kernel, dim3(grid), dim3(block), args, 0, s);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_flow_finish, dim3(1), dim3(64), 0, s, F.P);
-    launch_scene_finish(s, F.P);
-    if (n_dv > 0)
-        hipLaunchKernelGGL(k_flow_select_dv, dim3((n_dv + 255) / 256), dim3(256), 0, s, F.P.dv, F.dv_alt, n_dv,
-                           F.P.iters_used, F.P.per_scene ? F.P.scene_used : nullptr, B.desc);
     return hipGetLastError();
+}
+void launch_flow_end(hipStream_t s, const FlowArgs& F, const SetupArgs& S, int cap, int n_dv) {
+    const bool find = F.P.iterations <= kFindSweeps;
+    if (!find) hipLaunchKernelGGL(k_flow_finish, dim3(1), dim3(64), 0, s, F.P);
+    launch_scene_finish(s, F.P);
+    hipLaunchKernelGGL(k_flow_end, dim3((std::max(cap, n_dv) + 255) / 256), dim3(256), 0, s, F, S, n_dv, cap,
+                       find ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------

@@ -106,6 +106,35 @@ struct FlowArgs {
 void fill_int(hipStream_t s, int* p, int n, int v);
 void fill_double(hipStream_t s, double* p, int n, double v);
 void fill_u64(hipStream_t s, void* p, size_t n, unsigned long long v);
+
+// Fills and device copies that do not depend on each other, up to 12 to a
+// launch: a launch costs the host about 5 us, more than any of them takes at
+// the sizes of most scenes.  Sizes are multiples of 4 bytes.
+class MemBatch {
+public:
+    static constexpr int kMax = 12;
+    struct Job {
+        void* dst;
+        const void* src;  // null: fill
+        unsigned long long value;
+        size_t words;  // of 4 bytes
+        unsigned end;  // first workgroup past it
+    };
+    struct Jobs {
+        Job job[kMax];
+        int n;
+    };
+    explicit MemBatch(hipStream_t s) : s_(s) { j_.n = 0; }
+    void fill_int(int* p, size_t n, int v) { add(p, nullptr, (unsigned)v | (unsigned long long)(unsigned)v << 32, n); }
+    void fill_u64(void* p, size_t n, unsigned long long v) { add(p, nullptr, v, 2 * n); }
+    void copy(void* dst, const void* src, size_t bytes) { add(dst, src, 0, bytes / 4); }
+    void run();
+
+private:
+    void add(void* dst, const void* src, unsigned long long v, size_t words);
+    hipStream_t s_;
+    Jobs j_;
+};
 void launch_groups(hipStream_t s, int cap, const int* n_contacts, const int* cb1, const int* cb2, const int* slot,
                    const int* parent, int* flags, int* scanned, int* group_start, int* group_a, int* group_b,
                    int* d_n_groups, void* scan_temp);
@@ -143,12 +172,14 @@ void launch_group_scene(hipStream_t s, const int* group_desc, int n_groups, cons
 // sweeps used per scene (first sweep under the tolerance, else all)
 void launch_scene_finish(hipStream_t s, const PgsArgs& P);
 void launch_unpack(hipStream_t s, const SetupArgs& S, int cap);
+// the sweeps used, then deltaV and the contacts from the last sweep's buffers
+struct FlowArgs;
+void launch_flow_end(hipStream_t s, const FlowArgs& F, const SetupArgs& S, int cap, int n_dv);
 int pgs_max_blocks(int block, bool* ok);
 hipError_t launch_pgs(hipStream_t s, const PgsArgs& P, int grid, int block, bool plain);
 int pgs_flow_max_blocks(bool* ok);
 // block 64: k_pgs_flow; kResidentThreads: the resident kernel
-hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain, int n_dv,
-                           const BodiesView& B);
+hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain);
 int pgs_resident_max_blocks(bool* ok);
 // what `waves` resident waves would hold: used[] LDS doubles of each, plan[0]
 // those of the fullest workgroup, plan[1] steps of the busiest wave
