@@ -1317,8 +1317,7 @@ AMD_INLINE void row_contact_fast(const FlowArgs& F, const WaveRec& c, int k, int
         } else {
             const double limit = c.mu * lam[0];
             chk.limit_hi_max = max(chk.limit_hi_max, hi_word(limit));
-            const double a = l < -limit ? -limit : l;
-            l = a > limit ? limit : a;
+            l = __builtin_fmin(__builtin_fmax(l, -limit), limit);
         }
         lam[r] = l;
         const double diff = l - prev;
@@ -1600,9 +1599,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
                 __hip_atomic_fetch_add(pend_done, pend_add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 pend_done = nullptr;
             }
-            // empty the slot read above only now, so that this wait does not
-            // include the store (the publish below waits for it)
-            if (src) st_coherent(src, __longlong_as_double((long long)kSlotEmpty));
             // rows with fewer contacts idle; contacts past the LDS slots
             // (groups of more than kDmaSlots contacts) read global memory
             double smx = 0.0;  // this step's max |dl| and NaN flag (row-uniform)
@@ -1683,18 +1679,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
             }
             mx = fmax(mx, smx);
             nan = nan || snan;
-            // Publish deltaV to this group's slots.  The emptied slot must be
-            // seen empty before these values can be seen (the chain of
-            // updates they start leads to that slot's next writer), so the
-            // stores wait for this wave's earlier memory operations; with the
-            // fast update's lambdas still in LDS, only that store is left.
-            // The body's last update of the pass also goes to the pass's
-            // buffer, which holds the result when this is the last sweep.
-            __builtin_amdgcn_s_waitcnt(0);
+            // Publish deltaV to this group's slots.  The body's last update of
+            // the pass also goes to the pass's buffer, which holds the result
+            // when this is the last sweep.
             if (active && mine && dyn) {
                 st_coherent(slot_at(F, p & 1, 2 * qg + (side_b ? 1 : 0)) + comp, dv);
                 if (rank == deg - 1) st_coherent(&cur[e * 6 + comp], dv);
             }
+            // The slot that was read is emptied behind the values that the next
+            // update waits for.  It must be seen empty before its next writer
+            // fills it; that writer comes after this group's own publish of the
+            // next pass (the body's updates are one chain), and the stores of
+            // this pass have landed by the wait after that pass's poll.
+            if (src) st_coherent(src, __longlong_as_double((long long)kSlotEmpty));
             if (!general && active && li < 3) {
                 const int nl = min(n, kDmaSlots);
                 for (int t = 0; t < nl; t++) {
