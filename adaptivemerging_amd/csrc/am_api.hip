@@ -82,6 +82,7 @@ OldContactsView old_view(am_ctx* c) {
     O.prev_viol = c->o_prev.p;
     O.table = c->o_table.p;
     O.table_mask = c->table_mask;
+    O.first = c->o_first.p;
     return O;
 }
 
@@ -1771,11 +1772,16 @@ int am_warm_start(am_ctx* c, int32_t post, int32_t* bad, int32_t* repaired) {
     if (r) return r;
     MemBatch m(c->stream);
     m.fill_int(c->d_scalars.p + 7, 2, 0);
-    if (c->n_contacts > 0) m.fill_int(c->d_scalars.p + 2, 1, c->n_groups);
+    if (c->n_contacts > 0) {
+        AM_HIP(c, c->o_first.ensure(std::max(c->n_old, 1)));
+        AM_HIP(c, c->w_match.ensure(2 * (size_t)c->n_contacts));
+        m.fill_int(c->d_scalars.p + 2, 1, c->n_groups);
+        m.fill_int(c->o_first.p, c->n_old, 0x7fffffff);
+    }
     m.run();
     if (c->n_contacts > 0) {
-        launch_warm_start(c->stream, bodies_view(c), contacts_view(c), old_view(c), c->d_scalars.p + 2, c->n_groups,
-                          c->g_start.p, post, c->d_scalars.p + 7);
+        launch_warm_start(c->stream, bodies_view(c), contacts_view(c), old_view(c), c->n_contacts, post, c->w_match.p,
+                          c->d_scalars.p + 7);
         AM_HIP(c, hipGetLastError());
     }
     r = read_scalars(c, 7, 2);

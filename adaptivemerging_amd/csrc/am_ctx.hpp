@@ -168,6 +168,7 @@ struct am_ctx {
     // old contacts (warm start)
     int n_old = 0, table_mask = 0;
     DBuf<int> o_b1, o_b2, o_bv1, o_bv2, o_info, o_table;
+    DBuf<int> o_first, w_match;  // warm start: the first taker of each old contact; what each contact takes
     DBuf<double> o_pB1, o_lam, o_viol, o_prev;
 
     // groups, colouring, solve layout

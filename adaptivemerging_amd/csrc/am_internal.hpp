@@ -133,6 +133,7 @@ struct OldContactsView {
     const double* prev_viol;
     const int* table;   // open-addressing table of old indices, -1 empty
     int table_mask;
+    int* first;         // the first contact that takes and zeroes each
 };
 
 // Pair keys: slot_lo:20 | slot_hi:20 | sub_lo:12 | sub_hi:12.

@@ -189,8 +189,9 @@ void launch_flow_ranks(hipStream_t s, int n_groups, const int* bflags, const int
                        const int* inc_count, const int* inc_items, const int* spos, const int* group_desc,
                        int* flow, int* pred);
 void launch_map_insert(hipStream_t s, const OldContactsView& O, int* table);
-void launch_warm_start(hipStream_t s, BodiesView B, ContactsView C, OldContactsView O, const int* n_groups, int cap,
-                       const int* group_start, int post, int* counters);
+// O.first: one word for each old contact, INT_MAX before the call; match: 2 n words
+void launch_warm_start(hipStream_t s, BodiesView B, ContactsView C, OldContactsView O, int n, int post, int* match,
+                       int* counters);
 void launch_redo_warm(hipStream_t s, ContactsView C, const int* n, int cap, int zero);
 void launch_clear(hipStream_t s, BodiesView B);
 void launch_gravity(hipStream_t s, BodiesView B, const int* targets, int n, double gx, double gy, double gz);
