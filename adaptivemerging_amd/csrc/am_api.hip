@@ -317,10 +317,7 @@ int rebuild_structure(am_ctx* c, bool bodies_changed) {
     AM_HIP(c, c->d_bucket_start.ensure(tsize + 1));
     AM_HIP(c, c->d_bucket_cursor.ensure(tsize));
     AM_HIP(c, c->d_bucket_items.ensure(std::max(ng, 1)));
-    const int nt = pair_tasks(std::max(ng, 1));
-    AM_HIP(c, c->d_pair_counts.ensure((size_t)nt + 1));
-    AM_HIP(c, c->d_pair_offsets.ensure((size_t)nt + 1));
-    int r = ensure_scan_temp(c, std::max(tsize, nt) + 1);
+    int r = ensure_scan_temp(c, std::max(tsize, n + 1) + 1);
     if (r) return r;
     // incidence arrays are per entity
     AM_HIP(c, c->inc_count.ensure(n + 1));
@@ -579,6 +576,7 @@ int do_detect(am_ctx* c) {
     MemBatch m(s);
     m.fill_int(c->d_bucket_count.p, tsize, 0);
     m.fill_int(c->d_bucket_cursor.p, tsize, 0);
+    m.fill_int(sc + 0, 1, 0);
     m.fill_int(sc + 4, 1, 0);
     m.fill_int(sc + 13, 1, 0);
     m.run();
@@ -603,26 +601,31 @@ int do_detect(am_ctx* c) {
     A.top_sleeping = c->d_top_sleeping.p;
     A.large = c->d_grid_large.p;
     A.n_large = (int)c->grid_large.size();
-    launch_pairs_impl(s, false, A, c->d_pair_counts.p, nullptr, nullptr, 0, sc + 4);
-    exclusive_scan(s, c->d_pair_counts.p, c->d_pair_offsets.p, pair_tasks(ng), sc + 0, c->d_scan_temp.p);
-    AM_HIP(c, hipGetLastError());
-    int r = read_scalars(c, 0, 1);
+    auto pair_room = [&](size_t np) -> int {
+        if (c->d_keys.n >= np) return AM_OK;
+        const size_t cap = np + np / 4 + 64;
+        AM_HIP(c, c->d_keys.ensure(cap));
+        AM_HIP(c, c->d_keys_unsorted.ensure(cap));
+        AM_HIP(c, c->d_narrow_counts.ensure(cap + 1));
+        AM_HIP(c, c->d_narrow_offsets.ensure(cap + 1));
+        size_t st = sort_temp_bytes((int)cap);
+        if (st > c->d_sort_temp.n) AM_HIP(c, c->d_sort_temp.ensure(st));
+        return ensure_scan_temp(c, (int)cap + 1);
+    };
+    int r = pair_room(4 * (size_t)ng);  // a pile has about as many
     if (r) return r;
-    int np = ng > 0 ? c->h_scalars[0] : 0;
+    launch_pairs(s, A, c->d_keys_unsorted.p, (int)c->d_keys.n, sc + 0);
+    AM_HIP(c, hipGetLastError());
+    if ((r = read_scalars(c, 0, 1))) return r;
+    const int np = ng > 0 ? c->h_scalars[0] : 0;
+    if ((size_t)np > c->d_keys.n) {
+        if ((r = pair_room(np))) return r;
+        fill_int(s, sc + 0, 1, 0);
+        launch_pairs(s, A, c->d_keys_unsorted.p, (int)c->d_keys.n, sc + 0);
+        AM_HIP(c, hipGetLastError());
+    }
     c->n_pairs = np;
     if (np > 0) {
-        if ((int)c->d_keys.n < np) {
-            size_t cap = (size_t)np + np / 4 + 64;
-            AM_HIP(c, c->d_keys.ensure(cap));
-            AM_HIP(c, c->d_keys_unsorted.ensure(cap));
-            AM_HIP(c, c->d_narrow_counts.ensure(cap + 1));
-            AM_HIP(c, c->d_narrow_offsets.ensure(cap + 1));
-            size_t st = sort_temp_bytes((int)cap);
-            if (st > c->d_sort_temp.n) AM_HIP(c, c->d_sort_temp.ensure(st));
-            r = ensure_scan_temp(c, (int)cap + 1);
-            if (r) return r;
-        }
-        launch_pairs_impl(s, true, A, nullptr, c->d_pair_offsets.p, c->d_keys_unsorted.p, (int)c->d_keys.n, sc + 4);
         sort_u64(s, c->d_keys_unsorted.p, c->d_keys.p, np, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
         int* trees = nullptr;
         if (c->big_trees) {

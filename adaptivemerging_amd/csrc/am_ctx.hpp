@@ -153,7 +153,7 @@ struct am_ctx {
 
     // broad phase
     DBuf<double> d_sphere;
-    DBuf<int> d_cell, d_bucket_count, d_bucket_start, d_bucket_cursor, d_bucket_items, d_pair_counts, d_pair_offsets;
+    DBuf<int> d_cell, d_bucket_count, d_bucket_start, d_bucket_cursor, d_bucket_items;
     DBuf<uint64_t> d_keys_unsorted, d_keys;
     DBuf<unsigned char> d_sort_temp, d_scan_temp;
     size_t sort_temp_size = 0;

@@ -124,7 +124,11 @@ AMD_INLINE bool skip_pair(const PairArgs& A, int slot_a, int slot_b) {
     return false;
 }
 
-// One thread per (gridded body, task): count (write=false) or write pairs.
+// One thread per (gridded body, task) finds its pairs; the first kPairsKept of
+// them wait in LDS (a thread with more looks for the rest again) for the
+// workgroup's one addition to the pair count, which gives every thread its place.
+// *count is all pairs, also those past cap (none of them written): the caller
+// makes room and launches again.
 // Tasks 0-26 are the 27 cells around the body's own: the pairs with grid
 // bodies of a higher slot found there.  Task 27 holds the pairs with every
 // large body (those stay out of the grid, whose cells are sized for the
@@ -132,12 +136,20 @@ AMD_INLINE bool skip_pair(const PairArgs& A, int slot_a, int slot_b) {
 // pairs with large bodies of a higher slot and with the planes.  Spreading a
 // body's cells over threads keeps each thread's chain of dependent loads
 // short.  The keys are sorted afterwards, so the emission order is free.
-constexpr int kPairTasks = 28;
-template <bool kWrite>
-__global__ void k_pairs(PairArgs A, int* counts, const int* offsets, uint64_t* keys, int cap, int* overflow) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long)A.n_grid * kPairTasks) return;
-    const int k = (int)(t / kPairTasks), task = (int)(t % kPairTasks);
+//
+// What bounds it is the chain of loads behind a neighbour.  Counting the pairs
+// first, for a scan to give each thread its place, went through them twice: 34 us
+// each and 13 for the scan with 777 boxes, 330 each with 20,000; this takes 57 and
+// 510.  Additions to one word take about 0.1 us each, one after the other: with one
+// a wave, 20,000 boxes took 1,390 us.
+constexpr int kPairTasks = 28, kPairsKept = 12, kPairThreads = 512;
+__global__ __launch_bounds__(kPairThreads) void k_pairs(PairArgs A, uint64_t* keys, int cap, int* count) {
+    __shared__ uint64_t kept[kPairsKept][kPairThreads];
+    __shared__ int wave_sum[kPairThreads / 64], begin;
+    const long all = (long)A.n_grid * kPairTasks, t0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool valid = t0 < all;
+    const long t = valid ? t0 : all - 1;
+    const int k = (int)(t / kPairTasks), task = valid ? (int)(t % kPairTasks) : kPairTasks;
     const BodiesView& B = A.B;
     const int bi = A.grid_order[k];
     const int slot_i = B.slot[bi], sub_i = B.sub[bi];
@@ -145,15 +157,16 @@ __global__ void k_pairs(PairArgs A, int* counts, const int* offsets, uint64_t* k
     const double ci[4] = {A.sphere[k * 4 + 0], A.sphere[k * 4 + 1], A.sphere[k * 4 + 2], A.sphere[k * 4 + 3]};
     const bool large_i = A.cell[k * 4 + 3] < 0;
     int n = 0;
-    const int base = kWrite ? offsets[t] : 0;
+    int skip = 0, at = 0;  // the second time: pairs written from LDS, this thread's place
     auto emit = [&](int slot_j, int sub_j) {
-        if (kWrite) {
-            const int pos = base + n;
-            if (pos < cap) keys[pos] = pair_key(slot_i, sub_i, slot_j, sub_j);
-            else atomicOr(overflow, 1);
+        if (skip == 0) {
+            if (n < kPairsKept) kept[n][threadIdx.x] = pair_key(slot_i, sub_i, slot_j, sub_j);
+        } else if (n >= skip && at + n < cap) {
+            keys[at + n] = pair_key(slot_i, sub_i, slot_j, sub_j);
         }
         n++;
     };
+    auto search = [&]() {
     if (task < 27) {
         // a large body scans no cells: every grid body pairs with it in its task 27
         if (!large_i) {
@@ -180,7 +193,7 @@ __global__ void k_pairs(PairArgs A, int* counts, const int* offsets, uint64_t* k
                 emit(slot_j, B.sub[bj]);
             }
         }
-    } else {
+    } else if (task == 27) {
         for (int q = 0; q < A.n_large; q++) {
             const int kj = A.large[q];
             if (kj == k) continue;
@@ -216,18 +229,40 @@ __global__ void k_pairs(PairArgs A, int* counts, const int* offsets, uint64_t* k
             emit(slot_p, B.sub[p]);
         }
     }
-    if (!kWrite) counts[t] = n;
+    };
+    search();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int sum = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(sum, o, 64);
+        if (lane >= o) sum += v;
+    }
+    if (lane == 63) wave_sum[wave] = sum;
+    __syncthreads();
+    int first = sum - n, total = 0;
+    for (int w = 0; w < kPairThreads / 64; w++) {
+        first += w < wave ? wave_sum[w] : 0;
+        total += wave_sum[w];
+    }
+    if (threadIdx.x == 0 && total > 0) begin = atomicAdd(count, total);
+    __syncthreads();
+    if (total > 0) first += begin;
+    for (int i = 0; i < min(n, kPairsKept); i++)
+        if (first + i < cap) keys[first + i] = kept[i][threadIdx.x];
+    if (n > kPairsKept) {
+        skip = kPairsKept;
+        at = first;
+        n = 0;
+        search();
+    }
 }
 
-int pair_tasks(int n_grid) { return n_grid * kPairTasks; }
-
-void launch_pairs_impl(hipStream_t s, bool write, const PairArgs& A, int* counts, const int* offsets, uint64_t* keys,
-                       int cap, int* overflow) {
+void launch_pairs(hipStream_t s, const PairArgs& A, uint64_t* keys, int cap, int* count) {
     if (A.n_grid <= 0) return;
     const long n = (long)A.n_grid * kPairTasks;
-    dim3 g((unsigned)((n + 255) / 256)), b(256);
-    if (write) hipLaunchKernelGGL(k_pairs<true>, g, b, 0, s, A, counts, offsets, keys, cap, overflow);
-    else hipLaunchKernelGGL(k_pairs<false>, g, b, 0, s, A, counts, offsets, keys, cap, overflow);
+    hipLaunchKernelGGL(k_pairs, dim3((unsigned)((n + kPairThreads - 1) / kPairThreads)), dim3(kPairThreads), 0, s, A, keys,
+                       cap, count);
 }
 
 // ---------------------------------------------------------------------------

@@ -194,9 +194,8 @@ void launch_tree_world_centres(hipStream_t s, BodiesView B, TreeView T, const in
                                int n_nodes);
 void launch_bounds(hipStream_t s, BodiesView B, TreeView T, const int* order, int n, double* sphere,
                    double cell, int* cell_key, int hash_mask, const int* is_large);
-int pair_tasks(int n_grid);  // threads of the pair passes: one per (grid body, task)
-void launch_pairs_impl(hipStream_t s, bool write, const PairArgs& A, int* counts, const int* offsets, uint64_t* keys,
-                       int cap, int* overflow);
+// Adds the pairs to keys[*count ..], as far as cap; *count is all of them
+void launch_pairs(hipStream_t s, const PairArgs& A, uint64_t* keys, int cap, int* count);
 // trees, n_trees: room for every pair and a counter that starts at 0 where the
 // scene has trees of more than kWaveTree nodes, else null
 void launch_narrow(hipStream_t s, bool write, BodiesView B, TreeView T, const uint64_t* keys,

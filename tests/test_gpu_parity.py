@@ -44,6 +44,28 @@ def test_detect_sphere_trees(gpu_lib):
     assert_contacts_equal(ctx.contacts(), orc.contacts())
 
 
+@pytest.mark.parametrize("n", [1, 2, 13, 14, 65, 130])
+def test_detect_pairs_beyond_the_room_for_them(gpu_lib, n):
+    """n spheres all in one cell: every pair of them is one, more than the twelve a
+    thread keeps and than the four a body there is room for at first; twice, the
+    second time with the room made by the first."""
+    from adaptivemerging_amd.scene import Scene
+
+    rng = np.random.default_rng(n)
+    s = Scene()
+    s.add_plane([0, 0, 0], [0, 1, 0])
+    for _ in range(n):
+        s.add_sphere(0.5, rng.uniform(0.0, 0.3, 3) + [0, 0.3, 0])
+    ctx, orc = twin(s)
+    n_o = orc.detect()
+    for _ in range(2):
+        n_g = ctx.detect(0.01)
+        print("contacts", n_g, n_o, flush=True)
+        assert n_g == n_o and n_g >= n * (n - 1) // 2
+        assert_contacts_equal(ctx.contacts(), orc.contacts())
+    ctx.close()
+
+
 def _tree(rng, fanouts, radius=0.05, size=0.4):
     """A sphere tree with fanouts[k] children for every node of level k."""
     centres, radii, children = [], [], []
