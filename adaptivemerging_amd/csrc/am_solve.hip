@@ -182,11 +182,13 @@ void launch_groups(hipStream_t s, int cap, const int* n_contacts, const int* cb1
 // Colouring.
 AMD_INLINE bool dynamic_body(const int* flags, int e) { return (flags[e] & AM_BODY_PINNED) == 0; }
 
+// A body's list names a group once, also where both its solve bodies are that body
+// (contacts given between members of one collection): ranks count groups.
 __global__ void k_incidence_count(int n_groups, const int* ga, const int* gb, const int* bflags, int* inc_count) {
     int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= n_groups) return;
     if (dynamic_body(bflags, ga[g])) atomicAdd(&inc_count[ga[g]], 1);
-    if (dynamic_body(bflags, gb[g])) atomicAdd(&inc_count[gb[g]], 1);
+    if (gb[g] != ga[g] && dynamic_body(bflags, gb[g])) atomicAdd(&inc_count[gb[g]], 1);
 }
 __global__ void k_incidence_fill(int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
                                  int* inc_cursor, int* inc_items) {
@@ -194,7 +196,7 @@ __global__ void k_incidence_fill(int n_groups, const int* ga, const int* gb, con
     if (g >= n_groups) return;
     int a = ga[g], b = gb[g];
     if (dynamic_body(bflags, a)) inc_items[inc_start[a] + atomicAdd(&inc_cursor[a], 1)] = g;
-    if (dynamic_body(bflags, b)) inc_items[inc_start[b] + atomicAdd(&inc_cursor[b], 1)] = g;
+    if (b != a && dynamic_body(bflags, b)) inc_items[inc_start[b] + atomicAdd(&inc_cursor[b], 1)] = g;
 }
 
 AMD_INLINE uint32_t prio(uint32_t g) {
@@ -322,14 +324,14 @@ AMD_INLINE void st_u64(unsigned long long* p, unsigned long long v) {
 // that sees it (settled 20,000-box pile, 104,000 groups: 84 us; a launch per
 // round of the colouring, which went through the lists again, took 1500).
 constexpr int kColourPolls = 20000;
-// rank[2 g + side]: the group's priority rank on its body, -1 for a pinned one
+// rank[2 g + side]: the group's priority rank on its body, -1 for a pinned one (or the other side's body again)
 __global__ void k_colour_ranks(int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
                                const int* inc_count, const int* inc_items, int* rank) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, g = i >> 1;
     if (g >= n_groups) return;
     const int e = (i & 1) ? gb[g] : ga[g];
     int r = -1;
-    if (dynamic_body(bflags, e)) {
+    if (dynamic_body(bflags, e) && !((i & 1) && e == ga[g])) {
         const int* list = &inc_items[inc_start[e]];
         r = colour_rank(g, inc_count[e], [&](int k) { return list[k]; });
     }
@@ -1970,6 +1972,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
 #pragma unroll
         for (int s = 0; s < 2; s++)
             if (body[k][s] >= 0 && !dynamic_body(A.bflags, body[k][s])) body[k][s] = -1;
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+        if (body[k][1] == body[k][0]) body[k][1] = -1;
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
         const int g = t + k * kSmallThreads;

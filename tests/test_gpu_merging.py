@@ -182,3 +182,25 @@ def test_unmerge_all_matches_oracle(gpu_lib):
     for step in range(13, 31):
         step_both(ctx, mo, dt, step)
         compare_world(ctx, mo, step)
+
+
+def test_layout_of_contacts_inside_one_collection(gpu_lib):
+    """Contacts given between two members of one collection have the same solve
+    body on both sides: the group counts once among that body's groups, so the
+    layout ends, with every contact in the order once."""
+    ctx = Context()
+    ctx.upload(workloads.merge_stack(seed=4))
+    ctx.set_params(**PARAMS)
+    for _ in range(25):
+        st = ctx.step(0.01)
+    assert st["n_collections"] >= 1
+    parent, _ = ctx.structure()
+    coll = max(parent)
+    a, b = [i for i, p in enumerate(parent) if p == coll][:2]
+    free = next(i for i, p in enumerate(parent) if p != coll and i not in (a, b, coll))
+    b1, b2 = [a, a, a, b], [b, b, free, free]
+    p = np.zeros((4, 3))
+    ctx.push_contacts(b1, b2, p, np.tile([0.0, 1.0, 0.0], (4, 1)), np.full(4, -1e-3), info=[0, 1, 0, 0])
+    print("collection", coll, "members", a, b, "other", free, flush=True)
+    assert sorted(ctx.solve_order().tolist()) == [0, 1, 2, 3]
+    ctx.close()
