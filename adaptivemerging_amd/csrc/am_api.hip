@@ -423,7 +423,7 @@ int build_layout(am_ctx* c) {
     if (ng >= (1 << 28)) return fail(c, AM_ERR_INVALID, "more than 2^28 contact groups");
     hipStream_t s = c->stream;
     int* sc = c->d_scalars.p;
-    AM_HIP(c, c->s_colour_start.ensure(kMaxColours + 5));
+    AM_HIP(c, c->s_colour_start.ensure(kLayoutWords));
     AM_HIP(c, c->s_group_desc.ensure((size_t)std::max(ng, 1) * 4));
     AM_HIP(c, c->s_flow.ensure((size_t)std::max(ng, 1) * 4));
     AM_HIP(c, c->s_pred.ensure((size_t)std::max(ng, 1) * 2));
@@ -475,7 +475,7 @@ int build_layout(am_ctx* c) {
             fill_u64(s, c->g_taken.p, 2 * (size_t)c->n_ent, 0);
         }
     }
-    int* left = c->s_colour_start.p + kMaxColours + 4;
+    int* left = c->s_colour_start.p + kWordLeft;
     const int* cs = c->h_scalars + kHostLayout;
     // again if groups were left without a colour (launch_colour)
     for (int round = 0;; round++) {
@@ -492,20 +492,22 @@ int build_layout(am_ctx* c) {
                                  c->g_sizes.p, c->g_pos_start.p, c->s_order.p, c->s_group_desc.p, c->s_pos_a.p,
                                  c->g_spos.p, sc + 9, c->d_scan_temp.p);
             launch_flow_ranks(s, ng, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p,
-                              c->g_spos.p, c->s_group_desc.p, c->s_flow.p, c->s_pred.p);
+                              c->g_spos.p, c->s_group_desc.p, c->s_flow.p, c->s_pred.p,
+                              c->s_colour_start.p + kWordOneBody);
             if (rgrid > 0)
                 launch_resident_plan(s, c->s_colour_start.p, c->s_group_desc.p, 4 * rgrid, c->s_used.p,
-                                     c->s_colour_start.p + kMaxColours + 2);
+                                     c->s_colour_start.p + kWordPlan);
         }
         AM_HIP(c, hipGetLastError());
-        AM_HIP(c, hipMemcpyAsync(c->h_scalars + kHostLayout, c->s_colour_start.p, (kMaxColours + 5) * sizeof(int),
+        AM_HIP(c, hipMemcpyAsync(c->h_scalars + kHostLayout, c->s_colour_start.p, kLayoutWords * sizeof(int),
                                  hipMemcpyDeviceToHost, s));
         AM_HIP(c, hipStreamSynchronize(s));
-        if (small || ng == 0 || cs[kMaxColours + 4] == 0) break;
+        if (small || ng == 0 || cs[kWordLeft] == 0) break;
         if (round == 1000) return fail(c, AM_ERR_HIP, "colouring stopped making progress");
     }
-    const bool fits = rgrid > 0 && cs[kMaxColours + 2] <= kResidentDoubles && cs[kMaxColours + 3] <= kResidentSteps;
+    const bool fits = rgrid > 0 && cs[kWordPlan] <= kResidentDoubles && cs[kWordPlan + 1] <= kResidentSteps;
     c->resident_grid = fits ? rgrid : 0;
+    c->one_body_groups = ng > 0 && cs[kWordOneBody] != 0;
     int ncol = 0, maxc = 0;
     for (int q = 0; q <= kMaxColours; q++) {
         int sz = cs[q + 1] - cs[q];
@@ -788,7 +790,7 @@ int start_residual(am_ctx* c, PgsArgs G, double* out) {
     pc.pgs_block = 0;
     int grid = 1, block = 256;
     pgs_shape(c, pc, &grid, &block);
-    AM_HIP(c, launch_pgs(s, G, grid, block, c->params.pgs_plain_launch != 0));
+    AM_HIP(c, launch_pgs(s, G, grid, block, c->params.pgs_plain_launch != 0, c->one_body_groups));
     AM_HIP(c, c->d_resid.ensure(1));
     fill_int(s, (int*)c->d_resid.p, 2, 0);
     launch_start_residual(s, c->s_rec.p, c->s_meta.p, c->d_dv.p, c->d_minv.p, c->d_jinv.p, c->n_contacts, G.omega,
@@ -802,10 +804,15 @@ int start_residual(am_ctx* c, PgsArgs G, double* out) {
     return AM_OK;
 }
 
+// Whether a solve under P runs a dataflow kernel.  A group with one body on both
+// sides needs the coloured one, which gives the same bits.
+bool pgs_dataflow(const am_ctx* c, const am_params& P) { return P.pgs_schedule == 0 && !c->one_body_groups; }
+
 // Launch shape of the PGS kernel under P (after build_layout): workgroups and
 // threads per workgroup, clamped to what can be co-resident.
 void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
     bool ok = false;
+    const bool flow = pgs_dataflow(c, P);
     // Everything resident in LDS wherever it fits: it was the faster on every
     // contact set tried (us per sweep, k_pgs_flow -> resident, by contacts: 12:
     // 9 -> 6.3; 1,100 in a tower, one long chain: 24 -> 24; 750 between sphere
@@ -813,12 +820,12 @@ void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
     // 47 -> 27; 8,000 in one colour: 13 -> 5.4; 27,000 in 48 scenes: 47 -> 30).
     // Its arrival words take 1 KiB a sweep, hence the bound on the sweeps.  A
     // given pgs_grid asks for k_pgs_flow.
-    if (P.pgs_schedule == 0 && P.pgs_grid == 0 && c->resident_grid > 0 && P.iterations <= kResidentMaxSweeps) {
+    if (flow && P.pgs_grid == 0 && c->resident_grid > 0 && P.iterations <= kResidentMaxSweeps) {
         *grid = c->resident_grid;
         *block = kResidentThreads;
         return;
     }
-    if (P.pgs_schedule == 0) {
+    if (flow) {
         if (c->flow_max_grid == 0) {
             c->flow_max_grid = pgs_flow_max_blocks(&ok);
             if (!ok) c->flow_max_grid = 1;
@@ -831,7 +838,8 @@ void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
         *block = 64;
         return;
     }
-    const int b = P.pgs_block > 0 ? P.pgs_block : 256;
+    const bool given = P.pgs_schedule == 1;  // else the knobs are the dataflow schedule's
+    const int b = given && P.pgs_block > 0 ? P.pgs_block : 256;
     int& mx = c->pgs_max_grid[b / 64];
     if (mx == 0) {
         mx = pgs_max_blocks(b, &ok);
@@ -839,7 +847,7 @@ void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
     }
     // groups of a colour are dealt block-cyclically; about 20 groups of the
     // largest colour per workgroup (the best measured on the settling box pile)
-    int g = P.pgs_grid > 0 ? P.pgs_grid : (c->max_colour_groups + 19) / 20;
+    int g = given && P.pgs_grid > 0 ? P.pgs_grid : (c->max_colour_groups + 19) / 20;
     *grid = std::max(1, std::min(g, mx));
     *block = b;
 }
@@ -880,7 +888,7 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
     S.lam_alt = nullptr;
     S.iters_used = nullptr;
     S.scene_used = nullptr;
-    const bool flow = P.pgs_schedule == 0;
+    const bool flow = pgs_dataflow(c, P);
     MemBatch m(s);
     m.fill_int(c->d_scalars.p + 1, 1, c->n_contacts);
     for (auto& e : c->kev)
@@ -1031,7 +1039,7 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         launch_flow_end(s, F, S, c->n_contacts, (int)n_dv);
     } else {
         AM_HIP(c, hipEventRecord(c->kev[1], s));
-        AM_HIP(c, launch_pgs(s, G, grid, block, P.pgs_plain_launch != 0));
+        AM_HIP(c, launch_pgs(s, G, grid, block, P.pgs_plain_launch != 0, c->one_body_groups));
         AM_HIP(c, hipEventRecord(c->kev[2], s));
         launch_scene_finish(s, G);
         launch_unpack(s, S, c->n_contacts);

@@ -115,7 +115,7 @@ struct ContactStore {
 
 namespace am_rt {
 // Words of the pinned mirror: the scalars, then the layout's colour starts, plan and flag
-constexpr int kHostLayout = 32, kHostInts = kHostLayout + am::kMaxColours + 5;
+constexpr int kHostLayout = 32, kHostInts = kHostLayout + am::kLayoutWords;
 constexpr int kSweepsRead = 4096;  // a solve's sweeps read back with its result
 }  // namespace am_rt
 
@@ -186,6 +186,7 @@ struct am_ctx {
     DBuf<double> dv_alt, s_lam_alt;
     int flow_max_grid = 0;
     int resident_max_grid = 0;  // co-resident workgroups of the resident kernel (-1: none)
+    bool one_body_groups = false;  // of the current layout: some group's two solve bodies are one dynamic body
     int resident_grid = 0;      // workgroups it takes on the current layout, 0 where it does not fit
     // poses advanced by dt for the position-level motion metric
     DBuf<double> pose_xa, pose_Ra;

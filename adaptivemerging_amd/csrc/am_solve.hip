@@ -433,12 +433,12 @@ __global__ void k_colour_keys(int n_groups, const int* colour, const int* group_
 
 // colour_start[c] = first sorted position with colour >= c, c = 0..kMaxColours;
 // colour_start[kMaxColours + 1] = n_groups (the tail holds every colour from
-// kMaxColours on, in colour order); the two words after it are cleared for
-// k_resident_plan
+// kMaxColours on, in colour order); the words after it (kWordPlan ...) are
+// cleared for the kernels that follow
 __global__ void k_colour_starts(int n_groups, const uint64_t* sorted, int* colour_start) {
     int c = threadIdx.x;
     if (c > kMaxColours + 1) {
-        if (c < kMaxColours + 4) colour_start[c] = 0;
+        if (c < kLayoutWords && c != kWordLeft) colour_start[c] = 0;
         return;
     }
     if (c == kMaxColours + 1) {
@@ -511,7 +511,8 @@ AMD_INLINE int flow_rank(int q, int deg, Spos spos_of, int& pred) {
 // entries are in flight together (a thread per body, one entry at a time, took
 // 193 us on the settled 20,000-box pile; this takes 17).
 __global__ void k_flow_ranks(int n_groups, const int* bflags, const int* inc_start, const int* inc_count,
-                             const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred) {
+                             const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred,
+                             int* one_body) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, q = i >> 1, side = i & 1;
     if (q >= n_groups) return;
     const int e = group_desc[4 * q + 2 + side];
@@ -522,16 +523,18 @@ __global__ void k_flow_ranks(int n_groups, const int* bflags, const int* inc_sta
         int of;
         rank = flow_rank(q, deg, [&](int k) { return spos[inc_items[start + k]]; }, of);
         before = 2 * of + (group_desc[4 * of + 2] == e ? 0 : 1);
+        if (side && e == group_desc[4 * q + 2]) *one_body = 1;
     }
     reinterpret_cast<int2*>(flow)[i] = make_int2(rank, deg);
     pred[i] = before;
 }
 
 void launch_flow_ranks(hipStream_t s, int n_groups, const int* bflags, const int* inc_start, const int* inc_count,
-                       const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred) {
+                       const int* inc_items, const int* spos, const int* group_desc, int* flow, int* pred,
+                       int* one_body) {
     if (n_groups > 0)
         hipLaunchKernelGGL(k_flow_ranks, dim3((2 * n_groups + 255) / 256), dim3(256), 0, s, n_groups, bflags, inc_start,
-                           inc_count, inc_items, spos, group_desc, flow, pred);
+                           inc_count, inc_items, spos, group_desc, flow, pred, one_body);
 }
 
 // The division (D lambda - omega (b + J.dv)) / (D + C) of a row.  The
@@ -782,8 +785,9 @@ AMD_INLINE Row row_of(const double* rec, int r) {
     return Row{ld3(q + kRecAw), ld3(q + kRecBv), ld3(q + kRecBw), ld3(q + kRecTa), ld3(q + kRecTb)};
 }
 
-// PGS.updateDeltaVwithLambdai (PGS.java:221-245)
-AMD_INLINE void apply_row(const Row& R, double lambda, BodyRegs& A, BodyRegs& Bb) {
+// PGS.updateDeltaVwithLambdai (PGS.java:221-245).  one: both sides are the same
+// body, whose deltaV takes A's half first, then B's.
+AMD_INLINE void apply_row(const Row& R, double lambda, BodyRegs& A, BodyRegs& Bb, bool one) {
     double s1 = A.minv * lambda;
     A.dv[0] = s1 * -R.bv.x + A.dv[0];
     A.dv[1] = s1 * -R.bv.y + A.dv[1];
@@ -791,6 +795,9 @@ AMD_INLINE void apply_row(const Row& R, double lambda, BodyRegs& A, BodyRegs& Bb
     A.dv[3] = lambda * R.ta.x + A.dv[3];
     A.dv[4] = lambda * R.ta.y + A.dv[4];
     A.dv[5] = lambda * R.ta.z + A.dv[5];
+    if (one)
+#pragma unroll
+        for (int i = 0; i < 6; i++) Bb.dv[i] = A.dv[i];
     double s2 = Bb.minv * lambda;
     Bb.dv[0] = s2 * R.bv.x + Bb.dv[0];
     Bb.dv[1] = s2 * R.bv.y + Bb.dv[1];
@@ -798,6 +805,9 @@ AMD_INLINE void apply_row(const Row& R, double lambda, BodyRegs& A, BodyRegs& Bb
     Bb.dv[3] = lambda * R.tb.x + Bb.dv[3];
     Bb.dv[4] = lambda * R.tb.y + Bb.dv[4];
     Bb.dv[5] = lambda * R.tb.z + Bb.dv[5];
+    if (one)
+#pragma unroll
+        for (int i = 0; i < 6; i++) A.dv[i] = Bb.dv[i];
 }
 // Contact.getJdv (Contact.java:362-378)
 AMD_INLINE double jdv(const Row& R, const BodyRegs& A, const BodyRegs& Bb) {
@@ -824,12 +834,14 @@ AMD_INLINE void load_rec(const double2* src, Rec& r) {
 // One group (the contacts of one body pair): mode 0 is confidentWarmStart
 // (PGS.java:250-256), mode 1 one PGS pass (PGS.java:100-184).  recs points at
 // the group's first record; lambda and the contact state are written back at
-// sweep position k.
+// sweep position k.  kOneBody: groups may have one body on both sides.
+template <bool kOneBody>
 AMD_INLINE void process_group(const PgsArgs& P, int4 gd, const double2* recs, int mode, bool last_iter, double& mx) {
     const int k0 = gd.x, k1 = gd.y, A = gd.z, Bi = gd.w;
     BodyRegs ra, rb;
     load_body(P, A, ra);
     load_body(P, Bi, rb);
+    const bool one = kOneBody && A == Bi;
     bool nan = false;
     for (int k = k0; k < k1; k++) {
         Rec cur;
@@ -838,7 +850,7 @@ AMD_INLINE void process_group(const PgsArgs& P, int4 gd, const double2* recs, in
         double lam[3] = {rec[kRecLambda + 0], rec[kRecLambda + 1], rec[kRecLambda + 2]};
         if (mode == 0) {
 #pragma unroll
-            for (int r = 0; r < 3; r++) apply_row(row_of(rec, r), lam[r], ra, rb);
+            for (int r = 0; r < 3; r++) apply_row(row_of(rec, r), lam[r], ra, rb, one);
         } else {
             const bool clamp = rec[kRecClamp] != 0.0;
             const double mu = rec[kRecMu];
@@ -861,7 +873,7 @@ AMD_INLINE void process_group(const PgsArgs& P, int4 gd, const double2* recs, in
                 }
                 lam[r] = l;
                 double diff = l - prev;
-                apply_row(R, diff, ra, rb);
+                apply_row(R, diff, ra, rb, one);
                 // Math.max over |diff| (PGS.java:125); a NaN is carried separately
                 mx = fmax(mx, fabs(diff));
                 nan = nan || diff != diff;
@@ -931,8 +943,11 @@ AMD_INLINE bool grid_barrier(const PgsArgs& P, unsigned& epoch) {
 // (group j of the colour goes to block j % grid, lane j / grid) so every
 // workgroup, hence every CU in use, gets a share.  The per-sweep max |delta
 // lambda| is reduced with an integer atomic max on the bit pattern (non-
-// negative doubles order as their bits) into a slot per sweep.
-template <bool kSingleBlock>
+// negative doubles order as their bits) into a slot per sweep.  kOneBody: for
+// contact sets where some group's two solve bodies are the same one (contacts
+// given between members of one collection).  Only this kernel knows such groups:
+// a thread holds both sides, where the dataflow kernels' lanes keep a deltaV each.
+template <bool kSingleBlock, bool kOneBody>
 __global__ __launch_bounds__(256) void k_pgs(PgsArgs P) {
     const int* cs = P.colour_start;
     const int slot0 = threadIdx.x * gridDim.x + blockIdx.x;
@@ -968,7 +983,7 @@ __global__ __launch_bounds__(256) void k_pgs(PgsArgs P) {
     // after the grid barrier), and each group's max goes to its scene too
     auto run_group = [&](int q, int4 gd, int mode, bool last, double& mx) {
         if (!P.per_scene || mode == 0) {
-            process_group(P, gd, grec + (size_t)gd.x * kRec2, mode, last, mx);
+            process_group<kOneBody>(P, gd, grec + (size_t)gd.x * kRec2, mode, last, mx);
             return;
         }
         const int sc = P.g_scene[q];
@@ -978,7 +993,7 @@ __global__ __launch_bounds__(256) void k_pgs(PgsArgs P) {
             if (prev < P.tolerance) return;
         }
         double gmx = 0.0;
-        process_group(P, gd, grec + (size_t)gd.x * kRec2, mode, last, gmx);
+        process_group<kOneBody>(P, gd, grec + (size_t)gd.x * kRec2, mode, last, gmx);
         if (!(gmx <= 0))
             atomicMax(&P.scene_max[(size_t)sc * P.iterations + it], (unsigned long long)__double_as_longlong(gmx));
         mx = gmx != gmx ? gmx : fmax(mx, gmx);
@@ -1052,24 +1067,29 @@ int pgs_max_blocks(int block, bool* ok) {
     int dev = 0, n_cu = 0, per_cu = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pgs<false>, block, 0);
+    int one_body = 0;
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pgs<false, false>, block, 0);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&one_body, k_pgs<false, true>, block, 0);
+    per_cu = std::min(per_cu, one_body);
     *ok = per_cu > 0;
     return n_cu * (per_cu > 0 ? per_cu : 1);
 }
 
-hipError_t launch_pgs(hipStream_t s, const PgsArgs& P, int grid, int block, bool plain) {
+hipError_t launch_pgs(hipStream_t s, const PgsArgs& P, int grid, int block, bool plain, bool one_body) {
+    void (*single)(PgsArgs) = one_body ? k_pgs<true, true> : k_pgs<true, false>;
+    void (*kernel)(PgsArgs) = one_body ? k_pgs<false, true> : k_pgs<false, false>;
     if (grid <= 1) {
-        hipLaunchKernelGGL(k_pgs<true>, dim3(1), dim3(block), 0, s, P);
+        hipLaunchKernelGGL(single, dim3(1), dim3(block), 0, s, P);
         return hipGetLastError();
     }
     if (plain) {
         // the caller clamps grid to the co-resident limit; the barrier's spin
         // limit turns a grid that is not co-resident into an error
-        hipLaunchKernelGGL(k_pgs<false>, dim3(grid), dim3(block), 0, s, P);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, s, P);
         return hipGetLastError();
     }
     void* args[] = {(void*)&P};
-    return hipLaunchCooperativeKernel((const void*)k_pgs<false>, dim3(grid), dim3(block), args, 0, s);
+    return hipLaunchCooperativeKernel((const void*)kernel, dim3(grid), dim3(block), args, 0, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1918,6 +1938,7 @@ struct SmallLds {
     int cs[kMaxColours + 2];
     int n_items;
     int plan[2];
+    int one_body;
     ResidentSteps steps;
 };
 static_assert(sizeof(SmallLds) <= 160 * 1024, "LDS of a CU");
@@ -2208,6 +2229,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
     }
     if (t <= kMaxColours + 1) A.colour_start[t] = L.cs[t];
     if (t < 2) L.plan[t] = 0;
+    if (t == 2) L.one_body = 0;
     __syncthreads();
     for (int q = t / 4; q < n; q += kSmallThreads / 4) {
         const int g = L.sorted[q], o = L.pos[q], size = L.pos[q + 1] - o, k0 = A.group_start[g];
@@ -2228,6 +2250,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
             int of;
             rank = flow_rank(q, deg, [&](int k) { return (int)L.colour[L.item[s0 + k]]; }, of);
             pred = 2 * of + (A.ga[L.sorted[of]] == e ? 0 : 1);
+            if ((i & 1) && e == A.ga[g]) L.one_body = 1;
         }
         reinterpret_cast<int2*>(A.flow)[i] = make_int2(rank, deg);
         A.pred[i] = pred;
@@ -2252,7 +2275,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
         }
     }
     __syncthreads();
-    if (t < 2) A.colour_start[kMaxColours + 2 + t] = L.plan[t];
+    if (t < 2) A.colour_start[kWordPlan + t] = L.plan[t];
+    if (t == 2) A.colour_start[kWordOneBody] = L.one_body;
 }
 void launch_layout_small(hipStream_t s, const SmallLayoutArgs& A) {
     hipLaunchKernelGGL(k_layout_small, dim3(1), dim3(kSmallThreads), 0, s, A);

@@ -85,6 +85,12 @@ constexpr int kResidentThreads = 320;
 constexpr int kResidentMaxWaves = 1024;
 constexpr int kResidentMaxSweeps = 65536;
 
+// Words behind the colour starts (kMaxColours + 2 of them), read back with them:
+// the resident kernel's plan (2), whether groups are left without a colour, and
+// whether some group's two solve bodies are one dynamic body.
+constexpr int kWordPlan = kMaxColours + 2, kWordLeft = kMaxColours + 4, kWordOneBody = kMaxColours + 5,
+              kLayoutWords = kMaxColours + 6;
+
 struct FlowArgs {
     PgsArgs P;
     const int* flow;       // int4 per sorted group: rank_a, deg_a, rank_b, deg_b
@@ -176,7 +182,8 @@ void launch_unpack(hipStream_t s, const SetupArgs& S, int cap);
 struct FlowArgs;
 void launch_flow_end(hipStream_t s, const FlowArgs& F, const SetupArgs& S, int cap, int n_dv);
 int pgs_max_blocks(int block, bool* ok);
-hipError_t launch_pgs(hipStream_t s, const PgsArgs& P, int grid, int block, bool plain);
+// one_body: some group's two solve bodies are the same one
+hipError_t launch_pgs(hipStream_t s, const PgsArgs& P, int grid, int block, bool plain, bool one_body);
 int pgs_flow_max_blocks(bool* ok);
 // block 64: k_pgs_flow; kResidentThreads: the resident kernel
 hipError_t launch_pgs_flow(hipStream_t s, const FlowArgs& F, int grid, int block, bool plain);
@@ -187,7 +194,7 @@ void launch_resident_plan(hipStream_t s, const int* colour_start, const int* gro
                           int* plan);
 void launch_flow_ranks(hipStream_t s, int n_groups, const int* bflags, const int* inc_start,
                        const int* inc_count, const int* inc_items, const int* spos, const int* group_desc,
-                       int* flow, int* pred);
+                       int* flow, int* pred, int* one_body);
 void launch_map_insert(hipStream_t s, const OldContactsView& O, int* table);
 // O.first: one word for each old contact, INT_MAX before the call; match: 2 n words
 void launch_warm_start(hipStream_t s, BodiesView B, ContactsView C, OldContactsView O, int n, int post, int* match,

@@ -170,7 +170,8 @@ typedef struct am_params {
                                          support cooperative launches (0 = cooperative) */
     int32_t pgs_schedule;             /* 0: dataflow (each body's deltaV handed from update to update, no grid barriers);
                                          1: colour by colour with a grid barrier between colours.
-                                         Both give bit-identical results (the exported sweep order) */
+                                         Both give bit-identical results (the exported sweep order).  Contacts pushed
+                                         between two members of one collection are always solved by the second */
     /* learned warm start (no reference counterpart): 0 plain previous-frame
      * start; 1 the MLP's predicted start, falling back to the plain start
      * whenever its start residual is not smaller */

@@ -204,3 +204,53 @@ def test_layout_of_contacts_inside_one_collection(gpu_lib):
     print("collection", coll, "members", a, b, "other", free, flush=True)
     assert sorted(ctx.solve_order().tolist()) == [0, 1, 2, 3]
     ctx.close()
+
+
+@pytest.mark.parametrize("iterations", [0, 1, 2, 7])
+def test_solve_of_contacts_inside_one_collection(gpu_lib, iterations):
+    """A group with the same solve body on both sides: both halves of its updates
+    act on that body's one deltaV, under every schedule and launch shape, as in the
+    oracle's sequential sweep (bit for bit).  Such groups alone, before and behind
+    groups with another body, listed either way round, with lambdas to start from."""
+    ctx, mo = make(workloads.merge_stack(seed=4), enable_merge_pinned=0)
+    dt = 0.01
+    for step in range(1, 26):
+        step_both(ctx, mo, dt, step)
+    mo.set_params(iterations=iterations, tolerance=0.0)
+    parent, _ = ctx.structure()
+    coll = max(parent)
+    inside = [i for i, p in enumerate(parent) if p == coll]
+    assert coll >= 0 and len(inside) >= 2 and not mo.pinned(coll)
+    a, b = inside[:2]
+    free = next(i for i, p in enumerate(parent[:mo.n_phys]) if p != coll and not mo.pinned(i))
+    x = ctx.pull_state(mo.n_phys)[0]
+    rng = np.random.default_rng(iterations)
+    f = rng.normal(size=(mo.n_entities, 3))
+    for pairs in ([(a, b)] * 3, [(a, b), (b, a), (a, free), (b, free), (b, free)], [(a, free), (a, b), (b, a)]):
+        n = len(pairs)
+        b1, b2 = np.array(pairs, np.int32).T.copy()
+        p = (x[b1] + x[b2]) / 2 + rng.uniform(-0.1, 0.1, (n, 3))
+        nrm = rng.normal(size=(n, 3))
+        nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+        lam = np.abs(rng.normal(size=(n, 3)))
+        for shape in (dict(), dict(pgs_grid=64), dict(pgs_schedule=1), dict(pgs_plain_launch=1)):
+            ctx.set_params(**{**dict(iterations=iterations, tolerance=0.0, pgs_schedule=0, pgs_grid=0,
+                                     pgs_plain_launch=0), **shape})
+            for o in (ctx, mo.o):
+                o.clear_bodies()
+                o.push_forces(f, f[::-1].copy())
+                o.push_contacts(b1, b2, p, nrm, np.full(n, -1e-3), info=np.arange(n))
+                o.push_lambdas(lam)
+            it_g, _ = ctx.solve(dt)
+            it_o, _, _ = mo.o.solve(ctx.solve_order(), dt)
+            print(pairs, shape, "shape", ctx.launch_shape(), "sweeps", it_g, flush=True)
+            assert it_g == it_o == iterations
+            assert_contacts_equal(ctx.contacts(), mo.o.contacts())
+            dv = ctx.pull_deltav(mo.n_entities)
+            assert_bits_equal("deltaV", dv, mo.o.pull_deltav())
+            # the halves of a group inside the collection cancel, the other groups' do not
+            assert np.any(dv[coll] != 0) == any(free in q for q in pairs)
+        ctx.set_params(pgs_schedule=0, pgs_grid=0, pgs_plain_launch=0)
+    if iterations:
+        ctx.autotune(dt, sweeps=3, reps=1, apply=False)  # raises on a shape that changes the bits
+    ctx.close()
