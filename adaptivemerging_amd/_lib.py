@@ -154,7 +154,7 @@ SYMBOLS = [
     "am_springs_set", "am_apply_spring_forces", "am_wake", "am_sleep", "am_wake_all", "am_sleep_state_pull", "am_unmerge_all",
     "am_update_contacts_map", "am_detect", "am_contacts_push", "am_contacts_pull", "am_lambdas_push",
     "am_warm_start", "am_redo_warm_start", "am_no_warm_start", "am_solve", "am_solve_order_pull",
-    "am_colours_pull", "am_update_in_collections", "am_changes_pull", "am_advance_velocities",
+    "am_colours_pull", "am_colour_polls_set", "am_update_in_collections", "am_changes_pull", "am_advance_velocities",
     "am_advance_positions", "am_accumulate_for_unmerging", "am_unmerge", "am_clear_top_level",
     "am_clear_body_pair_contacts", "am_accumulate_for_merging", "am_merge", "am_body_pairs_pull",
     "am_internal_contacts_pull",
@@ -225,6 +225,7 @@ def load(path: str = LIB_PATH) -> C.CDLL:
         "am_solve": (C.c_int, [ctxp, dbl, i32, C.POINTER(i32), C.POINTER(dbl)]),
         "am_solve_order_pull": (C.c_int, [ctxp, vp, i32, C.POINTER(i32)]),
         "am_colours_pull": (C.c_int, [ctxp, vp, i32, C.POINTER(i32)]),
+        "am_colour_polls_set": (C.c_int, [ctxp, i32]),
         "am_update_in_collections": (C.c_int, [ctxp, dbl, C.POINTER(i32)]),
         "am_accumulate_for_unmerging": (C.c_int, [ctxp, dbl]),
         "am_unmerge": (C.c_int, [ctxp, dbl, C.POINTER(i32)]),

@@ -338,6 +338,10 @@ class Context:
         self._check(self.lib.am_colours_pull(self.h, ptr(col) if nc else None, nc, C.byref(k)))
         return col, k.value
 
+    def set_colour_polls(self, polls: int):
+        """Bound of the colouring's polls (am_colour_polls_set; for tests)."""
+        self._check(self.lib.am_colour_polls_set(self.h, polls))
+
     def changes(self) -> np.ndarray:
         n = C.c_int32()
         self._check(self.lib.am_changes_pull(self.h, None, 0, C.byref(n)))

@@ -415,49 +415,13 @@ int refresh_jinv(am_ctx* c) {
     return AM_OK;
 }
 
-// Colouring and sweep layout for the current groups (depends only on the
-// contact list and the solve bodies).
-int build_layout(am_ctx* c) {
-    if (c->layout_valid) return AM_OK;
+// The layout's launches: colours (with again, only those that the last time left
+// open), then all that follows from them.
+int layout_by_launches(am_ctx* c, bool again, int rgrid) {
     const int ng = c->n_groups;
-    if (ng >= (1 << 28)) return fail(c, AM_ERR_INVALID, "more than 2^28 contact groups");
     hipStream_t s = c->stream;
     int* sc = c->d_scalars.p;
-    AM_HIP(c, c->s_colour_start.ensure(kLayoutWords));
-    AM_HIP(c, c->s_group_desc.ensure((size_t)std::max(ng, 1) * 4));
-    AM_HIP(c, c->s_flow.ensure((size_t)std::max(ng, 1) * 4));
-    AM_HIP(c, c->s_pred.ensure((size_t)std::max(ng, 1) * 2));
-    AM_HIP(c, c->s_used.ensure(kResidentMaxWaves));
-    if (c->resident_max_grid == 0) {
-        bool ok = false;
-        c->resident_max_grid = pgs_resident_max_blocks(&ok);
-        if (!ok) c->resident_max_grid = -1;
-    }
-    // a group a wave as far as there are waves
-    const int rgrid = std::max(0, std::min((std::min(ng, kResidentMaxWaves) + 3) / 4, c->resident_max_grid));
-    const bool small = ng > 0 && ng <= kSmallLayout;
-    if (small) {
-        SmallLayoutArgs A;
-        A.n_groups = ng;
-        A.n_ent = c->n_ent;
-        A.waves = 4 * rgrid;
-        A.ga = c->g_a.p;
-        A.gb = c->g_b.p;
-        A.bflags = c->d_flags.p;
-        A.group_start = c->g_start.p;
-        A.layer = c->layout_layer;
-        A.inc_count = c->inc_count.p;
-        A.inc_start = c->inc_start.p;
-        A.colour_start = c->s_colour_start.p;
-        A.pos_start = c->g_pos_start.p;
-        A.order = c->s_order.p;
-        A.pos_a = c->s_pos_a.p;
-        A.group_desc = c->s_group_desc.p;
-        A.flow = c->s_flow.p;
-        A.pred = c->s_pred.p;
-        A.used = c->s_used.p;
-        launch_layout_small(s, A);
-    } else if (ng > 0) {
+    if (ng > 0 && !again) {
         fill_int(s, c->inc_count.p, c->n_ent + 1, 0);
         fill_int(s, c->inc_cursor.p, c->n_ent + 1, 0);
         launch_incidence(s, false, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_count.p, nullptr, nullptr, nullptr);
@@ -475,34 +439,83 @@ int build_layout(am_ctx* c) {
             fill_u64(s, c->g_taken.p, 2 * (size_t)c->n_ent, 0);
         }
     }
-    int* left = c->s_colour_start.p + kWordLeft;
+    if (ng > 0) {
+        int* left = c->s_colour_start.p + kWordLeft;
+        fill_int(s, left, 1, 0);
+        launch_colour(s, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p,
+                      c->g_colour.p, c->g_taken.p, c->g_rank.p, left, c->layout_layer, c->g_blocker.p, again,
+                      c->colour_polls > 0 ? c->colour_polls : kColourPolls);
+        launch_colour_keys(s, ng, c->g_colour.p, c->g_start.p, c->g_keys.p);
+        sort_u64(s, c->g_keys.p, c->g_keys_sorted.p, ng, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
+    }
+    launch_colour_layout(s, ng, c->g_keys_sorted.p, c->g_start.p, c->g_a.p, c->g_b.p, c->s_colour_start.p,
+                         c->g_sizes.p, c->g_pos_start.p, c->s_order.p, c->s_group_desc.p, c->s_pos_a.p, c->g_spos.p,
+                         sc + 9, c->d_scan_temp.p);
+    launch_flow_ranks(s, ng, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p, c->g_spos.p,
+                      c->s_group_desc.p, c->s_flow.p, c->s_pred.p, c->s_colour_start.p + kWordOneBody);
+    if (rgrid > 0)
+        launch_resident_plan(s, c->s_colour_start.p, c->s_group_desc.p, 4 * rgrid, c->s_used.p,
+                             c->s_colour_start.p + kWordPlan);
+    return AM_OK;
+}
+
+// Colouring and sweep layout for the current groups (depends only on the
+// contact list and the solve bodies).
+int build_layout(am_ctx* c) {
+    if (c->layout_valid) return AM_OK;
+    const int ng = c->n_groups;
+    if (ng >= (1 << 28)) return fail(c, AM_ERR_INVALID, "more than 2^28 contact groups");
+    hipStream_t s = c->stream;
+    AM_HIP(c, c->s_colour_start.ensure(kLayoutWords));
+    AM_HIP(c, c->s_group_desc.ensure((size_t)std::max(ng, 1) * 4));
+    AM_HIP(c, c->s_flow.ensure((size_t)std::max(ng, 1) * 4));
+    AM_HIP(c, c->s_pred.ensure((size_t)std::max(ng, 1) * 2));
+    AM_HIP(c, c->s_used.ensure(kResidentMaxWaves));
+    if (c->resident_max_grid == 0) {
+        bool ok = false;
+        c->resident_max_grid = pgs_resident_max_blocks(&ok);
+        if (!ok) c->resident_max_grid = -1;
+    }
+    // a group a wave as far as there are waves
+    const int rgrid = std::max(0, std::min((std::min(ng, kResidentMaxWaves) + 3) / 4, c->resident_max_grid));
     const int* cs = c->h_scalars + kHostLayout;
+    // The whole layout in one workgroup, or (also where that gave up) by launches,
     // again if groups were left without a colour (launch_colour)
-    for (int round = 0;; round++) {
-        if (!small) {
-            if (ng > 0) {
-                fill_int(s, left, 1, 0);
-                launch_colour(s, ng, c->g_a.p, c->g_b.p, c->d_flags.p, c->inc_start.p, c->inc_count.p,
-                              c->inc_items.p, c->g_colour.p, c->g_taken.p, c->g_rank.p, left, c->layout_layer,
-                              c->g_blocker.p, round > 0);
-                launch_colour_keys(s, ng, c->g_colour.p, c->g_start.p, c->g_keys.p);
-                sort_u64(s, c->g_keys.p, c->g_keys_sorted.p, ng, c->d_sort_temp.p, c->d_sort_temp.n, 0, 64);
-            }
-            launch_colour_layout(s, ng, c->g_keys_sorted.p, c->g_start.p, c->g_a.p, c->g_b.p, c->s_colour_start.p,
-                                 c->g_sizes.p, c->g_pos_start.p, c->s_order.p, c->s_group_desc.p, c->s_pos_a.p,
-                                 c->g_spos.p, sc + 9, c->d_scan_temp.p);
-            launch_flow_ranks(s, ng, c->d_flags.p, c->inc_start.p, c->inc_count.p, c->inc_items.p,
-                              c->g_spos.p, c->s_group_desc.p, c->s_flow.p, c->s_pred.p,
-                              c->s_colour_start.p + kWordOneBody);
-            if (rgrid > 0)
-                launch_resident_plan(s, c->s_colour_start.p, c->s_group_desc.p, 4 * rgrid, c->s_used.p,
-                                     c->s_colour_start.p + kWordPlan);
+    bool small = ng > 0 && ng <= kSmallLayout;
+    for (int round = 0;;) {
+        if (small) {
+            SmallLayoutArgs A;
+            A.n_groups = ng;
+            A.n_ent = c->n_ent;
+            A.waves = 4 * rgrid;
+            A.max_polls = c->colour_polls > 0 ? c->colour_polls : kSmallPolls;
+            A.ga = c->g_a.p;
+            A.gb = c->g_b.p;
+            A.bflags = c->d_flags.p;
+            A.group_start = c->g_start.p;
+            A.layer = c->layout_layer;
+            A.inc_count = c->inc_count.p;
+            A.inc_start = c->inc_start.p;
+            A.colour_start = c->s_colour_start.p;
+            A.pos_start = c->g_pos_start.p;
+            A.order = c->s_order.p;
+            A.pos_a = c->s_pos_a.p;
+            A.group_desc = c->s_group_desc.p;
+            A.flow = c->s_flow.p;
+            A.pred = c->s_pred.p;
+            A.used = c->s_used.p;
+            launch_layout_small(s, A);
+        } else {
+            int r = layout_by_launches(c, round > 0, rgrid);
+            if (r) return r;
+            round++;
         }
         AM_HIP(c, hipGetLastError());
         AM_HIP(c, hipMemcpyAsync(c->h_scalars + kHostLayout, c->s_colour_start.p, kLayoutWords * sizeof(int),
                                  hipMemcpyDeviceToHost, s));
         AM_HIP(c, hipStreamSynchronize(s));
-        if (small || ng == 0 || cs[kWordLeft] == 0) break;
+        if (ng == 0 || cs[kWordLeft] == 0) break;
+        small = false;
         if (round == 1000) return fail(c, AM_ERR_HIP, "colouring stopped making progress");
     }
     const bool fits = rgrid > 0 && cs[kWordPlan] <= kResidentDoubles && cs[kWordPlan + 1] <= kResidentSteps;
@@ -2125,6 +2138,14 @@ int am_colours_pull(am_ctx* c, int32_t* colour_of_contact, int32_t capacity, int
                 for (int k = pos[q]; k < pos[q + 1]; k++)
                     if (order[k] < capacity) colour_of_contact[order[k]] = col;
     }
+    return AM_OK;
+}
+
+int am_colour_polls_set(am_ctx* c, int32_t polls) {
+    if (!c) return AM_ERR_INVALID;
+    if (polls < 0) return fail(c, AM_ERR_INVALID, "polls must be >= 0");
+    c->colour_polls = polls;
+    c->layout_valid = false;
     return AM_OK;
 }
 

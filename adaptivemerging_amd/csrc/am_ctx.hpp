@@ -275,6 +275,7 @@ struct am_ctx {
     DBuf<int> g_layer, bfs_mark;
     DBuf<int> g_blocker, g_rank;  // colouring: the neighbour a layered group waits for; priority ranks
     DBuf<am::TakenColours> g_taken;
+    int colour_polls = 0;         // am_colour_polls_set
     const int* layout_layer = nullptr;  // set while the single sweep builds its layout
     DBuf<int> sweep_order;              // order of the last single sweep inside collections
     int sweep_order_n = -1;             // -1: none since the last solve or detection

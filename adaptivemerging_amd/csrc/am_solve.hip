@@ -323,7 +323,6 @@ AMD_INLINE void st_u64(unsigned long long* p, unsigned long long v) {
 // groups each waiting for another, a link of which costs a store and the load
 // that sees it (settled 20,000-box pile, 104,000 groups: 84 us; a launch per
 // round of the colouring, which went through the lists again, took 1500).
-constexpr int kColourPolls = 20000;
 // rank[2 g + side]: the group's priority rank on its body, -1 for a pinned one (or the other side's body again)
 __global__ void k_colour_ranks(int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
                                const int* inc_count, const int* inc_items, int* rank) {
@@ -338,7 +337,7 @@ __global__ void k_colour_ranks(int n_groups, const int* ga, const int* gb, const
     rank[i] = r;
 }
 __global__ __launch_bounds__(256) void k_colour(int n_groups, const int* ga, const int* gb, const int* rank,
-                                                int* colour, TakenColours* taken, int* remaining) {
+                                                int* colour, TakenColours* taken, int* remaining, int max_polls) {
     const int threads = gridDim.x * blockDim.x, first = blockIdx.x * blockDim.x + threadIdx.x;
     struct Group {
         int a, b, ra, rb;
@@ -378,7 +377,7 @@ __global__ __launch_bounds__(256) void k_colour(int n_groups, const int* ga, con
         for (int g = first + threads; g < n_groups; g += threads)
             if (colour[g] < 0 && !attempt(g, load(g))) left = true;
         if (!__any(left)) return;
-        if (polls >= kColourPolls) {
+        if (polls >= max_polls) {
             *remaining = 1;
             return;
         }
@@ -388,7 +387,7 @@ __global__ __launch_bounds__(256) void k_colour(int n_groups, const int* ga, con
 __global__ __launch_bounds__(256) void k_colour_layered(int n_groups, const int* ga, const int* gb, const int* bflags,
                                                         const int* inc_start, const int* inc_count,
                                                         const int* inc_items, int* colour, int* remaining,
-                                                        const int* layer, int* blocker) {
+                                                        const int* layer, int* blocker, int max_polls) {
     const int quads = gridDim.x * (blockDim.x / 4), quad = (blockIdx.x * blockDim.x + threadIdx.x) / 4;
     for (int polls = 0;; polls++) {
         bool left = false;
@@ -411,7 +410,7 @@ __global__ __launch_bounds__(256) void k_colour_layered(int n_groups, const int*
             left = left || c < 0;
         }
         if (!__any(left)) return;
-        if (polls >= kColourPolls) {
+        if (polls >= max_polls) {
             *remaining = 1;
             return;
         }
@@ -1937,6 +1936,7 @@ struct SmallLds {
     int wave_sum[kSmallWaves];
     int cs[kMaxColours + 2];
     int n_items;
+    int gave_up;
     int plan[2];
     int one_body;
     ResidentSteps steps;
@@ -1978,7 +1978,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
 
     // incidence lists: a body's groups in any order
     for (int e = t; e < A.n_ent; e += kSmallThreads) st_int(&A.inc_count[e], 0);
-    if (t == 0) L.n_items = 0;
+    if (t == 0) L.n_items = L.gave_up = 0;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int body[kPer][2], at[kPer][2], count[kPer][2];  // this thread's groups; -1: a pinned body
@@ -2060,7 +2060,11 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
                                              : 0;
         }
         bool left = true;
-        while (left) {
+        for (int polls = 0; left; polls++) {
+            if (polls > A.max_polls) {
+                L.gave_up = 1;
+                break;
+            }
             left = false;
 #pragma unroll
             for (int k = 0; k < kPer; k++) {
@@ -2101,7 +2105,11 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
             __hip_atomic_store(p, (short)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         };
         bool left = true;
-        while (__any(left)) {
+        for (int polls = 0; __any(left); polls++) {
+            if (polls > A.max_polls) {
+                L.gave_up = 1;
+                break;
+            }
             left = false;
             for (int g = t / 4; g < n; g += kSmallThreads / 4) {
                 if (get(&L.colour[g]) >= 0) continue;
@@ -2120,6 +2128,10 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
         }
     }
     __syncthreads();
+    if (L.gave_up) {
+        if (t == 0) A.colour_start[kWordLeft] = 1;
+        return;
+    }
 
     // sorted positions: a stable counting sort over (colour, larger groups first)
     for (int i = t; i < kSmallWaves * (kSmallBins + 7); i += kSmallThreads) (&L.hist[0][0])[i] = 0;
@@ -2277,6 +2289,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
     __syncthreads();
     if (t < 2) A.colour_start[kWordPlan + t] = L.plan[t];
     if (t == 2) A.colour_start[kWordOneBody] = L.one_body;
+    if (t == 3) A.colour_start[kWordLeft] = 0;
 }
 void launch_layout_small(hipStream_t s, const SmallLayoutArgs& A) {
     hipLaunchKernelGGL(k_layout_small, dim3(1), dim3(kSmallThreads), 0, s, A);
@@ -3701,20 +3714,21 @@ void launch_incidence(hipStream_t s, bool fill, int n_groups, const int* ga, con
 }
 void launch_colour(hipStream_t s, int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
                    const int* inc_count, const int* inc_items, int* colour, TakenColours* taken, int* rank,
-                   int* remaining, const int* layer, int* blocker, bool again) {
+                   int* remaining, const int* layer, int* blocker, bool again, int max_polls) {
     if (n_groups <= 0) return;
-    // at most 8 workgroups on each of 256 CUs: as many as can run at once
+    // at most 8 workgroups on each of 256 CUs (workgroups that wait for others that
+    // are not resident give up in the end and leave room for them)
     const int per = layer ? 64 : 256;
     const dim3 g(std::min((n_groups + per - 1) / per, 2048)), b(256);
     if (layer) {
         hipLaunchKernelGGL(k_colour_layered, g, b, 0, s, n_groups, ga, gb, bflags, inc_start, inc_count, inc_items,
-                           colour, remaining, layer, blocker);
+                           colour, remaining, layer, blocker, max_polls);
         return;
     }
     if (!again)
         hipLaunchKernelGGL(k_colour_ranks, dim3((2 * n_groups + 255) / 256), b, 0, s, n_groups, ga, gb, bflags,
                            inc_start, inc_count, inc_items, rank);
-    hipLaunchKernelGGL(k_colour, g, b, 0, s, n_groups, ga, gb, rank, colour, taken, remaining);
+    hipLaunchKernelGGL(k_colour, g, b, 0, s, n_groups, ga, gb, rank, colour, taken, remaining, max_polls);
 }
 void launch_colour_keys(hipStream_t s, int n_groups, const int* colour, const int* group_start, uint64_t* keys) {
     if (n_groups > 0)

@@ -152,16 +152,21 @@ struct TakenColours {
 };
 // colour[] and blocker[] start at -1, taken[] (by body) at 0; blocker is for
 // layers, taken and rank (2 n_groups) for none.  *remaining: some group has no
-// colour yet (launch again)
+// colour yet (launch again); its thread gave up after max_polls polls
+constexpr int kColourPolls = 20000;  // each a memory round trip
 void launch_colour(hipStream_t s, int n_groups, const int* ga, const int* gb, const int* bflags, const int* inc_start,
                    const int* inc_count, const int* inc_items, int* colour, TakenColours* taken, int* rank,
-                   int* remaining, const int* layer, int* blocker, bool again);
+                   int* remaining, const int* layer, int* blocker, bool again, int max_polls);
 // The whole layout of at most kSmallLayout groups in one workgroup: as many as
 // its LDS holds.  A solve takes 45 us less with it than with the launches for
 // any number (300, 1,700 and 2,000 groups measured).
+// A wave that polled max_polls times gives up and sets the kWordLeft word instead
+// of a layout (0 with one); nothing is laid out then.
 constexpr int kSmallLayout = 4096;
+constexpr int kSmallPolls = 1 << 22;  // each a few LDS round trips
 struct SmallLayoutArgs {
     int n_groups, n_ent, waves;  // waves: of the resident kernel (0: no plan)
+    int max_polls;
     const int *ga, *gb, *bflags, *group_start, *layer;
     int *inc_count, *inc_start;  // n_ent each
     int *colour_start, *pos_start, *order, *pos_a, *group_desc, *flow, *pred, *used;

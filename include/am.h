@@ -412,6 +412,10 @@ int am_solve(am_ctx* ctx, double dt, int32_t post_stabilization, int32_t* iterat
 int am_solve_order_pull(am_ctx* ctx, int32_t* order, int32_t capacity, int32_t* n);
 /* Colour of every contact in the current layout (64 = sequential tail). */
 int am_colours_pull(am_ctx* ctx, int32_t* colour_of_contact, int32_t capacity, int32_t* n_colours);
+/* For tests: the polls after which the colouring's kernels give up waiting for
+ * other groups and leave theirs to the next launch (0: automatic, far above what
+ * any colouring takes).  The colours do not depend on it. */
+int am_colour_polls_set(am_ctx* ctx, int32_t polls);
 /* CollisionProcessor.updateInCollections (CollisionProcessor.java:232-303):
  * one PGS sweep over the external and internal contacts with sub-body
  * Jacobians (computeInCollection), in colour order over physical body pairs
