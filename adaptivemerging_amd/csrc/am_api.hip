@@ -486,7 +486,6 @@ int build_layout(am_ctx* c) {
         if (small) {
             SmallLayoutArgs A;
             A.n_groups = ng;
-            A.n_ent = c->n_ent;
             A.waves = 4 * rgrid;
             A.max_polls = c->colour_polls > 0 ? c->colour_polls : kSmallPolls;
             A.ga = c->g_a.p;

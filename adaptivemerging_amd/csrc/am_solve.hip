@@ -1976,11 +1976,10 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, n = A.n_groups;
     constexpr int kPer = kSmallLayout / kSmallThreads;
 
-    // incidence lists: a body's groups in any order
-    for (int e = t; e < A.n_ent; e += kSmallThreads) st_int(&A.inc_count[e], 0);
+    // Incidence lists: a body's groups in any order.  Only bodies with groups are
+    // looked at: the groups clear their bodies' counts, and the first one counted at
+    // a body takes its place in the list.
     if (t == 0) L.n_items = L.gave_up = 0;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
     int body[kPer][2], at[kPer][2], count[kPer][2];  // this thread's groups; -1: a pinned body
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
@@ -1997,6 +1996,13 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
     for (int k = 0; k < kPer; k++)
         if (body[k][1] == body[k][0]) body[k][1] = -1;
 #pragma unroll
+    for (int k = 0; k < kPer; k++)
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            if (body[k][s] >= 0) st_int(&A.inc_count[body[k][s]], 0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
     for (int k = 0; k < kPer; k++) {
         const int g = t + k * kSmallThreads;
 #pragma unroll
@@ -2008,27 +2014,30 @@ __global__ __launch_bounds__(kSmallThreads) void k_layout_small(SmallLayoutArgs 
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (int e = t; e < A.n_ent; e += kSmallThreads) {
-        const int c = ld_int(&A.inc_count[e]);
-        if (c > 0) {
-            const int start = atomicAdd(&L.n_items, c);
-            st_int(&A.inc_start[e], start);
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            count[k][s] = body[k][s] >= 0 ? ld_int(&A.inc_count[body[k][s]]) : 0;
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            if (body[k][s] < 0 || at[k][s] != 0) continue;
+            const int start = atomicAdd(&L.n_items, count[k][s]);
+            st_int(&A.inc_start[body[k][s]], start);
             if (!A.layer) {
                 L.set[start] = 0;
                 L.in_tail[start] = 0;
             }
         }
-    }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int start[kPer][2];
 #pragma unroll
     for (int k = 0; k < kPer; k++)
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            start[k][s] = body[k][s] >= 0 ? ld_int(&A.inc_start[body[k][s]]) : 0;
-            count[k][s] = body[k][s] >= 0 ? ld_int(&A.inc_count[body[k][s]]) : 0;
-        }
+        for (int s = 0; s < 2; s++) start[k][s] = body[k][s] >= 0 ? ld_int(&A.inc_start[body[k][s]]) : 0;
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
         const int g = t + k * kSmallThreads;

@@ -158,17 +158,21 @@ void launch_colour(hipStream_t s, int n_groups, const int* ga, const int* gb, co
                    const int* inc_count, const int* inc_items, int* colour, TakenColours* taken, int* rank,
                    int* remaining, const int* layer, int* blocker, bool again, int max_polls);
 // The whole layout of at most kSmallLayout groups in one workgroup: as many as
-// its LDS holds.  A solve takes 45 us less with it than with the launches for
-// any number (300, 1,700 and 2,000 groups measured).
+// its LDS holds.  us of a layout and its read-back, here / by the launches, for
+// 300, 1,000, 2,000 and 4,096 groups of a pile (13 colours): 56 / 110, 63 / 112,
+// 80 / 125, 113 / 134, the same with 1,000 and with 150,000 bodies.  Groups that
+// all share one dynamic body wait for each other in turn: 230 / 362, 843 / 1,026,
+// 2,245 / 1,911, 7,007 / 3,802 (no scene here has such a body; with one launch per
+// round of the colouring each of its groups took a round).
 // A wave that polled max_polls times gives up and sets the kWordLeft word instead
 // of a layout (0 with one); nothing is laid out then.
 constexpr int kSmallLayout = 4096;
 constexpr int kSmallPolls = 1 << 22;  // each a few LDS round trips
 struct SmallLayoutArgs {
-    int n_groups, n_ent, waves;  // waves: of the resident kernel (0: no plan)
+    int n_groups, waves;  // waves: of the resident kernel (0: no plan)
     int max_polls;
     const int *ga, *gb, *bflags, *group_start, *layer;
-    int *inc_count, *inc_start;  // n_ent each
+    int *inc_count, *inc_start;  // by body
     int *colour_start, *pos_start, *order, *pos_a, *group_desc, *flow, *pred, *used;
 };
 void launch_layout_small(hipStream_t s, const SmallLayoutArgs& A);
