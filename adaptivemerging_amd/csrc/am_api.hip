@@ -786,7 +786,7 @@ int train_append(am_ctx* c) {
 }
 
 // Start residual of the lambdas currently in the records (sweep order).
-void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block);
+void pgs_shape(am_ctx* c, const am_params& P, int iterations, int* grid, int* block);
 
 int start_residual(am_ctx* c, PgsArgs G, double* out) {
     hipStream_t s = c->stream;
@@ -801,7 +801,7 @@ int start_residual(am_ctx* c, PgsArgs G, double* out) {
     pc.pgs_grid = 0;
     pc.pgs_block = 0;
     int grid = 1, block = 256;
-    pgs_shape(c, pc, &grid, &block);
+    pgs_shape(c, pc, 0, &grid, &block);
     AM_HIP(c, launch_pgs(s, G, grid, block, c->params.pgs_plain_launch != 0, c->one_body_groups));
     AM_HIP(c, c->d_resid.ensure(1));
     fill_int(s, (int*)c->d_resid.p, 2, 0);
@@ -820,9 +820,10 @@ int start_residual(am_ctx* c, PgsArgs G, double* out) {
 // sides needs the coloured one, which gives the same bits.
 bool pgs_dataflow(const am_ctx* c, const am_params& P) { return P.pgs_schedule == 0 && !c->one_body_groups; }
 
-// Launch shape of the PGS kernel under P (after build_layout): workgroups and
-// threads per workgroup, clamped to what can be co-resident.
-void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
+// Launch shape of the PGS kernel for `iterations` sweeps under P (after
+// build_layout): workgroups and threads per workgroup, clamped to what can be
+// co-resident.
+void pgs_shape(am_ctx* c, const am_params& P, int iterations, int* grid, int* block) {
     bool ok = false;
     const bool flow = pgs_dataflow(c, P);
     // Everything resident in LDS wherever it fits: it was the faster on every
@@ -832,7 +833,7 @@ void pgs_shape(am_ctx* c, const am_params& P, int* grid, int* block) {
     // 47 -> 27; 8,000 in one colour: 13 -> 5.4; 27,000 in 48 scenes: 47 -> 30).
     // Its arrival words take 1 KiB a sweep, hence the bound on the sweeps.  A
     // given pgs_grid asks for k_pgs_flow.
-    if (flow && P.pgs_grid == 0 && c->resident_grid > 0 && P.iterations <= kResidentMaxSweeps) {
+    if (flow && P.pgs_grid == 0 && c->resident_grid > 0 && iterations <= kResidentMaxSweeps) {
         *grid = c->resident_grid;
         *block = kResidentThreads;
         return;
@@ -978,7 +979,7 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         S.scene_used = c->scene_used.p;
     }
     int grid = 1, block = 64;
-    pgs_shape(c, P, &grid, &block);
+    pgs_shape(c, P, iterations, &grid, &block);
     if (main_solve) {
         c->last_grid = grid;
         c->last_block = block;
@@ -1892,7 +1893,7 @@ int am_autotune(am_ctx* c, double dt, int32_t sweeps, int32_t reps, int32_t appl
         P.pgs_grid = grid;
         P.pgs_block = block;
         int g = 1, b = 64;
-        pgs_shape(c, P, &g, &b);
+        pgs_shape(c, P, sweeps, &g, &b);
         for (const Cand& k : cands)
             if (k.sched == sched && k.grid_used == g && k.block_used == b) return;
         cands.push_back({sched, grid, block, g, b, 0.0});

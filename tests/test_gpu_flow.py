@@ -145,3 +145,43 @@ def test_resident_steps_at_their_edges(gpu_lib, spheres, boxes):
         assert_contacts_equal(ctx.contacts(), orc.contacts())
         assert_bits_equal("deltaV", ctx.pull_deltav(), orc.pull_deltav())
         ctx.close()
+
+
+def test_the_kernel_follows_the_sweeps_that_run(gpu_lib):
+    """The resident kernel takes up to 65,536 sweeps, with 1 KiB of arrival words
+    for each: those of the solve at hand, not of the other kind of solve nor of the
+    parameters that a tuning run replaces."""
+    import ctypes as C
+
+    from adaptivemerging_amd.context import Context
+
+    def free_bytes():
+        path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln)
+        free, total = C.c_size_t(), C.c_size_t()
+        assert C.CDLL(path).hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    ctx = Context()
+    ctx.upload(workloads.merge_stack(seed=4))
+    # the boards merge with each other but not with the ground: contacts for both solves
+    ctx.set_params(gravity_amount=9.81, iterations=100, tolerance=1e-10, enable_sleeping=0, enable_merge_pinned=0)
+    for _ in range(25):
+        st = ctx.step(0.01)
+    assert st["n_collections"] >= 1 and ctx.launch_shape()[1] == 320
+    # a bound of sweeps for the main solve: a tuning run of 2 sweeps lists what runs them
+    ctx.set_params(iterations=70000, tolerance=1e-3)
+    ctx.detect(0.01)
+    trials, _ = ctx.autotune(0.01, sweeps=2, reps=1, apply=False)
+    print("first trial", trials[0], flush=True)
+    assert trials[0]["block_used"] == 320
+    # many sweeps of the single sweep's solve: k_pgs_flow's words are 64 bytes a sweep
+    ctx.set_params(iterations=30)
+    ctx.update_in_collections(0.01)
+    before = free_bytes()
+    ctx.set_params(iterations_in_collection=100000)
+    ctx.detect(0.01)
+    ctx.update_in_collections(0.01)
+    taken = before - free_bytes()
+    print("bytes taken", taken, flush=True)
+    assert taken < 32 << 20
+    ctx.close()
