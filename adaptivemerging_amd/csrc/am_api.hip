@@ -826,14 +826,22 @@ bool pgs_dataflow(const am_ctx* c, const am_params& P) { return P.pgs_schedule =
 void pgs_shape(am_ctx* c, const am_params& P, int iterations, int* grid, int* block) {
     bool ok = false;
     const bool flow = pgs_dataflow(c, P);
-    // Everything resident in LDS wherever it fits: it was the faster on every
-    // contact set tried (us per sweep, k_pgs_flow -> resident, by contacts: 12:
-    // 9 -> 6.3; 1,100 in a tower, one long chain: 24 -> 24; 750 between sphere
-    // trees, up to 60 in a group: 46 -> 26; 5,000 in a pile: 30 -> 22; 37,000:
-    // 47 -> 27; 8,000 in one colour: 13 -> 5.4; 27,000 in 48 scenes: 47 -> 30).
-    // Its arrival words take 1 KiB a sweep, hence the bound on the sweeps.  A
-    // given pgs_grid asks for k_pgs_flow.
-    if (flow && P.pgs_grid == 0 && c->resident_grid > 0 && iterations <= kResidentMaxSweeps) {
+    // Everything resident in LDS wherever it fits: it was no slower on any contact
+    // set tried (us per sweep, k_pgs_flow at its automatic grid -> resident, by
+    // contacts: 40 and 8,000 in one colour: 1.3 -> 1.1, 13 -> 5.4; a rope of 19 and
+    // 6,000: 7.0 -> 7.1, 26 -> 12; walls of 156, 10,377 and 46,142: 12 -> 11,
+    // 31 -> 16, 42 -> 19; a body under 400 boxes: 941 -> 861; towers of 97 and 2,016:
+    // 18 -> 17, 25 -> 21; piles of 320, 6,212 and 26,812: 16 -> 15, 31 -> 22,
+    // 41 -> 26; 750 between sphere trees, up to 60 in a group: 46 -> 26; 1,176 in 4
+    // scenes and 13,784 in 40: 13 -> 10, 30 -> 12; with per-scene exits, 27,000 in
+    // 48: 47 -> 30).  Its arrival words take 1 KiB a sweep, hence the bound on the
+    // sweeps.  A given pgs_grid asks for k_pgs_flow.  So does an ordinary launch:
+    // nothing keeps those of several contexts from holding a part of the card each,
+    // and a resident workgroup takes most of a CU, so that two solves of 256 of them
+    // would both wait for room until their spin limits, where k_pgs_flow's 512 small
+    // ones at its automatic grid leave room for more.
+    if (flow && P.pgs_grid == 0 && P.pgs_plain_launch == 0 && c->resident_grid > 0 &&
+        iterations <= kResidentMaxSweeps) {
         *grid = c->resident_grid;
         *block = kResidentThreads;
         return;

@@ -164,10 +164,12 @@ typedef struct am_params {
     double threshold_breath;          /* 1e-5 */
     /* implementation knobs (no reference counterpart) */
     int32_t pgs_block;                /* threads per workgroup in the PGS kernel (0 = auto) */
-    int32_t pgs_grid;                 /* workgroups of the PGS kernel (0 = auto) */
+    int32_t pgs_grid;                 /* workgroups of the PGS kernel (0 = auto); a given number also asks for
+                                         the dataflow kernel that streams its records, at any size */
     int32_t pgs_plain_launch;         /* 1: launch the PGS kernel with an ordinary (not cooperative) launch,
                                          grid clamped to the co-resident limit; for profilers that do not
-                                         support cooperative launches (0 = cooperative) */
+                                         support cooperative launches (0 = cooperative).  The streaming
+                                         dataflow kernel then runs at any size */
     int32_t pgs_schedule;             /* 0: dataflow (each body's deltaV handed from update to update, no grid barriers);
                                          1: colour by colour with a grid barrier between colours.
                                          Both give bit-identical results (the exported sweep order).  Contacts pushed

@@ -185,3 +185,43 @@ def test_the_kernel_follows_the_sweeps_that_run(gpu_lib):
     print("bytes taken", taken, flush=True)
     assert taken < 32 << 20
     ctx.close()
+
+
+def test_ordinary_launches_of_two_contexts_at_once(gpu_lib):
+    """With pgs_plain_launch nothing keeps two contexts' kernels apart: the small
+    workgroups of k_pgs_flow run, at any size, which leave room for each other.
+    Two threads step a wall of boxes each (2,300 groups: 256 workgroups of the
+    resident kernel); both end where one alone does, bit for bit."""
+    import threading
+
+    from adaptivemerging_amd.context import Context
+    from adaptivemerging_amd.scene import Scene
+
+    scene = Scene()
+    scene.add_plane([0, 0, 0], [0, 1, 0], friction=0.8)
+    for j in range(30):
+        for i in range(40):
+            scene.add_box([0.4, 0.2, 0.3], [0.41 * i + 0.2 * (j % 2), 0.0999 + 0.1999 * j, 0])
+
+    def run(out, k):
+        ctx = Context()
+        ctx.upload(scene)
+        ctx.set_params(iterations=60, tolerance=0.0, gravity_amount=9.81, pgs_plain_launch=1, enable_merging=0,
+                       enable_sleeping=0)
+        for _ in range(20):
+            ctx.step(0.005)
+        out[k] = (ctx.launch_shape(), ctx.pull_state())
+        ctx.close()
+
+    alone, out = {}, {}
+    run(alone, 0)
+    print("shape", alone[0][0], flush=True)
+    assert alone[0][0] == (512, 64)
+    threads = [threading.Thread(target=run, args=(out, k)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(2):
+        for name, a, b in zip("xRvw", alone[0][1], out[k][1]):
+            assert_bits_equal(f"context {k} {name}", b, a)
