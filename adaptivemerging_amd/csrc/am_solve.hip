@@ -1153,6 +1153,9 @@ AMD_INLINE double row_jdv(double p) {
 }
 
 constexpr long kFlowSpinLimit = 1L << 22;  // polls of one wait (each a memory round trip)
+// Turns of a wait that may look at LDS only, and are shorter: the pass keeper's, and the sweeping waves' for it.  A wave that stops making
+// progress meets the limit above first, and its error flag ends these.
+constexpr long kLdsSpinLimit = 16 * kFlowSpinLimit;
 
 // Per-contact operands of one row: this lane's J entries and update
 // coefficients of the three rows, and the contact's uniform values.
@@ -2535,7 +2538,7 @@ AMD_INLINE void keep_passes(const FlowArgs& F, ResidentLds& L, int lane) {
             continue;
         }
         if (uniform(lds_int(&L.failed))) return;
-        if (++spins > kFlowSpinLimit ||
+        if (++spins > kLdsSpinLimit ||
             ((spins & 255) == 0 && uniform(__hip_atomic_load(P.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
             if (lane == 0) {
                 atomicOr(P.error, 1);
@@ -2719,7 +2722,7 @@ __global__ __launch_bounds__((kResWaves + 1) * 64) __attribute__((amdgpu_waves_p
                 // every wave runs the sweep after the converged one and leaves then
                 leave = (stop && stop <= need) || uniform(lds_int(&L.failed));
                 if (leave || (known >= need && pub >= p - 3)) break;
-                if (spins > 16 * kFlowSpinLimit) {  // the keeper gives up long before
+                if (spins > 4 * kLdsSpinLimit) {  // the keeper gives up long before
                     if (lane == 0) atomicOr(P.error, 1);
                     leave = true;
                     break;
