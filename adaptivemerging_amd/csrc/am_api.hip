@@ -907,7 +907,6 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
     S.post = main_solve ? post : 0;
     S.in_collection = main_solve ? 0 : 1;
     S.lam_alt = nullptr;
-    S.iters_used = nullptr;
     S.scene_used = nullptr;
     const bool flow = pgs_dataflow(c, P);
     MemBatch m(s);
@@ -1053,7 +1052,6 @@ int do_solve(am_ctx* c, double dt, int post, bool main_solve, int* iters, double
         F.resident_used = c->s_used.p;
         F.n_waves = (unsigned)fgrid;
         S.lam_alt = c->s_lam_alt.p;
-        S.iters_used = G.iters_used;
         AM_HIP(c, hipEventRecord(c->kev[1], s));
         AM_HIP(c, launch_pgs_flow(s, F, fgrid, block, P.pgs_plain_launch != 0));
         AM_HIP(c, hipEventRecord(c->kev[2], s));

@@ -167,68 +167,68 @@ __global__ __launch_bounds__(kPairThreads) void k_pairs(PairArgs A, uint64_t* ke
         n++;
     };
     auto search = [&]() {
-    if (task < 27) {
-        // a large body scans no cells: every grid body pairs with it in its task 27
-        if (!large_i) {
-            const int nx = A.cell[k * 4 + 0] + task % 3 - 1;
-            const int ny = A.cell[k * 4 + 1] + (task / 3) % 3 - 1;
-            const int nz = A.cell[k * 4 + 2] + task / 9 - 1;
-            const int h = cell_hash(nx, ny, nz, di.scene, A.mask);
-            const int s0 = A.bucket_start[h], cnt = A.bucket_count[h];
-            for (int q = 0; q < cnt; q++) {
-                const int kj = A.bucket_items[s0 + q];
-                if (A.cell[kj * 4 + 0] != nx || A.cell[kj * 4 + 1] != ny || A.cell[kj * 4 + 2] != nz) continue;
+        if (task < 27) {
+            // a large body scans no cells: every grid body pairs with it in its task 27
+            if (!large_i) {
+                const int nx = A.cell[k * 4 + 0] + task % 3 - 1;
+                const int ny = A.cell[k * 4 + 1] + (task / 3) % 3 - 1;
+                const int nz = A.cell[k * 4 + 2] + task / 9 - 1;
+                const int h = cell_hash(nx, ny, nz, di.scene, A.mask);
+                const int s0 = A.bucket_start[h], cnt = A.bucket_count[h];
+                for (int q = 0; q < cnt; q++) {
+                    const int kj = A.bucket_items[s0 + q];
+                    if (A.cell[kj * 4 + 0] != nx || A.cell[kj * 4 + 1] != ny || A.cell[kj * 4 + 2] != nz) continue;
+                    const int bj = A.grid_order[kj];
+                    if (B.desc[bj].scene != di.scene) continue;
+                    const int slot_j = B.slot[bj];
+                    if (slot_j <= slot_i) continue;
+                    if (skip_pair(A, slot_i, slot_j)) continue;
+                    const double ddx = A.sphere[kj * 4 + 0] - ci[0];
+                    const double ddy = A.sphere[kj * 4 + 1] - ci[1];
+                    const double ddz = A.sphere[kj * 4 + 2] - ci[2];
+                    const double rr = A.sphere[kj * 4 + 3] + ci[3];
+                    const double d2 = ddx * ddx + ddy * ddy + ddz * ddz;
+                    // superset of every narrow-phase first test (<= with slack)
+                    if (d2 > rr * rr * (1.0 + 1e-9) + 1e-300) continue;
+                    emit(slot_j, B.sub[bj]);
+                }
+            }
+        } else if (task == 27) {
+            for (int q = 0; q < A.n_large; q++) {
+                const int kj = A.large[q];
+                if (kj == k) continue;
                 const int bj = A.grid_order[kj];
                 if (B.desc[bj].scene != di.scene) continue;
                 const int slot_j = B.slot[bj];
-                if (slot_j <= slot_i) continue;
+                if (slot_j == slot_i || (large_i && slot_j < slot_i)) continue;
                 if (skip_pair(A, slot_i, slot_j)) continue;
                 const double ddx = A.sphere[kj * 4 + 0] - ci[0];
                 const double ddy = A.sphere[kj * 4 + 1] - ci[1];
                 const double ddz = A.sphere[kj * 4 + 2] - ci[2];
                 const double rr = A.sphere[kj * 4 + 3] + ci[3];
                 const double d2 = ddx * ddx + ddy * ddy + ddz * ddz;
-                // superset of every narrow-phase first test (<= with slack)
                 if (d2 > rr * rr * (1.0 + 1e-9) + 1e-300) continue;
                 emit(slot_j, B.sub[bj]);
             }
-        }
-    } else if (task == 27) {
-        for (int q = 0; q < A.n_large; q++) {
-            const int kj = A.large[q];
-            if (kj == k) continue;
-            const int bj = A.grid_order[kj];
-            if (B.desc[bj].scene != di.scene) continue;
-            const int slot_j = B.slot[bj];
-            if (slot_j == slot_i || (large_i && slot_j < slot_i)) continue;
-            if (skip_pair(A, slot_i, slot_j)) continue;
-            const double ddx = A.sphere[kj * 4 + 0] - ci[0];
-            const double ddy = A.sphere[kj * 4 + 1] - ci[1];
-            const double ddz = A.sphere[kj * 4 + 2] - ci[2];
-            const double rr = A.sphere[kj * 4 + 3] + ci[3];
-            const double d2 = ddx * ddx + ddy * ddy + ddz * ddz;
-            if (d2 > rr * rr * (1.0 + 1e-9) + 1e-300) continue;
-            emit(slot_j, B.sub[bj]);
-        }
-        for (int q = A.plane_start[di.scene]; q < A.plane_start[di.scene + 1]; q++) {
-            const int p = A.planes[q];
-            const am_body_desc& pd = B.desc[p];
-            const int slot_p = B.slot[p];
-            if (slot_p == slot_i) continue;
-            if (skip_pair(A, slot_i, slot_p)) continue;
-            const d3 nrm = ld3(pd.plane_n);
-            if (di.geom == AM_GEOM_BOX || di.geom == AM_GEOM_COMPOSITE) {
-                // first test of BoxPlane.dBoxPlane (for a composite: its enclosing sphere)
-                if (dot(ld3(&B.x[bi * 3]), nrm) + pd.plane_d > di.radius) continue;
-            } else {
-                // first (root) test of collideSphereTreeAndPlane
-                const d3 c = ld3(&A.T.cw[di.tree_first * 3]);
-                const double d = nrm.x * c.x + nrm.y * c.y + nrm.z * c.z + pd.plane_d - A.T.nodes[di.tree_first].r;
-                if (!(d < 0)) continue;
+            for (int q = A.plane_start[di.scene]; q < A.plane_start[di.scene + 1]; q++) {
+                const int p = A.planes[q];
+                const am_body_desc& pd = B.desc[p];
+                const int slot_p = B.slot[p];
+                if (slot_p == slot_i) continue;
+                if (skip_pair(A, slot_i, slot_p)) continue;
+                const d3 nrm = ld3(pd.plane_n);
+                if (di.geom == AM_GEOM_BOX || di.geom == AM_GEOM_COMPOSITE) {
+                    // first test of BoxPlane.dBoxPlane (for a composite: its enclosing sphere)
+                    if (dot(ld3(&B.x[bi * 3]), nrm) + pd.plane_d > di.radius) continue;
+                } else {
+                    // first (root) test of collideSphereTreeAndPlane
+                    const d3 c = ld3(&A.T.cw[di.tree_first * 3]);
+                    const double d = nrm.x * c.x + nrm.y * c.y + nrm.z * c.z + pd.plane_d - A.T.nodes[di.tree_first].r;
+                    if (!(d < 0)) continue;
+                }
+                emit(slot_p, B.sub[p]);
             }
-            emit(slot_p, B.sub[p]);
         }
-    }
     };
     search();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

@@ -25,8 +25,7 @@ struct SetupArgs {
     int post;
     int in_collection;
     const double* lam_alt;  // unpack: odd-sweep lambda of the dataflow schedule, stride 4 (null: coloured)
-    const int* iters_used;  // unpack: sweeps used (with lam_alt)
-    const int* scene_used = nullptr;  // unpack with lam_alt: sweeps used per scene (null: iters_used for all)
+    const int* scene_used = nullptr;  // unpack with lam_alt: sweeps used per scene (null: the same for all)
 };
 
 // Inputs of the persistent coloured PGS kernel.
