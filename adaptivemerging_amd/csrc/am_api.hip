@@ -839,8 +839,8 @@ void pgs_shape(am_ctx* c, const am_params& P, int iterations, int* grid, int* bl
     // nothing keeps those of several contexts from holding a part of the card each,
     // and a resident workgroup takes most of a CU, so that two solves of 256 of them
     // would both wait for room until their spin limits, where k_pgs_flow's 512 small
-    // ones at its automatic grid leave room for more.
-    if (flow && P.pgs_grid == 0 && P.pgs_plain_launch == 0 && c->resident_grid > 0 &&
+    // ones at its automatic grid leave room for more (2 asks for it all the same).
+    if (flow && P.pgs_grid == 0 && P.pgs_plain_launch != 1 && c->resident_grid > 0 &&
         iterations <= kResidentMaxSweeps) {
         *grid = c->resident_grid;
         *block = kResidentThreads;

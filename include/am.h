@@ -169,7 +169,9 @@ typedef struct am_params {
     int32_t pgs_plain_launch;         /* 1: launch the PGS kernel with an ordinary (not cooperative) launch,
                                          grid clamped to the co-resident limit; for profilers that do not
                                          support cooperative launches (0 = cooperative).  The streaming
-                                         dataflow kernel then runs at any size */
+                                         dataflow kernel then runs at any size.  2: an ordinary launch of the
+                                         kernel that 0 runs, for a process that solves in one context at a
+                                         time: solves in two at once may fail */
     int32_t pgs_schedule;             /* 0: dataflow (each body's deltaV handed from update to update, no grid barriers);
                                          1: colour by colour with a grid barrier between colours.
                                          Both give bit-identical results (the exported sweep order).  Contacts pushed

@@ -217,6 +217,16 @@ def test_ordinary_launches_of_two_contexts_at_once(gpu_lib):
     run(alone, 0)
     print("shape", alone[0][0], flush=True)
     assert alone[0][0] == (512, 64)
+    ctx = Context()
+    ctx.upload(scene)
+    ctx.set_params(iterations=60, tolerance=0.0, gravity_amount=9.81, pgs_plain_launch=2, enable_merging=0,
+                   enable_sleeping=0)
+    for _ in range(20):  # one context at a time: the resident kernel
+        ctx.step(0.005)
+    assert ctx.launch_shape() == (256, 320)
+    for name, a, b in zip("xRvw", alone[0][1], ctx.pull_state()):
+        assert_bits_equal(f"resident {name}", b, a)
+    ctx.close()
     threads = [threading.Thread(target=run, args=(out, k)) for k in range(2)]
     for t in threads:
         t.start()
